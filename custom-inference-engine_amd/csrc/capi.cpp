@@ -169,12 +169,32 @@ int cie_prefill_kernel(int B, int Hq, int Hk, int Lq, int Lk, int D, int causal,
 
 }  // extern "C"
 
+// Fixes the key splits of a launch (0: the library's rule) and takes its
+// partial states out of the workspace.
+static int flash_set_splits(cie::FlashParams* p, int D, int splits, void* workspace, size_t workspace_bytes) {
+  if (splits < 0 || splits > cie::kFlashMaxSplits)
+    return fail(CIE_EINVAL, "splits must be in [0, %d], got %d", cie::kFlashMaxSplits, splits);
+  p->splits = splits ? splits : cie::flash_splits(*p, D);
+  const size_t need = cie::flash_part_bytes(*p, D, p->splits);
+  if (need == 0) return CIE_OK;
+  if ((int64_t)p->n_wg * p->splits > 0x7fffffff / (4 * 32))  // workgroups of the merge pass
+    return fail(CIE_EINVAL, "problem too large for one launch with %d splits", p->splits);
+  if (!workspace || workspace_bytes < need)
+    return fail(CIE_EWORKSPACE, "workspace of %zu bytes required, %zu given", need,
+                workspace ? workspace_bytes : (size_t)0);
+  if (!aligned16(workspace)) return fail(CIE_EINVAL, "workspace: pointer is not 16-byte aligned");
+  p->part = static_cast<float*>(workspace);
+  return CIE_OK;
+}
+
+// splits: key splits of the launch (0: the library's rule; 1: none).
 static int flash_impl(const void* q, const void* k, const void* v, void* o,
                       const int64_t* q_stride, const int64_t* k_stride,
                       const int64_t* v_stride, const int64_t* o_stride,
                       int B, int Hq, int Hk, int Lq, int Lk, int D,
                       float scale, int causal, int dtype, void* stream,
-                      cie::RopeTables rope, const int32_t* q_pos0) {
+                      cie::RopeTables rope, const int32_t* q_pos0, int splits = 1,
+                      void* workspace = nullptr, size_t workspace_bytes = 0) {
   CIE_TRY(common_checks(Hq, Hk, D, dtype));
   if (B < 0 || Lq < 0 || Lk < 0) return fail(CIE_EINVAL, "negative size (B=%d, Lq=%d, Lk=%d)", B, Lq, Lk);
   if (!std::isfinite(scale)) return fail(CIE_EINVAL, "scale must be finite");
@@ -217,10 +237,124 @@ static int flash_impl(const void* q, const void* k, const void* v, void* o,
   const cie::DeviceShape dev = cie::device_shape();
   p.cus = dev.cus;
   p.xcd_shift = dev.xcd_shift;
+  CIE_TRY(flash_set_splits(&p, D, Lk > 0 ? splits : 1, workspace, workspace_bytes));
   return launch_status(cie::launch_flash(p, dtype, D, static_cast<hipStream_t>(stream)));
 }
 
+// Largest valid context length: the table bound, tightened by the caller's hint.
+static int paged_ctx_limit(int max_context, int block_size, int max_blocks_per_seq) {
+  const int64_t bound = (int64_t)max_blocks_per_seq * block_size;
+  return (int)(max_context > 0 ? std::min<int64_t>(max_context, bound) : bound);
+}
+
 extern "C" {
+
+size_t cie_flash_workspace_bytes(int B, int Hq, int Hk, int Lq, int Lk, int D, int causal, int splits) {
+  if (B <= 0 || Hq <= 0 || Hk <= 0 || Lq <= 0 || Lk <= 0 || Hq % Hk || !head_dim_ok(D) || splits < 0 ||
+      splits > cie::kFlashMaxSplits)
+    return 0;
+  const int64_t n_mt = ((int64_t)Lq + 127) / 128;
+  if (n_mt * B * Hq > 0x7fffffff) return 0;
+  cie::FlashParams p{};
+  p.B = B; p.Hq = Hq; p.Hk = Hk; p.Lq = Lq; p.Lk = Lk; p.group = Hq / Hk;
+  p.n_mt = (int)n_mt;
+  p.n_wg = (int)(n_mt * B * Hq);
+  p.causal = causal ? 1 : 0;
+  p.cus = cie::device_shape().cus;
+  return cie::flash_part_bytes(p, D, splits ? splits : cie::flash_splits(p, D));
+}
+
+int cie_flash_fwd_ex(const void* q, const void* k, const void* v, void* o,
+                     const int64_t* q_stride, const int64_t* k_stride,
+                     const int64_t* v_stride, const int64_t* o_stride,
+                     int B, int Hq, int Hk, int Lq, int Lk, int D,
+                     float scale, int causal, int dtype,
+                     const void* rope_cos, const void* rope_sin, int rope_rows, int rope_dtype,
+                     const int32_t* q_pos0, int splits, void* workspace, size_t workspace_bytes, void* stream) {
+  cie::RopeTables rope{nullptr, nullptr, 0, 0};
+  if (rope_cos || rope_sin) {
+    CIE_TRY(check_rope(rope_cos, rope_sin, rope_rows, rope_dtype));
+    rope = cie::RopeTables{rope_cos, rope_sin, rope_rows, rope_dtype};
+  }
+  return flash_impl(q, k, v, o, q_stride, k_stride, v_stride, o_stride, B, Hq, Hk, Lq, Lk, D, scale, causal, dtype,
+                    stream, rope, q_pos0, splits, workspace, workspace_bytes);
+}
+
+size_t cie_flash_paged_workspace_bytes(int B, int Hq, int Hk, int Lq, int D, int max_context, int block_size,
+                                       int max_blocks_per_seq, int splits) {
+  if (block_size <= 0 || max_blocks_per_seq <= 0 || (int64_t)max_blocks_per_seq * block_size > 0x7fffffff) return 0;
+  return cie_flash_workspace_bytes(B, Hq, Hk, Lq, paged_ctx_limit(max_context, block_size, max_blocks_per_seq), D, 1,
+                                   splits);
+}
+
+int cie_flash_paged(const void* q, const void* k_cache, const void* v_cache, const int32_t* block_tables,
+                    const int32_t* context_lens, void* o,
+                    const int64_t* q_stride, const int64_t* kc_stride,
+                    const int64_t* vc_stride, const int64_t* o_stride,
+                    int B, int Hq, int Hk, int Lq, int D,
+                    int num_blocks, int block_size, int max_blocks_per_seq,
+                    int max_context, float scale, int causal, int dtype,
+                    const void* rope_cos, const void* rope_sin, int rope_rows, int rope_dtype,
+                    int splits, void* workspace, size_t workspace_bytes, void* stream) {
+  CIE_TRY(common_checks(Hq, Hk, D, dtype));
+  if (B < 0 || Lq < 0) return fail(CIE_EINVAL, "negative size (B=%d, Lq=%d)", B, Lq);
+  if (block_size < 1) return fail(CIE_EINVAL, "block_size must be positive, got %d", block_size);
+  if (num_blocks < 0 || max_blocks_per_seq < 0)
+    return fail(CIE_EINVAL, "negative pool geometry (num_blocks=%d, max_blocks_per_seq=%d)", num_blocks,
+                max_blocks_per_seq);
+  if ((int64_t)max_blocks_per_seq * block_size > 0x7fffffff)
+    return fail(CIE_EINVAL, "max_blocks_per_seq * block_size exceeds 2^31");
+  const int ctx_limit = paged_ctx_limit(max_context, block_size, max_blocks_per_seq);
+  // positions, and the ends of the key and query tiles past the last one, stay below 2^31
+  if ((int64_t)ctx_limit + Lq > 0x7fffffff - 1024) return fail(CIE_EINVAL, "problem too large for one launch");
+  if (!std::isfinite(scale)) return fail(CIE_EINVAL, "scale must be finite");
+  if ((int64_t)B * Hq * Lq == 0) {
+    g_err.clear();
+    return CIE_OK;
+  }
+  CIE_TRY(check_ptr("q", q));
+  CIE_TRY(check_ptr("o", o));
+  CIE_TRY(check_ptr("k_cache", k_cache));
+  CIE_TRY(check_ptr("v_cache", v_cache));
+  if (!block_tables || !context_lens) return fail(CIE_EINVAL, "block_tables / context_lens: NULL pointer");
+  CIE_TRY(check_strides("q", q_stride));
+  CIE_TRY(check_strides("o", o_stride));
+  CIE_TRY(check_strides("k_cache", kc_stride));
+  CIE_TRY(check_strides("v_cache", vc_stride));
+  const int64_t n_mt = ((int64_t)Lq + 127) / 128;
+  if (n_mt * B * Hq > 0x7fffffff) return fail(CIE_EINVAL, "problem too large for one launch");
+
+  cie::FlashParams p{};
+  p.q = static_cast<const uint16_t*>(q);
+  p.k = static_cast<const uint16_t*>(k_cache);
+  p.v = static_cast<const uint16_t*>(v_cache);
+  p.o = static_cast<uint16_t*>(o);
+  p.qs0 = q_stride[0]; p.qs1 = q_stride[1]; p.qs2 = q_stride[2];
+  p.os0 = o_stride[0]; p.os1 = o_stride[1]; p.os2 = o_stride[2];
+  p.ks0 = kc_stride[0]; p.ks1 = kc_stride[2]; p.ks2 = kc_stride[1];  // block, head, token
+  p.vs0 = vc_stride[0]; p.vs1 = vc_stride[2]; p.vs2 = vc_stride[1];
+  p.ctx_limit = ctx_limit;
+  p.B = B; p.Hq = Hq; p.Hk = Hk; p.Lq = Lq; p.Lk = p.ctx_limit; p.group = Hq / Hk;
+  p.n_mt = (int)n_mt;
+  p.n_wg = (int)(n_mt * B * Hq);
+  set_scale(scale, &p.scale_log2, &p.q_sign);
+  p.causal = causal ? 1 : 0;
+  if (rope_cos || rope_sin) {
+    CIE_TRY(check_rope(rope_cos, rope_sin, rope_rows, rope_dtype));
+    p.rope = cie::RopeTables{rope_cos, rope_sin, rope_rows, rope_dtype};
+  }
+  p.bt = block_tables;
+  p.lens = context_lens;
+  p.max_blocks = max_blocks_per_seq;
+  p.num_blocks = num_blocks;
+  p.block_size = block_size;
+  p.bsdiv = cie::make_fastdiv((uint32_t)block_size);
+  const cie::DeviceShape dev = cie::device_shape();
+  p.cus = dev.cus;
+  p.xcd_shift = dev.xcd_shift;
+  CIE_TRY(flash_set_splits(&p, D, splits, workspace, workspace_bytes));
+  return launch_status(cie::launch_flash(p, dtype, D, static_cast<hipStream_t>(stream)));
+}
 
 int cie_flash_fwd(const void* q, const void* k, const void* v, void* o,
                   const int64_t* q_stride, const int64_t* k_stride,
@@ -241,12 +375,6 @@ int cie_flash_fwd_rope(const void* q, const void* k, const void* v, void* o,
   CIE_TRY(check_rope(rope_cos, rope_sin, rope_rows, rope_dtype));
   return flash_impl(q, k, v, o, q_stride, k_stride, v_stride, o_stride, B, Hq, Hk, Lq, Lk, D, scale, causal,
                     dtype, stream, cie::RopeTables{rope_cos, rope_sin, rope_rows, rope_dtype}, q_pos0);
-}
-
-// Largest valid context length: the table bound, tightened by the caller's hint.
-static int paged_ctx_limit(int max_context, int block_size, int max_blocks_per_seq) {
-  const int64_t bound = (int64_t)max_blocks_per_seq * block_size;
-  return (int)(max_context > 0 ? std::min<int64_t>(max_context, bound) : bound);
 }
 
 size_t cie_paged_workspace_bytes(int B, int Hq, int Hk, int Lq, int D, int max_context,

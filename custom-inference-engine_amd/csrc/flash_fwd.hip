@@ -95,6 +95,179 @@ struct FlashCfg {
   static_assert(NW >= 1 && BN * S == NW * 256, "tile must split evenly over 4 waves");
 };
 
+// How a launch of flash_fwd_kernel / flash_fwd_il_kernel reads K/V and leaves
+// its result.
+//   kKvDense: dense K/V, every workgroup sees all keys of its rows.
+//   kKvSplit: dense K/V, the key tiles of every query tile cut into p.splits
+//             contiguous runs, one workgroup each; flash_merge_kernel combines
+//             the partial states.
+//   kKvPaged: K/V read in place from a (num_blocks, block_size, Hk, D) pool
+//             through the int32 block table, with or without splits.
+enum KvMode { kKvDense = 0, kKvSplit = 1, kKvPaged = 2 };
+
+// The work item of a workgroup. Workgroups are dispatched round-robin over
+// the XCDs; each XCD gets a contiguous run of logical items so the query heads
+// of a kv head (and its neighbouring query tiles) share one L2. Within a kv
+// head the longest (last) query tiles go first; with splits the heads that
+// read the same keys are neighbours.
+struct FlashItem {
+  int b, kvh, hq, mt, sp;
+};
+template <int MODE>
+__device__ __forceinline__ FlashItem flash_item(const FlashParams& p) {
+  const int logical = xcd_logical(blockIdx.x, p.n_wg, p.xcd_shift);
+  const int G = p.group;
+  const int ns = MODE == kKvDense ? 1 : p.splits;
+  const int per_grp = p.n_mt * G * ns;
+  const int grp = logical / per_grp;
+  const int rem = logical - grp * per_grp;
+  const int rs = rem / G, g = rem - rs * G;
+  const int rank = MODE == kKvDense ? rs : rs / ns;
+  FlashItem w;
+  w.sp = MODE == kKvDense ? 0 : rs - rank * ns;
+  w.mt = p.n_mt - 1 - rank;
+  w.b = grp / p.Hk;
+  w.kvh = grp - w.b * p.Hk;
+  w.hq = w.kvh * G + g;
+  return w;
+}
+
+// Tile copies out of a paged pool (kKvPaged; C is the kernel's tile
+// configuration). A wave copies WR consecutive token rows of a tile; when the
+// block size is a multiple of WR they lie in one block, so one block id and
+// two scalar base addresses serve all of its copies, as in the dense kernel
+// (the 64-bit products of every copy's own id cost 0.2 us per tile with one
+// workgroup on a CU: 1000 new tokens on 4600, D=128, no splits, 123 us). Other
+// block sizes and the tile holding the last key form per-lane addresses. The block ids of the
+// workgroup's key range are staged in LDS once (kFlashIds of them: 16384
+// tokens of 16-token blocks); ids past those are read from the table. The
+// uniform copies take their ids from a register window of 64 consecutive
+// blocks (lane i holds block win + i, read with v_readlane): an LDS read in
+// front of every tile's copies is a round trip each wave waits for.
+template <typename C>
+struct PagedTiles {
+  static constexpr int RPI = 64 / C::S;     // token rows per copy instruction
+  static constexpr int WR = C::NW * RPI;    // token rows per wave and tile
+  const uint16_t* kb;
+  const uint16_t* vb;
+  const int32_t* row;  // the sequence's block table row
+  const int32_t* ids;  // LDS: blocks blk_lo, blk_lo + 1, ...
+  int blk_lo, last_key;
+  int win, win_id;  // register window of the uniform copies
+  bool uni;
+  int lrow[C::NW], lchk[C::NW];
+  uint32_t koff[C::NW], voff[C::NW];
+
+  // `bad` (workgroup-uniform): a block id of the keys [k0, k1) lies outside
+  // the pool. Staged ids are clamped into it, so nothing is ever read through
+  // a bad one.
+  __device__ __forceinline__ bool init(const FlashParams& p, const FlashItem& w, int32_t* sbt, int k0, int k1,
+                                       int Lk, int wave, int lane) {
+    kb = p.k + w.kvh * p.ks1;
+    vb = p.v + w.kvh * p.vs1;
+    row = p.bt + (int64_t)w.b * p.max_blocks;
+    ids = sbt;
+    last_key = max(Lk - 1, 0);
+    blk_lo = (int)fdiv((uint32_t)k0, p.bsdiv);
+    const int n = k1 > k0 ? (int)fdiv((uint32_t)(k1 - 1), p.bsdiv) - blk_lo + 1 : 0;
+    int bad = 0;
+    for (int x = threadIdx.x; x < n; x += 256) {
+      const int id = row[blk_lo + x];
+      const bool ok = (uint32_t)id < (uint32_t)p.num_blocks;
+      bad |= !ok;
+      if (x < kFlashIds) sbt[x] = ok ? id : 0;
+    }
+    bad = __syncthreads_or(bad);
+    win = blk_lo - 64;  // empty
+    win_id = 0;
+    // byte offsets within a block and the block strides fit 32 bits
+    uni = p.block_size % WR == 0 && max(p.ks0, p.vs0) < ((int64_t)1 << 31) &&
+          max(p.ks2, p.vs2) < ((int64_t)1 << 30) / p.block_size;
+#pragma unroll
+    for (int j = 0; j < C::NW; ++j) {
+      const int P = (wave * C::NW + j) * 64 + lane;
+      lrow[j] = P / C::S;
+      lchk[j] = 8 * ((P % C::S) ^ chunk_swizzle<C::S>(lrow[j]));
+      const int r = j * RPI + lane / C::S;  // row among the wave's
+      koff[j] = uni ? 2u * ((uint32_t)r * (uint32_t)p.ks2 + lchk[j]) : 0u;
+      voff[j] = uni ? 2u * ((uint32_t)r * (uint32_t)p.vs2 + lchk[j]) : 0u;
+    }
+    return bad != 0;
+  }
+  // Copies of the tile of keys [n0, n0 + BN) to the stage at LDS byte address
+  // st (this wave's part of it). Rows past the last key repeat it.
+  __device__ __forceinline__ void issue(const FlashParams& p, int n0, uint32_t st, int wave, int lane) {
+    const int blk_hi = (int)fdiv((uint32_t)min(n0 + C::BN - 1, last_key), p.bsdiv);
+    if (uni && n0 + C::BN - 1 <= last_key && blk_hi - blk_lo < kFlashIds) {
+      const uint32_t key = (uint32_t)__builtin_amdgcn_readfirstlane(n0 + wave * WR);
+      const uint32_t blk = fdiv(key, p.bsdiv);
+      if ((int)blk - win >= 64) {  // blocks ascend
+        win = (int)blk;
+        win_id = ids[min((int)blk - blk_lo + lane, kFlashIds - 1)];
+      }
+      const uint32_t off = key - blk * (uint32_t)p.block_size;
+      const uint64_t bid = (uint32_t)__builtin_amdgcn_readlane(win_id, (int)blk - win);
+      const void* kt = uniform_ptr(reinterpret_cast<const char*>(kb) + bid * (uint32_t)(2 * p.ks0) + off * (uint32_t)(2 * p.ks2));
+      const void* vt = uniform_ptr(reinterpret_cast<const char*>(vb) + bid * (uint32_t)(2 * p.vs0) + off * (uint32_t)(2 * p.vs2));
+#pragma unroll
+      for (int j = 0; j < C::NW; ++j) {
+        dma16_sv(kt, koff[j], st + 1024u * j);
+        dma16_sv(vt, voff[j], st + 2u * C::TILE + 1024u * j);
+      }
+    } else if (blk_hi - blk_lo < kFlashIds) {
+#pragma unroll
+      for (int j = 0; j < C::NW; ++j) {
+        const int key = min(n0 + lrow[j], last_key);
+        const int blk = (int)fdiv((uint32_t)key, p.bsdiv);
+        const int64_t off = key - blk * p.block_size, bid = ids[blk - blk_lo];
+        dma16_at(kb + bid * p.ks0 + off * p.ks2 + lchk[j], st + 1024u * j);
+        dma16_at(vb + bid * p.vs0 + off * p.vs2 + lchk[j], st + 2u * C::TILE + 1024u * j);
+      }
+    } else {  // past the staged ids: straight from the table (waits for the copies in flight)
+#pragma unroll
+      for (int j = 0; j < C::NW; ++j) {
+        const int key = min(n0 + lrow[j], last_key);
+        const int blk = (int)fdiv((uint32_t)key, p.bsdiv);
+        const int raw = row[blk];
+        const int64_t off = key - blk * p.block_size;
+        const int64_t bid = (uint32_t)raw < (uint32_t)p.num_blocks ? raw : 0;
+        dma16_at(kb + bid * p.ks0 + off * p.ks2 + lchk[j], st + 1024u * j);
+        dma16_at(vb + bid * p.vs0 + off * p.vs2 + lchk[j], st + 2u * C::TILE + 1024u * j);
+      }
+    }
+  }
+};
+
+// Partial state of one work item (p.part): the accumulator of each wave in
+// lane order (float4 slot x of lane l holds columns 8x + 4 (l / 32) .. +3 of
+// row l % 32: every store instruction writes 1 KiB in a row), then, after the
+// accumulators of all items, (reference max, row sum) of its 128 rows.
+__device__ __forceinline__ int64_t flash_part_item(const FlashParams& p, int b, int hq, int mt, int sp) {
+  return (((int64_t)b * p.Hq + hq) * p.n_mt + mt) * p.splits + sp;
+}
+template <int D>
+__device__ __forceinline__ float* flash_part_acc(const FlashParams& p, int64_t item) {
+  return p.part + item * (128 * D);
+}
+template <int D>
+__device__ __forceinline__ float2* flash_part_ml(const FlashParams& p, int64_t item) {
+  const int64_t items = (int64_t)p.B * p.Hq * p.n_mt * p.splits;
+  return reinterpret_cast<float2*>(p.part + items * (128 * D)) + item * 128;
+}
+template <int D, typename Acc>
+__device__ __forceinline__ void flash_store_partial(const FlashParams& p, const FlashItem& w, int wave, int lane,
+                                                    const Acc& acc, float m, float l) {
+  const int64_t item = flash_part_item(p, w.b, w.hq, w.mt, w.sp);
+  float* sl = flash_part_acc<D>(p, item) + wave * (32 * D) + 4 * lane;
+#pragma unroll
+  for (int x = 0; x < D / 8; ++x) {
+    const int dt = x / 4, g4 = x % 4;
+    *reinterpret_cast<float4*>(sl + 256 * x) =
+        float4{acc[dt][4 * g4], acc[dt][4 * g4 + 1], acc[dt][4 * g4 + 2], acc[dt][4 * g4 + 3]};
+  }
+  if (lane < 32) flash_part_ml<D>(p, item)[32 * wave + lane] = float2{m, l};
+}
+
 // vm_wait for the copies of `ahead` tiles issued after the one needed.
 template <int NST, int PER_TILE>
 __device__ __forceinline__ void wait_ahead(int ahead) {
@@ -103,30 +276,31 @@ __device__ __forceinline__ void wait_ahead(int ahead) {
   else vm_wait<0>();
 }
 
-template <int DTYPE, int D>
+template <int DTYPE, int D, int MODE>
 __global__ __launch_bounds__(256, FlashCfg<D>::OCC) void flash_fwd_kernel(const FlashParams p) {
   using C = FlashCfg<D>;
   using E = Elt<DTYPE>;
   constexpr int BN = C::BN;
   __shared__ __attribute__((aligned(16))) uint16_t ring[C::NST * C::STAGE];
 
-  // Workgroups are dispatched round-robin over the XCDs; give each XCD a
-  // contiguous run of logical tiles so the query heads of a kv head (and its
-  // neighbouring query tiles) share one L2. Within a kv head the longest
-  // (last) query tiles go first.
-  const int logical = xcd_logical(blockIdx.x, p.n_wg, p.xcd_shift);
-  const int G = p.group;
-  const int per_grp = p.n_mt * G;
-  const int grp = logical / per_grp;
-  const int rem = logical - grp * per_grp;
-  const int mt = p.n_mt - 1 - rem / G;
-  const int g = rem - (rem / G) * G;
-  const int b = grp / p.Hk, kvh = grp - b * p.Hk, hq = kvh * G + g;
+  const FlashItem w = flash_item<MODE>(p);
+  const int mt = w.mt, b = w.b, kvh = w.kvh, hq = w.hq;
 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int l32 = lane & 31, hl = lane >> 5;
   const int q0w = mt * C::BM + wave * 32;  // first row of this wave
   const int qi = q0w + l32;                // row owned by this lane
+
+  // Keys of the sequence (paged: its context length; one outside [0,
+  // ctx_limit] poisons the output).
+  int Lk = p.Lk;
+  bool poison = false;
+  if constexpr (MODE == kKvPaged) {
+    const int ctx = p.lens[b];
+    poison = ctx < 0 || ctx > p.ctx_limit || (ctx > 0 && p.num_blocks < 1);
+    Lk = poison ? 0 : ctx;
+  }
+  const bool no_keys = Lk == 0;
 
   // Q^T as the B operand: lane holds Q[qi][16kk + 8hl .. +8], its sign
   // flipped when the caller's scale is negative (p.scale_log2 is |scale| *
@@ -135,28 +309,42 @@ __global__ __launch_bounds__(256, FlashCfg<D>::OCC) void flash_fwd_kernel(const 
   u32x4 qf[C::KK];
 #pragma unroll
   for (int kk = 0; kk < C::KK; ++kk) qf[kk] = load16(qrow + 16 * kk + 8 * hl, qi < p.Lq);
-  if (p.rope.cos)  // RoPE fused into the load: row qi at position q_pos0[b] + qi
-    rope_q_lane<DTYPE, D>(qf, p.rope, (p.q_pos0 ? p.q_pos0[b] : 0) + qi, qi < p.Lq, hl);
+  if (p.rope.cos) {  // RoPE fused into the load: row qi at position q_pos0[b] + qi (paged: among the newest Lq)
+    const int pos0 = MODE == kKvPaged ? Lk - p.Lq : (p.q_pos0 ? p.q_pos0[b] : 0);
+    rope_q_lane<DTYPE, D>(qf, p.rope, pos0 + qi, qi < p.Lq, hl);
+  }
   const float c = p.scale_log2;
 #pragma unroll
   for (int kk = 0; kk < C::KK; ++kk) qf[kk] ^= u32x4{p.q_sign, p.q_sign, p.q_sign, p.q_sign};
 
   // Key range of the workgroup and of this wave; lim = last key this row sees.
   const int wg_last_row = min(p.Lq, mt * C::BM + C::BM) - 1;
-  int kend = p.Lk;
-  if (p.causal) kend = max(0, min(p.Lk, p.Lk - p.Lq + wg_last_row + 1));
+  int kend = Lk;
+  if (p.causal) kend = max(0, min(Lk, Lk - p.Lq + wg_last_row + 1));
   int wave_kend = 0;
   if (q0w < p.Lq) {
-    wave_kend = p.Lk;
-    if (p.causal) wave_kend = max(0, min(p.Lk, p.Lk - p.Lq + min(q0w + 31, p.Lq - 1) + 1));
+    wave_kend = Lk;
+    if (p.causal) wave_kend = max(0, min(Lk, Lk - p.Lq + min(q0w + 31, p.Lq - 1) + 1));
   }
-  const int lim = p.causal ? min(p.Lk - 1, p.Lk - p.Lq + qi) : p.Lk - 1;
-  const int wave_lim0 = p.causal ? min(p.Lk - 1, p.Lk - p.Lq + q0w) : p.Lk - 1;  // smallest lim in the wave
-  const int n_tiles = (kend + BN - 1) / BN;
+  int lim = p.causal ? min(Lk - 1, Lk - p.Lq + qi) : Lk - 1;
+  int wave_lim0 = p.causal ? min(Lk - 1, Lk - p.Lq + q0w) : Lk - 1;  // smallest lim in the wave
+  int n_tiles = (kend + BN - 1) / BN;
+  // With splits this workgroup takes tiles [t0, t1); from here on tiles and
+  // keys count from its first key.
+  int k_lo = 0;
+  if (MODE != kKvDense && p.splits > 1) {
+    const int t0 = (int)((int64_t)w.sp * n_tiles / p.splits), t1 = (int)((int64_t)(w.sp + 1) * n_tiles / p.splits);
+    k_lo = t0 * BN;
+    n_tiles = t1 - t0;
+    Lk -= k_lo;
+    lim -= k_lo;
+    wave_lim0 -= k_lo;
+    wave_kend = min(wave_kend - k_lo, n_tiles * BN);
+  }
 
-  const uint16_t* kb = p.k + b * p.ks0 + kvh * p.ks1;
-  const uint16_t* vb = p.v + b * p.vs0 + kvh * p.vs1;
-  const int last_key = max(p.Lk - 1, 0);
+  const uint16_t* kb = p.k + b * p.ks0 + kvh * p.ks1 + k_lo * p.ks2;
+  const uint16_t* vb = p.v + b * p.vs0 + kvh * p.vs1 + k_lo * p.vs2;
+  const int last_key = max(Lk - 1, 0);
 
   // Tile copy: copy j of this wave moves 16-byte chunk P = (wave*NW + j)*64 + lane
   // of the tile, i.e. row P / S, chunk (P % S) XOR chunk_swizzle(row). Rows
@@ -178,11 +366,16 @@ __global__ __launch_bounds__(256, FlashCfg<D>::OCC) void flash_fwd_kernel(const 
     koff[j] = off32 ? (uint32_t)(2 * ((int64_t)lrow[j] * p.ks2 + lchk[j])) : 0u;
     voff[j] = off32 ? (uint32_t)(2 * ((int64_t)lrow[j] * p.vs2 + lchk[j])) : 0u;
   }
+  __shared__ int32_t sbt[MODE == kKvPaged ? kFlashIds : 1];
+  PagedTiles<C> pt;
+  if constexpr (MODE == kKvPaged) poison |= pt.init(p, w, sbt, k_lo, min(k_lo + n_tiles * BN, k_lo + Lk), k_lo + Lk, wave, lane);
   const uint32_t ring_lds = lds_addr_of(ring);
   auto issue = [&](int t) CIE_INLINE {
     const int n0 = t * BN;
     const uint32_t st = ring_lds + 2u * (uint32_t)((t % C::NST) * C::STAGE + wave * C::NW * 512);
-    if (off32 && n0 + BN <= p.Lk) {
+    if constexpr (MODE == kKvPaged) {
+      pt.issue(p, k_lo + n0, st, wave, lane);
+    } else if (off32 && n0 + BN <= Lk) {
       const void* kt = uniform_ptr(kb + (int64_t)n0 * p.ks2);
       const void* vt = uniform_ptr(vb + (int64_t)n0 * p.vs2);
 #pragma unroll
@@ -407,8 +600,15 @@ __global__ __launch_bounds__(256, FlashCfg<D>::OCC) void flash_fwd_kernel(const 
 
   // Epilogue: rows with keys but none visible give 0 * inf = NaN like the
   // reference's softmax over an all -inf row; Lk == 0 gives zeros.
-  const float l_tot = l;  // l sums both lanes of the row
-  const float inv = p.Lk == 0 ? 0.f : 1.f / l_tot;
+  // (l sums both lanes of the row; a partial keeps reference 0 when its first
+  // tile had only -inf scores)
+  if (MODE != kKvDense && p.splits > 1) {
+    if (qi < p.Lq)
+      flash_store_partial<D>(p, w, wave, lane, acc, m == -INFINITY && l > 0.f ? 0.f : m, poison ? __builtin_nanf("") : l);
+    return;
+  }
+  float inv = no_keys ? 0.f : 1.f / l;
+  if (MODE == kKvPaged && poison) inv = __builtin_nanf("");
   if (qi < p.Lq) {
     uint16_t* orow = p.o + b * p.os0 + hq * p.os1 + (int64_t)qi * p.os2;
 #pragma unroll
@@ -485,52 +685,72 @@ __device__ __forceinline__ void wait_tiles(int k) {
   vm_wait<0>();
 }
 
-template <int DTYPE, int D>
+template <int DTYPE, int D, int MODE>
 __global__ __launch_bounds__(256, 2) void flash_fwd_il_kernel(const FlashParams p) {
   using C = IlCfg<D>;
   using E = Elt<DTYPE>;
   constexpr int BN = C::BN;
   __shared__ __attribute__((aligned(16))) uint16_t ring[C::NST * C::STAGE];
 
-  const int logical = xcd_logical(blockIdx.x, p.n_wg, p.xcd_shift);
-  const int G = p.group;
-  const int per_grp = p.n_mt * G;
-  const int grp = logical / per_grp;
-  const int rem = logical - grp * per_grp;
-  const int mt = p.n_mt - 1 - rem / G;
-  const int g = rem - (rem / G) * G;
-  const int b = grp / p.Hk, kvh = grp - b * p.Hk, hq = kvh * G + g;
+  const FlashItem w = flash_item<MODE>(p);
+  const int mt = w.mt, b = w.b, kvh = w.kvh, hq = w.hq;
 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int l32 = lane & 31, hl = lane >> 5;
   const int q0w = mt * C::BM + wave * 32;
   const int qi = q0w + l32;
 
+  // Keys of the sequence (paged: its context length; one outside [0,
+  // ctx_limit] poisons the output).
+  int Lk = p.Lk;
+  bool poison = false;
+  if constexpr (MODE == kKvPaged) {
+    const int ctx = p.lens[b];
+    poison = ctx < 0 || ctx > p.ctx_limit || (ctx > 0 && p.num_blocks < 1);
+    Lk = poison ? 0 : ctx;
+  }
+  const bool no_keys = Lk == 0;
+
   const uint16_t* qrow = p.q + b * p.qs0 + hq * p.qs1 + (int64_t)qi * p.qs2;
   u32x4 qf[C::KK];
 #pragma unroll
   for (int kk = 0; kk < C::KK; ++kk) qf[kk] = load16(qrow + 16 * kk + 8 * hl, qi < p.Lq);
-  if (p.rope.cos) rope_q_lane<DTYPE, D>(qf, p.rope, (p.q_pos0 ? p.q_pos0[b] : 0) + qi, qi < p.Lq, hl);
+  if (p.rope.cos) {
+    const int pos0 = MODE == kKvPaged ? Lk - p.Lq : (p.q_pos0 ? p.q_pos0[b] : 0);
+    rope_q_lane<DTYPE, D>(qf, p.rope, pos0 + qi, qi < p.Lq, hl);
+  }
 #pragma unroll
   for (int kk = 0; kk < C::KK; ++kk) qf[kk] ^= u32x4{p.q_sign, p.q_sign, p.q_sign, p.q_sign};
   const float c = p.scale_log2;
 
   const int wg_last_row = min(p.Lq, mt * C::BM + C::BM) - 1;
-  int kend = p.Lk;
-  if (p.causal) kend = max(0, min(p.Lk, p.Lk - p.Lq + wg_last_row + 1));
+  int kend = Lk;
+  if (p.causal) kend = max(0, min(Lk, Lk - p.Lq + wg_last_row + 1));
   int wave_kend = 0;
   if (q0w < p.Lq) {
-    wave_kend = p.Lk;
-    if (p.causal) wave_kend = max(0, min(p.Lk, p.Lk - p.Lq + min(q0w + 31, p.Lq - 1) + 1));
+    wave_kend = Lk;
+    if (p.causal) wave_kend = max(0, min(Lk, Lk - p.Lq + min(q0w + 31, p.Lq - 1) + 1));
   }
-  const int lim = p.causal ? min(p.Lk - 1, p.Lk - p.Lq + qi) : p.Lk - 1;
-  const int wave_lim0 = p.causal ? min(p.Lk - 1, p.Lk - p.Lq + q0w) : p.Lk - 1;
-  const int n_tiles = (kend + BN - 1) / BN;
-  const int wave_nt = (wave_kend + BN - 1) / BN;  // tiles this wave needs (0: no rows)
+  int lim = p.causal ? min(Lk - 1, Lk - p.Lq + qi) : Lk - 1;
+  int wave_lim0 = p.causal ? min(Lk - 1, Lk - p.Lq + q0w) : Lk - 1;
+  int n_tiles = (kend + BN - 1) / BN;
+  // With splits this workgroup takes tiles [t0, t1); from here on tiles and
+  // keys count from its first key.
+  int k_lo = 0;
+  if (MODE != kKvDense && p.splits > 1) {
+    const int t0 = (int)((int64_t)w.sp * n_tiles / p.splits), t1 = (int)((int64_t)(w.sp + 1) * n_tiles / p.splits);
+    k_lo = t0 * BN;
+    n_tiles = t1 - t0;
+    Lk -= k_lo;
+    lim -= k_lo;
+    wave_lim0 -= k_lo;
+    wave_kend = min(wave_kend - k_lo, n_tiles * BN);
+  }
+  const int wave_nt = max(0, wave_kend + BN - 1) / BN;  // tiles this wave needs (0: no rows)
 
-  const uint16_t* kb = p.k + b * p.ks0 + kvh * p.ks1;
-  const uint16_t* vb = p.v + b * p.vs0 + kvh * p.vs1;
-  const int last_key = max(p.Lk - 1, 0);
+  const uint16_t* kb = p.k + b * p.ks0 + kvh * p.ks1 + k_lo * p.ks2;
+  const uint16_t* vb = p.v + b * p.vs0 + kvh * p.vs1 + k_lo * p.vs2;
+  const int last_key = max(Lk - 1, 0);
 
   int lrow[C::NW], lchk[C::NW];
 #pragma unroll
@@ -546,11 +766,16 @@ __global__ __launch_bounds__(256, 2) void flash_fwd_il_kernel(const FlashParams 
     koff[j] = off32 ? (uint32_t)(2 * ((int64_t)lrow[j] * p.ks2 + lchk[j])) : 0u;
     voff[j] = off32 ? (uint32_t)(2 * ((int64_t)lrow[j] * p.vs2 + lchk[j])) : 0u;
   }
+  __shared__ int32_t sbt[MODE == kKvPaged ? kFlashIds : 1];
+  PagedTiles<C> pt;
+  if constexpr (MODE == kKvPaged) poison |= pt.init(p, w, sbt, k_lo, min(k_lo + n_tiles * BN, k_lo + Lk), k_lo + Lk, wave, lane);
   const uint32_t ring_lds = lds_addr_of(ring);
   auto issue = [&](int t) CIE_INLINE {
     const int n0 = t * BN;
     const uint32_t st = ring_lds + 2u * (uint32_t)((t % C::NST) * C::STAGE + wave * C::NW * 512);
-    if (off32 && n0 + BN <= p.Lk) {
+    if constexpr (MODE == kKvPaged) {
+      pt.issue(p, k_lo + n0, st, wave, lane);
+    } else if (off32 && n0 + BN <= Lk) {
       const void* kt = uniform_ptr(kb + (int64_t)n0 * p.ks2);
       const void* vt = uniform_ptr(vb + (int64_t)n0 * p.vs2);
 #pragma unroll
@@ -780,7 +1005,13 @@ __global__ __launch_bounds__(256, 2) void flash_fwd_il_kernel(const FlashParams 
 
   // Epilogue: rows with keys but none visible give 0 * inf = NaN like the
   // reference's softmax over an all -inf row; Lk == 0 gives zeros.
-  const float inv = p.Lk == 0 ? 0.f : 1.f / l;
+  if (MODE != kKvDense && p.splits > 1) {
+    if (qi < p.Lq)
+      flash_store_partial<D>(p, w, wave, lane, acc, m == -INFINITY && l > 0.f ? 0.f : m, poison ? __builtin_nanf("") : l);
+    return;
+  }
+  float inv = no_keys ? 0.f : 1.f / l;
+  if (MODE == kKvPaged && poison) inv = __builtin_nanf("");
   if (qi < p.Lq) {
     uint16_t* orow = p.o + b * p.os0 + hq * p.os1 + (int64_t)qi * p.os2;
 #pragma unroll
@@ -794,6 +1025,63 @@ __global__ __launch_bounds__(256, 2) void flash_fwd_il_kernel(const FlashParams 
       }
     }
   }
+}
+
+// ---------------------------------------------------------------------------
+// Second pass of a launch with splits: one thread per (query tile, wave,
+// accumulator slot, lane) combines that lane's four columns over the splits,
+// in split order. Every load is 16 contiguous bytes per lane of one partial.
+constexpr int kMergeAhead = 4;  // partials loaded together
+
+template <int DTYPE, int D>
+__global__ __launch_bounds__(256) void flash_merge_kernel(const FlashParams p) {
+  using E = Elt<DTYPE>;
+  constexpr int SL = D / 8;
+  const int lane = threadIdx.x & 63;
+  const uint32_t unit = blockIdx.x * 4u + (threadIdx.x >> 6);  // (item, wave, slot) of this wavefront
+  const uint32_t x = unit % SL;
+  const uint32_t rest = unit / SL;
+  const uint32_t nw = (uint32_t)(min(p.Lq, 128) + 31) / 32;  // waves of a query tile that can hold rows
+  const uint32_t wave = rest % nw, tile = rest / nw;
+  if (tile >= (uint32_t)(p.B * p.Hq * p.n_mt)) return;
+  const int mt = (int)(tile % p.n_mt), bh = (int)(tile / p.n_mt);
+  const int b = bh / p.Hq, hq = bh - b * p.Hq;
+  const int row = mt * 128 + (int)wave * 32 + (lane & 31);
+  if (row >= p.Lq) return;
+  const int64_t item0 = flash_part_item(p, b, hq, mt, 0);
+  const float* sl = flash_part_acc<D>(p, item0) + wave * (32 * D) + 256 * x + 4 * lane;
+  const float2* ml = flash_part_ml<D>(p, item0) + wave * 32 + (lane & 31);
+  float M = -INFINITY, L = 0.f;
+  float4 A = {0.f, 0.f, 0.f, 0.f};
+  for (int s0 = 0; s0 < p.splits; s0 += kMergeAhead) {
+    float4 a[kMergeAhead];
+    float2 st[kMergeAhead];
+#pragma unroll
+    for (int u = 0; u < kMergeAhead; ++u) {
+      const int s = min(s0 + u, p.splits - 1);
+      a[u] = *reinterpret_cast<const float4*>(sl + (int64_t)s * (128 * D));
+      st[u] = ml[(int64_t)s * 128];
+    }
+#pragma unroll
+    for (int u = 0; u < kMergeAhead; ++u) {
+      if (s0 + u < p.splits) {
+        const float Mn = maxf(M, st[u].x);
+        const float wo = rescale_weight(M, Mn), wn = rescale_weight(st[u].x, Mn);
+        L = L * wo + st[u].y * wn;
+        A.x = A.x * wo + a[u].x * wn;
+        A.y = A.y * wo + a[u].y * wn;
+        A.z = A.z * wo + a[u].z * wn;
+        A.w = A.w * wo + a[u].w * wn;
+        M = Mn;
+      }
+    }
+  }
+  // rows with keys but none visible give 0 * inf = NaN, an empty history zeros
+  // (an invalid length left NaN sums)
+  float inv = 1.f / L;
+  if (p.lens ? p.lens[b] == 0 : p.Lk == 0) inv = 0.f;
+  uint16_t* orow = p.o + b * p.os0 + hq * p.os1 + (int64_t)row * p.os2 + 8 * x + 4 * (lane >> 5);
+  *reinterpret_cast<u32x2*>(orow) = u32x2{E::pack2(A.x * inv, A.y * inv), E::pack2(A.z * inv, A.w * inv)};
 }
 
 // ---------------------------------------------------------------------------
@@ -1282,21 +1570,74 @@ FlashKernel flash_kernel_choice(const FlashParams& p, int D) {
   return kFlash32;
 }
 
+// Key splits of a launch of flash_fwd_kernel / flash_fwd_il_kernel (a pure
+// function of the arguments, and of B * Hq rather than the group size, so GQA
+// and its expanded MHA get the same arithmetic). Without splits a launch of
+// few query tiles leaves most of the GPU idle while each workgroup walks its
+// keys alone; with them every partial state is written and read once more. The
+// estimate, in microseconds: a workgroup walks its tiles at kStep each (25 %
+// slower when the waves of two workgroups share a CU; one wave of a short query
+// tile does not notice), launches in rounds of the workgroup slots, and a
+// split launch pays 4.2 us and 0.3 us per split for its second pass plus its
+// partial states at 1.6 MB/us. Measured, splits: us (B x Hq x Lq x Lk, D, causal):
+//   1x32x5x3001 D=64      1: 35.3  2: 22.5  4: 14.8  8: 11.9  16: 13.3
+//   1x32x5x300 D=64       1: 6.7   2: 8.4   4: 8.1
+//   1x32x5x16384 D=128    1: 260   4: 71.6  8: 40.7  16: 28.1
+//   1x32x300x1500 D=64    1: 21.9  2: 19.3  4: 18.9  8: 24.8
+//   1x32x1000x4600 D=128  1: 87.4  2: 78.2  3: 88.4  4: 84.6
+//   1x16x512x512 D=64     1: 10.0  2: 11.8  4: 13.3
+//   1x32x500x500 D=128    1: 14.6  2: 22.7
+int flash_splits(const FlashParams& p, int D) {
+  const int bn = D <= 32 ? 128 : (D == 64 ? 64 : 32);
+  const double kStep = D == 256 ? 1.35 : D == 128 ? 0.6 : D == 64 ? 0.75 : 1.05;
+  const int64_t items = p.n_wg, per_cu = D <= 128 ? 2 : 1, slots = per_cu * p.cus;
+  const int64_t nt = ((int64_t)p.Lk + bn - 1) / bn;  // tiles of the longest item
+  if (items < 1 || items >= slots) return 1;
+  const double mb = (double)p.B * p.Hq * p.Lq * (D + 2) * 4e-6;  // partial states of one split
+  auto cost = [&](int64_t s) {
+    const int64_t wg = items * s, rounds = (wg + slots - 1) / slots;
+    const double step = kStep * (wg > p.cus && p.Lq > 32 ? 1.25 : 1.0);
+    return (double)(rounds * ((nt + s - 1) / s)) * step + (s > 1 ? 4.2 + 0.3 * s + mb * s / 1.6 : 0.0);
+  };
+  int best = 1;
+  double best_us = 0.95 * (cost(1) + 3.0);  // a split has to pay by more than the estimate's noise
+  for (int s = 2; s <= kFlashMaxSplits && 2 * s <= nt; ++s)
+    if (cost(s) + 3.0 < best_us) best = s, best_us = cost(s) + 3.0;
+  return best;
+}
+
+size_t flash_part_bytes(const FlashParams& p, int D, int splits) {
+  if (splits <= 1) return 0;
+  return (size_t)p.n_wg * splits * (128 * D + 256) * sizeof(float);  // p.n_wg = B * Hq * n_mt items
+}
+
+template <int DTYPE, int D, int MODE>
+static hipError_t launch_mode(const FlashParams& p, hipStream_t stream) {
+  FlashParams q = p;
+  q.n_wg = p.n_wg * p.splits;
+  if constexpr (D == 128)
+    hipLaunchKernelGGL((flash_fwd_il_kernel<DTYPE, D, MODE>), dim3(q.n_wg), dim3(256), 0, stream, q);
+  else
+    hipLaunchKernelGGL((flash_fwd_kernel<DTYPE, D, MODE>), dim3(q.n_wg), dim3(256), 0, stream, q);
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess || p.splits <= 1) return e;
+  const int64_t units = (int64_t)p.n_wg * ((std::min(p.Lq, 128) + 31) / 32) * (D / 8);
+  hipLaunchKernelGGL((flash_merge_kernel<DTYPE, D>), dim3((unsigned)((units + 3) / 4)), dim3(256), 0, stream, p);
+  return hipGetLastError();
+}
+
 template <int DTYPE, int D>
 static hipError_t launch_flash_t(const FlashParams& p, hipStream_t stream) {
+  if (p.bt) return launch_mode<DTYPE, D, kKvPaged>(p, stream);
+  if (p.splits > 1) return launch_mode<DTYPE, D, kKvSplit>(p, stream);
   switch (flash_kernel_choice(p, D)) {
-    case kFlashIl:
-      if constexpr (D == 128) hipLaunchKernelGGL((flash_fwd_il_kernel<DTYPE, D>), dim3(p.n_wg), dim3(256), 0, stream, p);
-      break;
     case kFlashR64Heads:
       if constexpr (D == 64) launch_r64<DTYPE, D, true>(p, stream);
       break;
     case kFlashR64Rows:
       if constexpr (D == 64) launch_r64<DTYPE, D, false>(p, stream);
       break;
-    default:
-      if constexpr (D != 128) hipLaunchKernelGGL((flash_fwd_kernel<DTYPE, D>), dim3(p.n_wg), dim3(256), 0, stream, p);
-      break;
+    default: return launch_mode<DTYPE, D, kKvDense>(p, stream);
   }
   return hipGetLastError();
 }

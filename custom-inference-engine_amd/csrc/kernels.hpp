@@ -48,7 +48,7 @@ struct FlashParams {
   int64_t os0, os1, os2;
   int B, Hq, Hk, Lq, Lk, group;
   int n_mt;  // query tiles of 128 rows (the launcher recounts them for kernels with other tiles)
-  int n_wg;  // B * Hq * n_mt
+  int n_wg;  // B * Hq * n_mt (the kernels: times splits)
   float scale_log2;  // |scale| * log2(e), never below 1e-30
   uint32_t q_sign;   // 0x80008000 flips the sign of q when the caller's scale is negative
   int causal;
@@ -56,7 +56,22 @@ struct FlashParams {
   const int32_t* q_pos0;  // [B] or nullptr (position = row)
   int cus;                // compute units of the device (kernel choice)
   int xcd_shift;          // log2 of its XCDs (workgroup placement)
+  int splits;             // key splits (1: none); a split launch leaves partial states in part and merges them
+  float* part;            // see flash_part_item
+  // Paged K/V (bt != nullptr): k and v are a (num_blocks, block_size, Hk, D)
+  // pool with strides ks0 per block, ks1 per head, ks2 per token; sequence b
+  // holds lens[b] tokens, the Lq query rows its newest, in the blocks of row
+  // b of the block table. Lk is then the largest valid length.
+  const int32_t* bt;
+  const int32_t* lens;
+  int max_blocks, num_blocks, block_size, ctx_limit;
+  FastDiv bsdiv;
 };
+constexpr int kFlashIds = 1024;       // block ids of a workgroup's key range staged in LDS
+constexpr int kFlashMaxSplits = 32;
+// Splits of a launch (p.n_wg = B * Hq * n_mt, p.Lk the most keys a row sees) and the bytes of its partial states.
+int flash_splits(const FlashParams& p, int D);
+size_t flash_part_bytes(const FlashParams& p, int D, int splits);
 
 // Prefill kernel a launch takes (launch_flash); cie_prefill_kernel reports it.
 enum FlashKernel { kFlash32 = 0, kFlashR64Heads = 1, kFlashR64Rows = 2, kFlashIl = 3 };

@@ -34,6 +34,10 @@ EXPORTED_SYMBOLS = (
     "cie_device_cus",
     "cie_prefill_kernel",
     "cie_flash_fwd",
+    "cie_flash_workspace_bytes",
+    "cie_flash_fwd_ex",
+    "cie_flash_paged_workspace_bytes",
+    "cie_flash_paged",
     "cie_paged_workspace_bytes",
     "cie_paged_fwd",
     "cie_paged_fwd_noalloc",
@@ -76,6 +80,18 @@ def _declare(lib: ctypes.CDLL) -> None:
     lib.cie_flash_fwd.argtypes = [_vp, _vp, _vp, _vp, _i64p, _i64p, _i64p, _i64p,
                                   _i, _i, _i, _i, _i, _i, ctypes.c_float, _i, _i, _vp]
     lib.cie_flash_fwd.restype = _i
+    lib.cie_flash_workspace_bytes.argtypes = [_i, _i, _i, _i, _i, _i, _i, _i]
+    lib.cie_flash_workspace_bytes.restype = ctypes.c_size_t
+    lib.cie_flash_fwd_ex.argtypes = [_vp, _vp, _vp, _vp, _i64p, _i64p, _i64p, _i64p,
+                                     _i, _i, _i, _i, _i, _i, ctypes.c_float, _i, _i, _vp, _vp, _i, _i, _vp,
+                                     _i, _vp, ctypes.c_size_t, _vp]
+    lib.cie_flash_fwd_ex.restype = _i
+    lib.cie_flash_paged_workspace_bytes.argtypes = [_i, _i, _i, _i, _i, _i, _i, _i, _i]
+    lib.cie_flash_paged_workspace_bytes.restype = ctypes.c_size_t
+    lib.cie_flash_paged.argtypes = [_vp, _vp, _vp, _vp, _vp, _vp, _i64p, _i64p, _i64p, _i64p,
+                                    _i, _i, _i, _i, _i, _i, _i, _i, _i, ctypes.c_float, _i, _i,
+                                    _vp, _vp, _i, _i, _i, _vp, ctypes.c_size_t, _vp]
+    lib.cie_flash_paged.restype = _i
     lib.cie_paged_workspace_bytes.argtypes = [_i, _i, _i, _i, _i, _i, _i, _i]
     lib.cie_paged_workspace_bytes.restype = ctypes.c_size_t
     lib.cie_paged_fwd.argtypes = [_vp, _vp, _vp, _vp, _vp, _vp, _vp, ctypes.c_size_t,

@@ -14,6 +14,7 @@ Both accept fp16 and bf16 (the reference accepts fp16 only,
 from __future__ import annotations
 
 import ctypes
+import functools
 import math
 from dataclasses import dataclass
 
@@ -130,26 +131,103 @@ def flash_attention(
     lib = _lib.load()
     q, k, v = _kernel_layout(q), _kernel_layout(k), _kernel_layout(v)
     out = _output(out, (B, H, M, D), q)
+    rp = (None, None, 0, 0)
+    pos_p = None
+    if rope is not None:
+        rp = rope_args(rope, D, q.device)
+        if q_pos0 is not None:
+            if not q_pos0.is_cuda or q_pos0.device != q.device or q_pos0.dtype != torch.int32 \
+                    or q_pos0.shape != (B,) or not q_pos0.is_contiguous():
+                raise ValueError("q_pos0 must be a contiguous int32 (B,) tensor on q's device")
+            pos_p = q_pos0.data_ptr()
     with torch.cuda.device(q.device):
-        if rope is None:
-            rc = lib.cie_flash_fwd(
-                q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(),
+        args = (q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(),
                 _lib.strides(q), _lib.strides(k), _lib.strides(v), _lib.strides(out),
-                B, H, Hk, M, N, D, float(scale), 1 if causal else 0,
-                _lib.DTYPE_CODES[q.dtype], _lib.stream_handle(q.device))
+                B, H, Hk, M, N, D, float(scale), 1 if causal else 0, _lib.DTYPE_CODES[q.dtype])
+        # few query tiles over many keys: the library cuts the keys into runs,
+        # whose partial states need a workspace of this call's own
+        ws, nbytes = _split_workspace(_flash_workspace_bytes(q.device.index, B, H, Hk, M, N, D, bool(causal)), q)
+        if ws is not None:
+            rc = lib.cie_flash_fwd_ex(*args, *rp, pos_p, 0, ws.data_ptr(), nbytes, _lib.stream_handle(q.device))
+        elif rope is not None:
+            rc = lib.cie_flash_fwd_rope(*args, *rp, pos_p, _lib.stream_handle(q.device))
         else:
-            cos_p, sin_p, rows, tdt = rope_args(rope, D, q.device)
-            pos_p = None
-            if q_pos0 is not None:
-                if not q_pos0.is_cuda or q_pos0.device != q.device or q_pos0.dtype != torch.int32 \
-                        or q_pos0.shape != (B,) or not q_pos0.is_contiguous():
-                    raise ValueError("q_pos0 must be a contiguous int32 (B,) tensor on q's device")
-                pos_p = q_pos0.data_ptr()
-            rc = lib.cie_flash_fwd_rope(
-                q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(),
-                _lib.strides(q), _lib.strides(k), _lib.strides(v), _lib.strides(out),
-                B, H, Hk, M, N, D, float(scale), 1 if causal else 0,
-                _lib.DTYPE_CODES[q.dtype], cos_p, sin_p, rows, tdt, pos_p, _lib.stream_handle(q.device))
+            rc = lib.cie_flash_fwd(*args, _lib.stream_handle(q.device))
+    _lib.check(rc)
+    return out
+
+
+@functools.lru_cache(maxsize=1024)
+def _flash_workspace_bytes(device: int, B: int, H: int, Hk: int, M: int, N: int, D: int, causal: bool) -> int:
+    """``cie_flash_workspace_bytes`` of the library's own split rule on the
+    current device (``device``): a function of the shape and its CU count."""
+    return int(_lib.load().cie_flash_workspace_bytes(B, H, Hk, M, N, D, 1 if causal else 0, 0))
+
+
+def _split_workspace(nbytes: int, q: torch.Tensor) -> tuple[torch.Tensor | None, int]:
+    """Partial states of a split launch: allocated for the call (the caching
+    allocator orders its reuse on the stream), nothing when not split."""
+    if nbytes == 0:
+        return None, 0
+    return torch.empty(nbytes, dtype=torch.uint8, device=q.device), nbytes
+
+
+def paged_prefill(
+    q: torch.Tensor,
+    k_cache: torch.Tensor,
+    v_cache: torch.Tensor,
+    block_tables: torch.Tensor,
+    context_lens: torch.Tensor,
+    causal: bool = True,
+    scale: float | None = None,
+    max_context: int | None = None,
+    *,
+    rope: tuple[torch.Tensor, torch.Tensor] | None = None,
+    out: torch.Tensor | None = None,
+) -> torch.Tensor:
+    """Attention of the newest ``Lq`` tokens of each sequence over its paged
+    history with the prefill kernels (``cie_flash_paged``): any number of new
+    tokens, K and V read in place through the block tables. Arguments, result
+    and treatment of invalid lengths and block ids as in
+    :func:`paged_attention`, which is the faster one for few query rows."""
+    for name, t in (("q", q), ("k_cache", k_cache), ("v_cache", v_cache),
+                    ("block_tables", block_tables), ("context_lens", context_lens)):
+        if not t.is_cuda or t.device != q.device:
+            raise RuntimeError(f"paged_prefill requires CUDA tensors on one device ({name})")
+    if q.dim() != 4 or k_cache.dim() != 4 or v_cache.dim() != 4:
+        raise ValueError("paged_prefill expects q (B,Hq,Lq,D) and pools (num_blocks,block_size,Hk,D)")
+    B, Hq, Lq, D = q.shape
+    _check_head_dim(D)
+    _check_dtype(q)
+    if k_cache.dtype != q.dtype or v_cache.dtype != q.dtype:
+        raise ValueError(f"q and the KV pool must share a dtype, got {q.dtype}, {k_cache.dtype}, {v_cache.dtype}")
+    if tuple(k_cache.shape) != tuple(v_cache.shape) or k_cache.shape[-1] != D:
+        raise ValueError(f"pool shape mismatch: k {tuple(k_cache.shape)}, v {tuple(v_cache.shape)}, head_dim {D}")
+    num_blocks, block_size, Hk, _ = k_cache.shape
+    if Hk < 1 or Hq % Hk:
+        raise ValueError(f"num_heads {Hq} must be a multiple of num_kv_heads {Hk}")
+    if block_tables.dim() != 2 or block_tables.shape[0] != B:
+        raise ValueError(f"block_tables must be (B, max_blocks), got {tuple(block_tables.shape)}")
+    if context_lens.dim() != 1 or context_lens.shape[0] != B:
+        raise ValueError(f"context_lens must be (B,), got {tuple(context_lens.shape)}")
+    if scale is None:
+        scale = 1.0 / math.sqrt(D)
+    lib = _lib.load()
+    bt = block_tables.to(torch.int32).contiguous()
+    lens = context_lens.to(torch.int32).contiguous()
+    q, k_cache, v_cache = _kernel_layout(q), _kernel_layout(k_cache), _kernel_layout(v_cache)
+    out = _output(out, (B, Hq, Lq, D), q)
+    mc = int(max_context or 0)
+    rp = rope_args(rope, D, q.device) if rope is not None else (None, None, 0, 0)
+    with torch.cuda.device(q.device):
+        ws, nbytes = _split_workspace(lib.cie_flash_paged_workspace_bytes(B, Hq, Hk, Lq, D, mc, block_size,
+                                                                          bt.shape[1], 0), q)
+        rc = lib.cie_flash_paged(
+            q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), bt.data_ptr(), lens.data_ptr(), out.data_ptr(),
+            _lib.strides(q), _lib.strides(k_cache), _lib.strides(v_cache), _lib.strides(out),
+            B, Hq, Hk, Lq, D, num_blocks, block_size, bt.shape[1], mc, float(scale), 1 if causal else 0,
+            _lib.DTYPE_CODES[q.dtype], *rp, 0, ws.data_ptr() if ws is not None else None, nbytes,
+            _lib.stream_handle(q.device))
     _lib.check(rc)
     return out
 

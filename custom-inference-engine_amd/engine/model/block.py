@@ -17,20 +17,17 @@ each, with RoPE fused into the kernels when the model's tables are given:
   head_dim 256: ``paged_max_rows``): one rotary append, then paged attention
   reading K/V in place with q rotated as it is loaded;
 * a long chunk on top of a history (more query rows per kv head): the rotary
-  append, then paged attention in launches of at most that many rows per kv
-  head (see below) -- the history is never gathered.
+  append, then the prefill kernels over the paged history
+  (``paged_prefill``) -- the history is never gathered.
 
 :func:`attention_section_rows` takes a ragged step (a different number of
 new tokens per sequence, e.g. a prefill chunk next to decode tokens) as
-packed rows: one append for all, then paged attention per group of
-sequences with equal counts, long groups again split into launches.
+packed rows: one append for all, then one launch per group of sequences with
+equal counts, ``paged_attention`` or ``paged_prefill`` by the same bound.
 
-Splitting is exact: the Lq new tokens of a sequence of context length ctx
-sit at positions ctx - Lq .. ctx - 1 (the reference appends before it
-attends, block.py:57-65), and row i sees keys <= ctx - Lq + i. Rows i0 ..
-i1 - 1 alone are the i1 - i0 newest tokens of a context of length
-ctx - Lq + i1, for which the paged kernel's rule and RoPE positions give
-the same keys and positions.
+The Lq new tokens of a sequence of context length ctx sit at positions
+ctx - Lq .. ctx - 1 (the reference appends before it attends,
+block.py:57-65), and row i sees keys <= ctx - Lq + i.
 
 The Q/K/V projections and the output projection around it are unchanged.
 """
@@ -41,7 +38,7 @@ import math
 
 import torch
 
-from engine.attention import flash_attention, paged_attention, paged_max_rows
+from engine.attention import flash_attention, paged_attention, paged_max_rows, paged_prefill
 from engine.cache import PagedKVCache, StepBatch
 
 
@@ -120,9 +117,8 @@ def attention_section_rows(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, la
     layout of ``step.cu_new``), at positions ``starts[b] + i``, un-rotated
     when ``rope`` is given. ``step`` is ``cache.prepare_step(tables,
     counts)``. Returns (T, Hq * D), row for row. One append for every
-    sequence, then paged attention per group of sequences with equal
-    counts, in launches of at most ``paged_max_rows(D)`` query rows per kv
-    head."""
+    sequence, then one attention launch per group of sequences with equal
+    counts."""
     T, Hq, D = q.shape
     Hk = k.shape[1]
     if T != step.total_new or k.shape[0] != T or v.shape[0] != T or k.shape[1:] != (Hk, D) \
@@ -138,12 +134,15 @@ def attention_section_rows(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, la
 def _paged_rows(q_rows: torch.Tensor, layer_idx: int, cache: PagedKVCache, step: StepBatch,
                 rope: tuple[torch.Tensor, torch.Tensor] | None, out_rows: torch.Tensor) -> None:
     """Paged attention of the packed new-token rows of ``step`` (already
-    appended) over each sequence's history, into ``out_rows`` (T, Hq, D).
-    Sequences are grouped by their count of new tokens; a group's tokens go
-    in chunks of at most ``paged_max_rows(D) // (Hq / Hk)`` per launch, chunk
-    [i0, i1) as the newest tokens of a context of length ctx - count + i1.
-    The device index tensors of each launch are built on the first call of
-    the step and reused by every layer."""
+    appended) over each sequence's history, into ``out_rows`` (T, Hq, D): one
+    launch per count of new tokens, ``paged_attention`` up to
+    ``paged_max_rows(D)`` query rows per kv head and ``paged_prefill`` above
+    (1000 new tokens on 4600, 32/8 heads, D=128 bf16: 90 us, against 1000 in
+    paged_attention launches of that many rows each, which reread the history
+    once per 64 tokens). A group whose rows are consecutive is read and
+    written in place, others through an index (two more launches). The
+    device index tensors of each launch are built on the first call of the
+    step and reused by every layer."""
     T, Hq, D = q_rows.shape
     Hk = cache.cfg.num_kv_heads
     scale = 1.0 / math.sqrt(D)
@@ -159,15 +158,29 @@ def _paged_rows(q_rows: torch.Tensor, layer_idx: int, cache: PagedKVCache, step:
         q_rows = rope_apply(q_rows.transpose(0, 1).unsqueeze(0), rope[0], rope[1],
                             positions=step.cache[key])[0].transpose(0, 1)
         rope = None
-    chunk = max(1, paged_max_rows(D) // (Hq // Hk))
-    key = ("launches", chunk)
+    key = ("launches",)
     if key not in step.cache:
-        step.cache[key] = _launches(step, chunk, dev)
-    for tables, rows, lens, Lsub in step.cache[key]:
-        qs = q_rows[rows].view(-1, Lsub, Hq, D).transpose(1, 2)
-        o = paged_attention(qs, cache.k[layer_idx], cache.v[layer_idx], tables, lens,
-                            causal=True, scale=scale, max_context=step.max_context, rope=rope)
-        out_rows[rows] = o.transpose(1, 2).reshape(-1, Hq, D)
+        step.cache[key] = [(*launch, *_group_span(step, launch[3]))
+                           for launch in _launches(step, max(1, step.max_new), dev)]
+    for tables, rows, lens, L, r0, max_context in step.cache[key]:
+        n = lens.shape[0]
+        # (a group of more query heads per kv head than paged_attention takes is refused there)
+        attend = paged_prefill if Hq // Hk <= paged_max_rows(D) < Hq // Hk * L else paged_attention
+        qs = (q_rows[rows] if r0 is None else q_rows[r0:r0 + n * L]).view(n, L, Hq, D).transpose(1, 2)
+        out = None if r0 is None else out_rows[r0:r0 + n * L].view(n, L, Hq, D).transpose(1, 2)
+        o = attend(qs, cache.k[layer_idx], cache.v[layer_idx], tables, lens, causal=True, scale=scale,
+                   max_context=max_context, rope=rope, out=out)
+        if r0 is None:
+            out_rows[rows] = o.transpose(1, 2).reshape(-1, Hq, D)
+
+
+def _group_span(step: StepBatch, count: int) -> tuple[int | None, int]:
+    """First packed row of the sequences with ``count`` new tokens when their
+    rows are consecutive (else None), and their longest context."""
+    seqs = [b for b, c in enumerate(step.new_counts) if c == count]
+    between = step.new_counts[seqs[0]:seqs[-1] + 1]
+    contiguous = all(c in (count, 0) for c in between)
+    return (sum(step.new_counts[:seqs[0]]) if contiguous else None), max(step.lengths_host[b] for b in seqs)
 
 
 def _launches(step: StepBatch, chunk: int, dev: torch.device) -> list:

@@ -311,6 +311,47 @@ int cie_flash_fwd_rope(const void* q, const void* k, const void* v, void* o,
                        const int32_t* q_pos0, void* stream);
 
 /*
+ * cie_flash_fwd / cie_flash_fwd_rope (rope_cos NULL: no rotation) with the keys
+ * of every query tile cut into `splits` contiguous runs that different
+ * workgroups take, their partial states left in `workspace` and combined by a
+ * second launch: what a launch of few query tiles over many keys needs to fill
+ * the GPU. splits 0 lets the library choose (1, no splits, whenever the query
+ * tiles fill it); at most 32. `workspace`: 16-byte aligned device memory of at
+ * least cie_flash_workspace_bytes bytes for the same arguments (0 bytes, NULL
+ * allowed, without splits), used until the launches end.
+ */
+size_t cie_flash_workspace_bytes(int B, int Hq, int Hk, int Lq, int Lk, int D, int causal, int splits);
+int cie_flash_fwd_ex(const void* q, const void* k, const void* v, void* o,
+                     const int64_t* q_stride, const int64_t* k_stride,
+                     const int64_t* v_stride, const int64_t* o_stride,
+                     int B, int Hq, int Hk, int Lq, int Lk, int D,
+                     float scale, int causal, int dtype,
+                     const void* rope_cos, const void* rope_sin, int rope_rows, int rope_dtype,
+                     const int32_t* q_pos0, int splits, void* workspace, size_t workspace_bytes, void* stream);
+
+/*
+ * The prefill kernels over a paged history: attention of the newest Lq tokens
+ * of each sequence, any Lq, K and V read in place from the pool (a prefill
+ * chunk on top of a history; the reference gathers the history and runs
+ * flash_attention over it, engine/model/block.py:65-71). Arguments and results
+ * as in cie_paged_fwd (query rows of a kv head are not bounded here): a context
+ * length outside [0, min(max_context, max_blocks_per_seq * block_size)] or a
+ * block id outside [0, num_blocks) is never dereferenced and gives NaN rows.
+ * RoPE (rope_cos not NULL), splits and workspace as in cie_flash_fwd_ex.
+ */
+size_t cie_flash_paged_workspace_bytes(int B, int Hq, int Hk, int Lq, int D, int max_context, int block_size,
+                                       int max_blocks_per_seq, int splits);
+int cie_flash_paged(const void* q, const void* k_cache, const void* v_cache, const int32_t* block_tables,
+                    const int32_t* context_lens, void* o,
+                    const int64_t* q_stride, const int64_t* kc_stride,
+                    const int64_t* vc_stride, const int64_t* o_stride,
+                    int B, int Hq, int Hk, int Lq, int D,
+                    int num_blocks, int block_size, int max_blocks_per_seq,
+                    int max_context, float scale, int causal, int dtype,
+                    const void* rope_cos, const void* rope_sin, int rope_rows, int rope_dtype,
+                    int splits, void* workspace, size_t workspace_bytes, void* stream);
+
+/*
  * cie_paged_fwd with RoPE fused into the query load: query row i of sequence
  * b is rotated at position context_lens[b] - Lq + i, the position of that
  * token in the sequence (the same alignment the causal mask uses; the
