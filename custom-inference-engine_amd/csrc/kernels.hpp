@@ -115,8 +115,8 @@ struct PagedParams {
   RopeTables rope;  // rotate q row i of sequence b at position lens[b] - Lq + i as it is loaded
   // Fused append (kn != nullptr): the Lq newest tokens of sequence b are rows
   // b * Lq + i of kn / vn ((B * Lq, Hk, D), strides kns0 / vns0 per token,
-  // kns1 / vns1 per head). Attention reads them from there, and the
-  // workgroup whose range holds a new token writes it into the pool.
+  // kns1 / vns1 per head). The workgroup whose range holds a new token writes
+  // it into the pool before it requests that tile.
   const uint16_t* kn;
   const uint16_t* vn;
   int64_t kns0, kns1, vns0, vns1;

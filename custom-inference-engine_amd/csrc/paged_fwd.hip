@@ -375,12 +375,6 @@ __global__ __launch_bounds__(64 * paged_max_waves(D)) void paged_fwd_kernel(cons
   // (P % NCH) ^ row_swizzle(token) of the token's group row.
   int ltok[C::DPW];
   int32_t goffk[C::DPW], goffv[C::DPW];  // head + column offsets (the host bounds them below 2^31)
-  // Fused append: the chunk's (head, column) within a new-token row, kept as
-  // the chunk index only; the offsets are formed on the few tiles that hold
-  // new tokens (keeping them as 64-bit offsets pushed the kernel past the
-  // register file, and the spill reloads waited for every copy in flight).
-  constexpr int NA = APPEND ? C::DPW : 1;
-  int nch_of[NA];
 #pragma unroll
   for (int x = 0; x < C::DPW; ++x) {
     const int P = 64 * (hh * C::DPW + x) + lane;
@@ -389,7 +383,6 @@ __global__ __launch_bounds__(64 * paged_max_waves(D)) void paged_fwd_kernel(cons
     const int hd = c / C::S, dc = c % C::S;
     ltok[x] = tk;
     goffk[x] = (gh * p.Hg + hd) * (int32_t)p.ks2 + 8 * dc;
-    if constexpr (APPEND) nch_of[x] = c;
     goffv[x] = (gh * p.Hg + hd) * (int32_t)p.vs2 + 8 * dc;
   }
   // Fragment reads: K row l32 (chunk 2 kk + hl of head hh), V^T rows.
@@ -406,7 +399,6 @@ __global__ __launch_bounds__(64 * paged_max_waves(D)) void paged_fwd_kernel(cons
 
   // Issue cursor.
   int ie = 0, i_base = 0, i_end = __builtin_amdgcn_readfirstlane(ent[0][3]);
-  int i_b = __builtin_amdgcn_readfirstlane(ent[0][0]);
   int i_ctx = __builtin_amdgcn_readfirstlane(ent[0][1]), i_ttlo = __builtin_amdgcn_readfirstlane(ent[0][2]);
   int i_idb = __builtin_amdgcn_readfirstlane(ent[0][4]), i_blk = __builtin_amdgcn_readfirstlane(ent[0][5]);
   int i_stage = 0;
@@ -419,37 +411,10 @@ __global__ __launch_bounds__(64 * paged_max_waves(D)) void paged_fwd_kernel(cons
       i_ttlo = __builtin_amdgcn_readfirstlane(ent[ie][2]);
       i_idb = __builtin_amdgcn_readfirstlane(ent[ie][4]);
       i_blk = __builtin_amdgcn_readfirstlane(ent[ie][5]);
-      i_b = __builtin_amdgcn_readfirstlane(ent[ie][0]);
     }
     const int tbase = kPagedTile * (i_ttlo + k - i_base);
     const uint32_t st = ring_lds + 2u * (uint32_t)(i_stage * STAGE_EL) + 1024u * (uint32_t)(hh * C::DPW);
     i_stage = i_stage + 1 == NST ? 0 : i_stage + 1;
-    if (APPEND && tbase + kPagedTile > i_ctx - p.Lq) {
-      // a tile holding new tokens: those rows come from kn / vn, the rest
-      // from the pool (per-lane addresses)
-#pragma unroll
-      for (int x = 0; x < C::DPW; ++x) {
-        const int tk = min(tbase + ltok[x], i_ctx - 1);
-        const uint16_t *sk, *sv;
-        if (tk >= i_ctx - p.Lq) {
-          const int64_t row = (int64_t)i_b * p.Lq + (tk - (i_ctx - p.Lq));
-          int c = nch_of[APPEND ? x : 0];
-          asm volatile("" : "+v"(c));  // keeps the offset arithmetic on this path (not hoisted and kept live)
-          const int hd = gh * p.Hg + c / C::S, col = 8 * (c % C::S);
-          sk = p.kn + row * p.kns0 + (int64_t)hd * p.kns1 + col;
-          sv = p.vn + row * p.vns0 + (int64_t)hd * p.vns1 + col;
-        } else {
-          const int blk = (int)fdiv((uint32_t)tk, p.bsdiv);
-          const int off = tk - blk * p.block_size;
-          const int bid = max(sbt[i_idb + blk - i_blk], 0);
-          sk = p.kc + (int64_t)bid * p.ks0 + (int64_t)off * p.ks1 + goffk[x];
-          sv = p.vc + (int64_t)bid * p.vs0 + (int64_t)off * p.vs1 + goffv[x];
-        }
-        dma16_at_nt(sk, st + 1024u * x);
-        dma16_at_nt(sv, st + 2u * TILE_EL + 1024u * x);
-      }
-      return;
-    }
     int bid[C::DPW], off[C::DPW];
 #pragma unroll
     for (int x = 0; x < C::DPW; ++x) {  // all block-id reads in flight together
@@ -477,8 +442,8 @@ __global__ __launch_bounds__(64 * paged_max_waves(D)) void paged_fwd_kernel(cons
     }
   };
 
-  // q rows of the first QPRE sequences, then the first tiles; the wait below
-  // covers the q loads only (the tile copies issued after them stay in flight)
+  // q rows of the first QPRE sequences, then the first tiles; the wait after
+  // them covers the q loads only (the tile copies issued after them stay in flight)
   const uint16_t* qrow = p.q + hq * p.qs1 + (int64_t)i * p.qs2;
   u32x4 qpre[C::QARR][C::KK];
 #pragma unroll
@@ -487,18 +452,85 @@ __global__ __launch_bounds__(64 * paged_max_waves(D)) void paged_fwd_kernel(cons
 #pragma unroll
     for (int kk = 0; kk < C::KK; ++kk) qpre[e][kk] = load16(qrow + b * p.qs0 + 16 * kk + 8 * hl, rv && e < ne);
   }
+  if (p.rope.cos) {
+    // RoPE fused into the load: row i at position ctx - Lq + i. The table rows
+    // are requested beside q, ahead of the tile copies (loads return in
+    // order: behind them, they waited for the first tile). Slots past the
+    // range's sequences repeat the first one and are never used.
+    RopeRow<D> rr[C::QARR];
+#pragma unroll
+    for (int e = 0; e < C::QPRE; ++e) rr[e] = rope_row_load<D>(p.rope, ent[e < ne ? e : 0][1] - p.Lq + i, hl);
+#pragma unroll
+    for (int e = 0; e < C::QPRE; ++e) rope_row_apply<DTYPE, D>(qpre[e], p.rope, rr[e], rv, hl);
+  }
+
+  // Fused append: the new tokens inside this range go into the pool, the
+  // head group's rows of each (16-byte chunks over the whole workgroup), K
+  // rotated, before any tile is requested: the tile copies below then read
+  // them from the pool like every other row. A range holds whole tiles, so no
+  // other workgroup reads or writes these rows. (Reading the new rows from kn
+  // / vn in the tile copies, rotating K in LDS and writing the pool after the
+  // loop made the workgroups holding a sequence's end finish last, at 31-36 us
+  // of a decode step of 32 sequences where the median workgroup ended at 26;
+  // and the rotary table loads of that path counted as pending at the first
+  // MFMA of every tile, whose wait drained the copies in flight. Launch pair,
+  // pools out of cache, before / after: 8 x 5 rows over 1024-8192 at D=128
+  // bf16 79 / 54 us, at D=64 42 / 33; decode of 32 x 256-4096 at D=128 70 /
+  // 64, at D=64 38 / 37; of 64 x 500-1500 at D=128 68 / 61.)
+  if (APPEND) {
+    const int cpr = p.Hg * (D / 8);  // chunks of one tensor per token row of the head group
+    const bool rot = p.rope.cos != nullptr;
+    bool wrote = false;  // workgroup-uniform
+    for (int e = 0; e < ne; ++e) {
+      const int ctx = ent[e][1], tt_lo = ent[e][2], n = ent[e][3], idb = ent[e][4], blk_lo = ent[e][5];
+      const int lo = max(ctx - p.Lq, kPagedTile * tt_lo), hi = min(ctx, kPagedTile * (tt_lo + n));
+      const int b = ent[e][0];
+      wrote |= hi > lo;
+      for (int u = threadIdx.x; u < (hi > lo ? hi - lo : 0) * cpr * 2; u += blockDim.x) {
+        const int tsr = u / (2 * cpr), rem = u - tsr * 2 * cpr;
+        const int tensor = rem / cpr, c = rem - tensor * cpr;
+        const int pos = lo + tsr;
+        const int blk = (int)fdiv((uint32_t)pos, p.bsdiv);
+        const int bid = sbt[idb + blk - blk_lo];
+        if (bid < 0) continue;  // invalid block id: the output is NaN, nothing is written
+        // a position outside the rotary tables: NaN output rows, neither K nor
+        // V written (as the rotating append leaves the pool)
+        if (rot && pos >= p.rope.rows) continue;
+        const int off = pos - blk * p.block_size;
+        const int h = gh * p.Hg + c / (D / 8), d = 8 * (c % (D / 8));
+        const int64_t row = (int64_t)b * p.Lq + (pos - (ctx - p.Lq));
+        if (tensor == 0 && rot) {
+          // K rotated at its position: the thread of the pair's first chunk writes both
+          if (d >= D / 2) continue;
+          const uint16_t* src = p.kn + row * p.kns0 + (int64_t)h * p.kns1 + d;
+          u32x4 a = *reinterpret_cast<const u32x4*>(src), bb = *reinterpret_cast<const u32x4*>(src + D / 2);
+          rope_apply8<DTYPE>(a, bb, rope_load(p.rope, (int64_t)pos * (D / 2) + d), p.rope.dt);
+          uint16_t* dst = const_cast<uint16_t*>(p.kc) + (int64_t)bid * p.ks0 + (int64_t)off * p.ks1 +
+                          (int64_t)h * p.ks2 + d;
+          *reinterpret_cast<u32x4*>(dst) = a;
+          *reinterpret_cast<u32x4*>(dst + D / 2) = bb;
+        } else if (tensor == 0)
+          *reinterpret_cast<u32x4*>(const_cast<uint16_t*>(p.kc) + (int64_t)bid * p.ks0 + (int64_t)off * p.ks1 +
+                                    (int64_t)h * p.ks2 + d) =
+              *reinterpret_cast<const u32x4*>(p.kn + row * p.kns0 + (int64_t)h * p.kns1 + d);
+        else
+          *reinterpret_cast<u32x4*>(const_cast<uint16_t*>(p.vc) + (int64_t)bid * p.vs0 + (int64_t)off * p.vs1 +
+                                    (int64_t)h * p.vs2 + d) =
+              *reinterpret_cast<const u32x4*>(p.vn + row * p.vns0 + (int64_t)h * p.vns1 + d);
+      }
+    }
+    if (wrote) {
+      vm_wait<0>();     // this wave's rows are in the cache the tile copies read
+      __syncthreads();  // and every other wave's
+    }
+  }
+
   const int pro = min(NST - 1, T);
   if (issuer) {
     for (int k = 0; k < pro; ++k) issue(k);
     wait_tiles_ahead<C::DPW>(pro);
   } else {
     vm_wait<0>();
-  }
-  if (p.rope.cos) {  // RoPE fused into the load: row i at position ctx - Lq + i
-#pragma unroll
-    for (int e = 0; e < C::QPRE; ++e)
-      if (e < ne)  // wave-uniform: preload slots past the range's sequences hold zeros and are never used
-        rope_q_lane<DTYPE, D>(qpre[e], p.rope, ent[e][1] - p.Lq + i, rv, hl);
   }
 #pragma unroll
   for (int e = 0; e < C::QPRE; ++e)
@@ -531,6 +563,10 @@ __global__ __launch_bounds__(64 * paged_max_waves(D)) void paged_fwd_kernel(cons
         bool bad = false;
         for (int x = lane; x < blk_hi - blk_lo + 1; x += 64) bad |= sbt[idb + x] < 0;
         poison = __builtin_amdgcn_ballot_w64(bad) != 0;
+        // a new token outside the rotary tables was not written: its query row
+        // is NaN, and so is, without the causal mask, every row that sees it
+        if (APPEND && p.rope.cos && !p.causal)
+          poison |= min(c_ctx, kPagedTile * (c_ttlo + ent[ce][3])) > max(p.rope.rows, c_ctx - p.Lq);
       }
       if (decltype(FIRST)::value && C::QPRE > 0) {
 #pragma unroll
@@ -574,31 +610,6 @@ __global__ __launch_bounds__(64 * paged_max_waves(D)) void paged_fwd_kernel(cons
     const uint16_t* vst = kst + TILE_EL;
     c_stage = c_stage + 1 == NST ? 0 : c_stage + 1;
     const int t0 = kPagedTile * (c_ttlo + n - c_base);
-    if (APPEND && p.rope.cos && t0 + kPagedTile > c_ctx - p.Lq) {
-      // fused append with RoPE: the new K rows of this tile arrived
-      // unrotated from kn; rotate them in LDS at their positions (pairs of
-      // 16-byte chunks j, j + D/16 of each head, found through the row
-      // swizzle), then publish the rotated tile
-      const int first = max(c_ctx - p.Lq, t0), last = min(c_ctx, t0 + kPagedTile);
-      const int items = (last - first) * p.Hg * (D / 16);
-      for (int u = threadIdx.x; u < items; u += blockDim.x) {
-        const int tr = u / (p.Hg * (D / 16)), rem = u - tr * p.Hg * (D / 16);
-        const int hd = rem / (D / 16), jj = rem - hd * (D / 16);
-        const int pos = first + tr, t = pos - t0;
-        const int sw = row_swizzle(NCH, t);
-        uint16_t* rowp = const_cast<uint16_t*>(kst) + (t << lg_nch) * 8;
-        u32x4* lo = reinterpret_cast<u32x4*>(rowp + ((hd * C::S + jj) ^ sw) * 8);
-        u32x4* hi = reinterpret_cast<u32x4*>(rowp + ((hd * C::S + jj + C::S / 2) ^ sw) * 8);
-        u32x4 a = *lo, b = *hi;
-        const bool ok = pos < p.rope.rows;
-        const int64_t tr0 = (ok ? (int64_t)pos : 0) * (D / 2) + 8 * jj;
-        rope_apply8<DTYPE>(a, b, rope_load(p.rope, tr0), p.rope.dt);
-        if (!ok) a = b = u32x4{0x7fff7fffu, 0x7fff7fffu, 0x7fff7fffu, 0x7fff7fffu};
-        *lo = a;
-        *hi = b;
-      }
-      __syncthreads();
-    }
 
     f32x16 sc = f32x16{};
 #pragma unroll
@@ -684,52 +695,6 @@ __global__ __launch_bounds__(64 * paged_max_waves(D)) void paged_fwd_kernel(cons
   }
 
   CIE_STAMP(paged_timeline, 3);  // tile loop done
-
-  // Fused append: the new tokens inside this range go into the pool, the
-  // head group's rows of each (16-byte chunks over the whole workgroup).
-  // Nothing in this launch reads those pool rows (the tiles holding them
-  // took the rows from kn / vn), so no ordering is needed.
-  if (APPEND) {
-    const int cpr = p.Hg * (D / 8);  // chunks of one tensor per token row of the head group
-    const bool rot = p.rope.cos != nullptr;
-    for (int e = 0; e < ne; ++e) {
-      const int ctx = ent[e][1], tt_lo = ent[e][2], n = ent[e][3], idb = ent[e][4], blk_lo = ent[e][5];
-      const int lo = max(ctx - p.Lq, kPagedTile * tt_lo), hi = min(ctx, kPagedTile * (tt_lo + n));
-      const int b = ent[e][0];
-      for (int u = threadIdx.x; u < (hi > lo ? hi - lo : 0) * cpr * 2; u += blockDim.x) {
-        const int tsr = u / (2 * cpr), rem = u - tsr * 2 * cpr;
-        const int tensor = rem / cpr, c = rem - tensor * cpr;
-        const int pos = lo + tsr;
-        const int blk = (int)fdiv((uint32_t)pos, p.bsdiv);
-        const int bid = sbt[idb + blk - blk_lo];
-        if (bid < 0) continue;  // invalid block id: the output is NaN, nothing is written
-        // a position outside the rotary tables: NaN output rows, neither K nor
-        // V written (as the rotating append leaves the pool)
-        if (rot && pos >= p.rope.rows) continue;
-        const int off = pos - blk * p.block_size;
-        const int h = gh * p.Hg + c / (D / 8), d = 8 * (c % (D / 8));
-        const int64_t row = (int64_t)b * p.Lq + (pos - (ctx - p.Lq));
-        if (tensor == 0 && rot) {
-          // K rotated at its position: the thread of the pair's first chunk writes both
-          if (d >= D / 2) continue;
-          const uint16_t* src = p.kn + row * p.kns0 + (int64_t)h * p.kns1 + d;
-          u32x4 a = *reinterpret_cast<const u32x4*>(src), bb = *reinterpret_cast<const u32x4*>(src + D / 2);
-          rope_apply8<DTYPE>(a, bb, rope_load(p.rope, (int64_t)pos * (D / 2) + d), p.rope.dt);
-          uint16_t* dst = const_cast<uint16_t*>(p.kc) + (int64_t)bid * p.ks0 + (int64_t)off * p.ks1 +
-                          (int64_t)h * p.ks2 + d;
-          *reinterpret_cast<u32x4*>(dst) = a;
-          *reinterpret_cast<u32x4*>(dst + D / 2) = bb;
-        } else if (tensor == 0)
-          *reinterpret_cast<u32x4*>(const_cast<uint16_t*>(p.kc) + (int64_t)bid * p.ks0 + (int64_t)off * p.ks1 +
-                                    (int64_t)h * p.ks2 + d) =
-              *reinterpret_cast<const u32x4*>(p.kn + row * p.kns0 + (int64_t)h * p.kns1 + d);
-        else
-          *reinterpret_cast<u32x4*>(const_cast<uint16_t*>(p.vc) + (int64_t)bid * p.vs0 + (int64_t)off * p.vs1 +
-                                    (int64_t)h * p.vs2 + d) =
-              *reinterpret_cast<const u32x4*>(p.vn + row * p.vns0 + (int64_t)h * p.vns1 + d);
-      }
-    }
-  }
 
   CIE_STAMP(paged_timeline, 4);  // end
 }

@@ -113,35 +113,60 @@ __device__ __forceinline__ void rope_apply8(u32x4& lo, u32x4& hi, const RopeChun
   else rope8<DTYPE>(lo, hi, widen8<1 - DTYPE>(r.c0), widen8<1 - DTYPE>(r.s0));
 }
 
+// The table entries a lane needs to rotate its part of a query row in the
+// MFMA B-operand layout (rope_row_apply), loaded apart from the rotation. An
+// out-of-range position reads row 0.
+template <int D>
+struct RopeRow {
+  RopeChunk c[D / 16 > 1 ? D / 32 : 1];
+  bool ok;
+};
+template <int D>
+__device__ __forceinline__ RopeRow<D> rope_row_load(const RopeTables& t, int pos, int hl) {
+  constexpr int KK = D / 16;
+  RopeRow<D> r;
+  r.ok = pos >= 0 && pos < t.rows;
+  const int64_t row = r.ok ? (int64_t)pos * (D / 2) : 0;
+  if constexpr (KK == 1) {
+    r.c[0] = rope_load(t, row);
+  } else {
+#pragma unroll
+    for (int kk = 0; kk < KK / 2; ++kk) r.c[kk] = rope_load(t, row + 16 * kk + 8 * hl);
+  }
+  return r;
+}
+
 // Rotates the query row a lane holds in the MFMA B-operand layout
-// (q[16 kk + 8 hl .. +8] in register kk, hl = lane / 32) at position pos.
+// (q[16 kk + 8 hl .. +8] in register kk, hl = lane / 32).
 // For D >= 32 the partner of register kk < D/32 is register kk + D/32 of the
 // same lane; for D = 16 it is the same register of lane ^ 32 (every lane of
 // the wave must call this then). An out-of-range position makes the row NaN
-// when the lane's row is live; the table reads stay in row 0 then.
+// when the lane's row is live.
 template <int DTYPE, int D>
-__device__ __forceinline__ void rope_q_lane(u32x4 (&qf)[D / 16], const RopeTables& t, int pos, bool live, int hl) {
+__device__ __forceinline__ void rope_row_apply(u32x4 (&qf)[D / 16], const RopeTables& t, const RopeRow<D>& r,
+                                               bool live, int hl) {
   constexpr int KK = D / 16;
-  const bool ok = pos >= 0 && pos < t.rows;
-  const int64_t row = ok ? (int64_t)pos * (D / 2) : 0;
   if constexpr (KK == 1) {
     u32x4 other;
 #pragma unroll
     for (int e = 0; e < 4; ++e) other[e] = (uint32_t)__shfl_xor((int)qf[0][e], 32);
     u32x4 lo = hl ? other : qf[0], hi = hl ? qf[0] : other;
-    rope_apply8<DTYPE>(lo, hi, rope_load(t, row), t.dt);
+    rope_apply8<DTYPE>(lo, hi, r.c[0], t.dt);
     qf[0] = hl ? hi : lo;
   } else {
-    RopeChunk r[KK / 2];
 #pragma unroll
-    for (int kk = 0; kk < KK / 2; ++kk) r[kk] = rope_load(t, row + 16 * kk + 8 * hl);
-#pragma unroll
-    for (int kk = 0; kk < KK / 2; ++kk) rope_apply8<DTYPE>(qf[kk], qf[kk + KK / 2], r[kk], t.dt);
+    for (int kk = 0; kk < KK / 2; ++kk) rope_apply8<DTYPE>(qf[kk], qf[kk + KK / 2], r.c[kk], t.dt);
   }
-  if (live && !ok) {
+  if (live && !r.ok) {
 #pragma unroll
     for (int kk = 0; kk < KK; ++kk) qf[kk] = u32x4{0x7fff7fffu, 0x7fff7fffu, 0x7fff7fffu, 0x7fff7fffu};
   }
+}
+
+// Both at once, for position pos.
+template <int DTYPE, int D>
+__device__ __forceinline__ void rope_q_lane(u32x4 (&qf)[D / 16], const RopeTables& t, int pos, bool live, int hl) {
+  rope_row_apply<DTYPE, D>(qf, t, rope_row_load<D>(t, pos, hl), live, hl);
 }
 
 }  // namespace cie

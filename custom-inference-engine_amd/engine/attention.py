@@ -412,8 +412,8 @@ def paged_attention(
 
     ``new_kv``: (k_new, v_new), each (B * Lq, Hk, D) with row b * Lq + i =
     new token i of sequence b, not yet in the pool. The append happens in the
-    same launch pair (``cie_paged_fwd_append``): attention reads those rows
-    directly and writes them into the pool at positions
+    same launch pair (``cie_paged_fwd_append``): the workgroup that attends
+    over those rows writes them into the pool first, at positions
     ``context_lens[b] - Lq + i``, so the pool and the result equal
     ``kv_append`` followed by ``paged_attention`` bit for bit. Every context
     must count its Lq new tokens (a shorter one gives NaN rows). With

@@ -185,3 +185,29 @@ def test_fused_append_rejects_bad_shapes():
     with pytest.raises(ValueError):
         paged_attention(q.to(DEV), kp.to(DEV), vp.to(DEV), bt.to(DEV), lt.to(DEV),
                         new_kv=(k_new.to(DEV), v_new.to(DEV).float()))
+
+
+@pytest.mark.parametrize("D,dtype", [(16, torch.float16), (64, torch.float16), (128, torch.bfloat16),
+                                     (256, torch.float16)])
+@pytest.mark.parametrize("rope", [False, True])
+def test_fused_append_rows_are_written_before_they_are_read(D, dtype, rope):
+    """40 new tokens over histories ending at every position of the two tiles
+    around a tile edge, the pool slots of the new tokens holding NaN: a tile
+    requested before its rows are written shows in the output."""
+    from engine.model.rope import build_rope_cache
+
+    Lq, bs, Hk = 40, 16, 2
+    lens = [Lq + h for h in (0, 1, 8, 23, 24, 25, 31, 32, 33, 56, 63, 64, 65, 600)]
+    q, kp, vp, bt, lt = make_paged(lens, Lq, D, dtype, bs, Hq=4, Hk=Hk, seed=D, vscale=0.5)
+    for b, n in enumerate(lens):
+        for pos in range(n - Lq, n):
+            kp[bt[b, pos // bs], pos % bs] = vp[bt[b, pos // bs], pos % bs] = float("nan")
+    k_new, v_new = _new_rows(len(lens), Lq, Hk, D, dtype, seed=D + 1)
+    tabs = tuple(t.to(DEV) for t in build_rope_cache(1024, D)) if rope else None
+    kd, vd = kp.to(DEV), vp.to(DEV)
+    cu = torch.arange(0, len(lens) * Lq + 1, Lq, dtype=torch.int32, device=DEV)
+    kv_append(k_new.to(DEV), v_new.to(DEV), kd, vd, bt.to(DEV), cu, (lt - Lq).to(DEV), max_new=Lq, rope=tabs)
+    want = paged_attention(q.to(DEV), kd, vd, bt.to(DEV), lt.to(DEV), rope=tabs).cpu()
+    out, k1, v1 = _fused(q, kp, vp, bt, lt, k_new, v_new, rope=tabs)
+    assert torch.isfinite(want).all() and torch.equal(out, want)
+    assert torch.equal(k1, kd.cpu()) and torch.equal(v1, vd.cpu())
