@@ -5,7 +5,7 @@
 
 Every source is compiled for gfx950 with hipcc (objects under ``_build/``,
 compiled in parallel) and linked into ``custom-inference-engine_amd/libcie_attn.so``,
-which the Python layer loads with ctypes. Packed-FP32 VALU instructions are
+which the Python layer loads with ctypes and calls through ``cie_host.so``. Packed-FP32 VALU instructions are
 disabled for all device code.
 """
 
@@ -22,6 +22,7 @@ CSRC = os.path.join(PKG_DIR, "csrc")
 INCLUDE = os.path.join(REPO, "include")
 BUILD = os.path.join(PKG_DIR, "_build")
 LIB_PATH = os.path.join(PKG_DIR, "libcie_attn.so")
+HOST_PATH = os.path.join(PKG_DIR, "cie_host.so")  # CPython extension: the Python layer's calls into the library
 TIMELINE_LIB_PATH = os.path.join(PKG_DIR, "libcie_attn_timeline.so")
 # stand-alone microbenchmarks (benchmarks/<name>.hip -> _build/<name>), not part of the library
 BENCH_TOOLS = ("vector_rates", "read_floor", "prefill_step")
@@ -71,10 +72,31 @@ def _build_lib(out: str, objdir: str, defines: list[str]) -> None:
     os.replace(tmp, out)
 
 
+def _build_host() -> None:
+    """csrc/host.cpp against torch's C++ headers (host code only)."""
+    import sysconfig
+
+    import torch
+    from torch.utils.cpp_extension import include_paths, library_paths
+
+    inc = [f"-I{d}" for d in (INCLUDE, sysconfig.get_paths()["include"], "/opt/rocm/include")]
+    inc += [f"-isystem{d}" for d in include_paths()]
+    libs = [x for d in library_paths() for x in (f"-L{d}", f"-Wl,-rpath,{d}")]
+    tmp = HOST_PATH + ".tmp"
+    _run(["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+          f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", *inc, os.path.join(CSRC, "host.cpp"),
+          "-o", tmp, *libs, "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_python"])
+    os.replace(tmp, HOST_PATH)
+
+
 def build(verbose: bool = False) -> str:
-    """Compile every source and link the shared library; returns its path."""
+    """Compile every source and link the shared library and the extension that
+    calls it; returns the library's path."""
     os.makedirs(BUILD, exist_ok=True)
-    _build_lib(LIB_PATH, BUILD, [])
+    with ThreadPoolExecutor(max_workers=1) as ex:
+        host = ex.submit(_build_host)
+        _build_lib(LIB_PATH, BUILD, [])
+        host.result()
     # the microbenchmarks behind benchmarks/vector_rates.py, read_floor.py and prefill_step.py
     tools = [[HIPCC, *COMMON, "-x", "hip", os.path.join(PKG_DIR, "benchmarks", t + ".hip"), "-o", os.path.join(BUILD, t)]
              for t in BENCH_TOOLS]

@@ -1,0 +1,452 @@
+// The Python layer's calls into libcie_attn.so as a CPython extension
+// (cie_host.so, built next to it): tensor checks, output and workspace
+// allocation and the C ABI call of one operation without interpreter work in
+// between. A call through ctypes with its argument conversion, stride arrays
+// and device context took 17-24 us of host time per operation, more than most
+// of the kernels it launches; here it takes 4-7.
+//
+// Every function handles the arguments a kernel can take as they are (exact
+// tensors on one GPU, supported dtypes and shapes, rows the kernels can read in
+// place) and returns None for everything else, before any side effect: the
+// Python function then copies, converts or raises as the case needs. A
+// non-zero status of the library comes back as an int.
+//
+// The library's functions are bound by address (bind), so the extension works
+// with whichever build of the library the package loaded.
+#include <Python.h>
+
+#include <ATen/ATen.h>
+#include <c10/core/DeviceGuard.h>
+#include <c10/hip/HIPStream.h>
+#include <torch/csrc/autograd/python_variable.h>
+
+#include <cmath>
+
+#include "cie_attn.h"
+
+namespace {
+
+struct Api {
+  decltype(&cie_flash_workspace_bytes) flash_ws;
+  decltype(&cie_flash_fwd_ex) flash;
+  decltype(&cie_flash_paged_workspace_bytes) flash_paged_ws;
+  decltype(&cie_flash_paged) flash_paged;
+  decltype(&cie_paged_workspace_bytes) paged_ws;
+  decltype(&cie_paged_fwd_ex) paged;
+  decltype(&cie_kv_append) append;
+  decltype(&cie_kv_append_rope) append_rope;
+  decltype(&cie_int8_matmul_workspace_bytes) int8_ws;
+  decltype(&cie_int8_matmul) int8;
+} api;
+const char* const kNames[] = {"cie_flash_workspace_bytes", "cie_flash_fwd_ex", "cie_flash_paged_workspace_bytes",
+                              "cie_flash_paged", "cie_paged_workspace_bytes", "cie_paged_fwd_ex", "cie_kv_append",
+                              "cie_kv_append_rope", "cie_int8_matmul_workspace_bytes", "cie_int8_matmul"};
+constexpr size_t kFns = sizeof(kNames) / sizeof(kNames[0]);
+static_assert(sizeof(Api) == kFns * sizeof(void*), "one name per function, in order");
+
+using at::Tensor;
+
+// The tensor behind an object that is exactly a Tensor or Parameter (no
+// subclass: those may override what a call does), else nullptr.
+const Tensor* tensor(PyObject* o) { return THPVariable_CheckExact(o) ? &THPVariable_Unpack(o) : nullptr; }
+// The same, None allowed (*ok false when it is neither).
+const Tensor* tensor_or_none(PyObject* o, bool* ok) {
+  if (o == Py_None) return nullptr;
+  const Tensor* t = tensor(o);
+  *ok &= t != nullptr;
+  return t;
+}
+
+int dtype_code(const Tensor& t) {
+  return t.scalar_type() == at::kHalf ? CIE_DTYPE_F16 : t.scalar_type() == at::kBFloat16 ? CIE_DTYPE_BF16 : -1;
+}
+int any_code(const Tensor& t) { return t.scalar_type() == at::kFloat ? CIE_TABLE_F32 : dtype_code(t); }
+
+bool strided(const Tensor& t) { return t.layout() == at::kStrided && !t.is_conj() && !t.is_neg(); }
+bool on_gpu(const Tensor& t) { return t.is_cuda() && strided(t); }
+
+bool head_dim_ok(int64_t D) { return D == 16 || D == 32 || D == 64 || D == 128 || D == 256; }
+bool fits(int64_t x) { return x >= 0 && x <= 0x7fffffff; }
+
+// What the kernels read in place: unit last stride, 16-byte aligned rows.
+bool kernel_layout(const Tensor& t) {
+  const int64_t n = t.dim();
+  if (t.stride(n - 1) != 1 || (reinterpret_cast<uintptr_t>(t.data_ptr()) & 15)) return false;
+  for (int64_t i = 0; i < n - 1; ++i)
+    if (t.size(i) != 1 && (t.stride(i) % 8 || t.stride(i) < 0)) return false;
+  return true;
+}
+
+struct Strides {
+  int64_t s[4];
+  explicit Strides(const Tensor& t) {  // a size-1 dimension's stride is never multiplied: 0
+    const int64_t n = t.dim();
+    for (int64_t i = 0; i < n; ++i) s[i] = i < n - 1 && t.size(i) == 1 ? 0 : t.stride(i);
+  }
+};
+
+struct Rope {
+  const void *cos = nullptr, *sin = nullptr;
+  int rows = 0, dt = 0;
+  bool ok = true;
+  Rope(PyObject* c, PyObject* s, int64_t D, const Tensor& like) {
+    const Tensor* ct = tensor_or_none(c, &ok);
+    const Tensor* st = tensor_or_none(s, &ok);
+    ok = ok && (ct == nullptr) == (st == nullptr);
+    if (!ok || !ct) return;
+    for (const Tensor* t : {ct, st})
+      ok = ok && on_gpu(*t) && t->device() == like.device() && t->dim() == 2 && t->size(1) == D / 2 &&
+           t->is_contiguous() && any_code(*t) >= 0 && !(reinterpret_cast<uintptr_t>(t->data_ptr()) & 15);
+    ok = ok && ct->sizes() == st->sizes() && ct->size(0) >= 1 && fits(ct->size(0)) &&
+         ct->scalar_type() == st->scalar_type();
+    if (!ok) return;
+    cos = ct->data_ptr();
+    sin = st->data_ptr();
+    rows = (int)ct->size(0);
+    dt = any_code(*ct);
+  }
+};
+
+void* stream_of(const Tensor& t) { return c10::hip::getCurrentHIPStream(t.device().index()).stream(); }
+
+Tensor bytes_like(size_t n, const Tensor& t) { return at::empty({(int64_t)n}, t.options().dtype(at::kByte)); }
+
+// Runs f without the GIL (as ctypes does), on the tensor's device; f returns a status.
+template <typename F>
+int launch(const Tensor& t, F&& f) {
+  int rc;
+  Py_BEGIN_ALLOW_THREADS;
+  rc = f();
+  Py_END_ALLOW_THREADS;
+  return rc;
+}
+
+PyObject* result(int rc, const Tensor& out) { return rc ? PyLong_FromLong(rc) : THPVariable_Wrap(out); }
+
+#define CIE_PY_BEGIN try {
+#define CIE_PY_END                                    \
+  }                                                   \
+  catch (const std::exception& e) {                   \
+    PyErr_SetString(PyExc_RuntimeError, e.what());    \
+    return nullptr;                                   \
+  }
+
+bool number(PyObject* o, double* v) {
+  *v = PyFloat_AsDouble(o);
+  if (!PyErr_Occurred()) return true;
+  PyErr_Clear();
+  return false;
+}
+
+// flash(q, k, v, causal, scale | None, cos | None, sin | None, q_pos0 | None, out | None)
+PyObject* flash(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  CIE_PY_BEGIN
+  if (n != 9) Py_RETURN_NONE;
+  const Tensor *q = tensor(a[0]), *k = tensor(a[1]), *v = tensor(a[2]);
+  bool ok = q && k && v;
+  const Tensor* pos = tensor_or_none(a[7], &ok);
+  const Tensor* o = tensor_or_none(a[8], &ok);
+  if (!ok || !on_gpu(*q) || !on_gpu(*k) || !on_gpu(*v) || q->dim() != 4 || k->dim() != 4 || v->dim() != 4) Py_RETURN_NONE;
+  const int dt = dtype_code(*q);
+  const int64_t B = q->size(0), H = q->size(1), M = q->size(2), D = q->size(3), Hk = k->size(1), N = k->size(2);
+  if (dt < 0 || k->scalar_type() != q->scalar_type() || v->scalar_type() != q->scalar_type() ||
+      k->device() != q->device() || v->device() != q->device() || !head_dim_ok(D) || v->sizes() != k->sizes() ||
+      k->size(0) != B || k->size(3) != D || Hk < 1 || H % Hk || !fits(B) || !fits(H) || !fits(M) || !fits(N) ||
+      !kernel_layout(*q) || !kernel_layout(*k) || !kernel_layout(*v))
+    Py_RETURN_NONE;
+  if (o && (!on_gpu(*o) || o->sizes() != q->sizes() || o->scalar_type() != q->scalar_type() ||
+            o->device() != q->device() || !kernel_layout(*o)))
+    Py_RETURN_NONE;
+  const Rope rope(a[5], a[6], D, *q);
+  if (!rope.ok || (pos && (!rope.cos || !on_gpu(*pos) || pos->device() != q->device() ||
+                           pos->scalar_type() != at::kInt || pos->dim() != 1 || pos->size(0) != B ||
+                           !pos->is_contiguous())))
+    Py_RETURN_NONE;
+  double scale = 1.0 / std::sqrt((double)D);
+  if (a[4] != Py_None && !number(a[4], &scale)) Py_RETURN_NONE;
+  const int causal = PyObject_IsTrue(a[3]);
+  if (causal < 0) return nullptr;
+  const c10::OptionalDeviceGuard guard(q->device());
+  const Tensor out = o ? *o : at::empty({B, H, M, D}, q->options());
+  const size_t nbytes = api.flash_ws((int)B, (int)H, (int)Hk, (int)M, (int)N, (int)D, causal, 0);
+  const Tensor ws = nbytes ? bytes_like(nbytes, *q) : Tensor();
+  const Strides sq(*q), sk(*k), sv(*v), so(out);
+  void* stream = stream_of(*q);
+  const int rc = launch(*q, [&] {
+    return api.flash(q->data_ptr(), k->data_ptr(), v->data_ptr(), out.data_ptr(), sq.s, sk.s, sv.s, so.s, (int)B,
+                     (int)H, (int)Hk, (int)M, (int)N, (int)D, (float)scale, causal, dt, rope.cos, rope.sin, rope.rows,
+                     rope.dt, pos ? static_cast<const int32_t*>(pos->data_ptr()) : nullptr, 0,
+                     nbytes ? ws.data_ptr() : nullptr, nbytes, stream);
+  });
+  return result(rc, out);
+  CIE_PY_END
+}
+
+// A launch over one layer's pools; the tables are int32 and contiguous.
+struct Pools {
+  const Tensor *kc, *vc, *bt, *lens;
+  int64_t num_blocks = 0, block_size = 0, Hk = 0, width = 0;
+  bool ok;
+  Pools(PyObject* k, PyObject* v, PyObject* t, PyObject* l, const Tensor& like, int64_t B, int64_t D)
+      : kc(tensor(k)), vc(tensor(v)), bt(tensor(t)), lens(tensor(l)) {
+    ok = kc && vc && bt && lens;
+    if (!ok) return;
+    for (const Tensor* x : {kc, vc})
+      ok = ok && on_gpu(*x) && x->device() == like.device() && x->dim() == 4 && x->scalar_type() == like.scalar_type() &&
+           x->size(3) == D && kernel_layout(*x);
+    for (const Tensor* x : {bt, lens})
+      ok = ok && on_gpu(*x) && x->device() == like.device() && x->scalar_type() == at::kInt && x->is_contiguous();
+    ok = ok && kc->sizes() == vc->sizes() && bt->dim() == 2 && bt->size(0) == B && lens->dim() == 1 && lens->size(0) == B;
+    if (!ok) return;
+    num_blocks = kc->size(0), block_size = kc->size(1), Hk = kc->size(2), width = bt->size(1);
+    ok = Hk >= 1 && fits(num_blocks) && fits(block_size) && fits(Hk) && fits(width);
+  }
+};
+
+// The plan of a launch (PagedPlan.data, .split, .key): none, or one built for
+// exactly this launch.
+struct Plan {
+  const Tensor* data = nullptr;
+  int split = -1;
+  bool ok = true;
+  Plan(PyObject* d, PyObject* s, PyObject* key, std::initializer_list<int64_t> want, const Tensor& like) {
+    data = tensor_or_none(d, &ok);
+    if (!ok || !data) return;
+    ok = PyLong_Check(s) && PyTuple_Check(key) && PyTuple_GET_SIZE(key) == (Py_ssize_t)want.size() && on_gpu(*data) &&
+         data->device() == like.device() && data->is_contiguous();
+    if (!ok) return;
+    split = (int)PyLong_AsLong(s);
+    Py_ssize_t i = 0;
+    for (int64_t w : want) {
+      const int64_t x = PyLong_AsLongLong(PyTuple_GET_ITEM(key, i++));
+      ok = ok && x == w;
+    }
+    if (PyErr_Occurred()) {
+      PyErr_Clear();
+      ok = false;
+    }
+  }
+};
+
+// Launches paged attention (kn: with the new rows appended) or, prefill, the
+// prefill kernels over the pools.
+int paged_launch(const Tensor& q, const Pools& P, const Tensor& out, const Rope& rope, const Plan& plan, int64_t mc,
+                 double scale, int causal, const void* kn, const void* vn, const int64_t* kns, const int64_t* vns,
+                 bool prefill) {
+  const int B = (int)q.size(0), Hq = (int)q.size(1), Lq = (int)q.size(2), D = (int)q.size(3), dt = dtype_code(q);
+  const int nb = (int)P.num_blocks, bs = (int)P.block_size, Hk = (int)P.Hk, w = (int)P.width, m = (int)mc;
+  size_t nbytes = 0;
+  if (prefill) nbytes = api.flash_paged_ws(B, Hq, Hk, Lq, D, m, bs, w, 0);
+  else if (!plan.data || plan.split) nbytes = api.paged_ws(B, Hq, Hk, Lq, D, m, bs, w);
+  const Tensor ws = nbytes ? bytes_like(nbytes, q) : Tensor();
+  const Strides sq(q), sk(*P.kc), sv(*P.vc), so(out);
+  void* const wp = nbytes ? ws.data_ptr() : nullptr;
+  void* stream = stream_of(q);
+  const int32_t *bt = static_cast<const int32_t*>(P.bt->data_ptr()), *lens = static_cast<const int32_t*>(P.lens->data_ptr());
+  return launch(q, [&] {
+    if (prefill)
+      return api.flash_paged(q.data_ptr(), P.kc->data_ptr(), P.vc->data_ptr(), bt, lens, out.data_ptr(), sq.s, sk.s,
+                             sv.s, so.s, B, Hq, Hk, Lq, D, nb, bs, w, m, (float)scale, causal, dt, rope.cos, rope.sin,
+                             rope.rows, rope.dt, 0, wp, nbytes, stream);
+    return api.paged(q.data_ptr(), kn, vn, P.kc->data_ptr(), P.vc->data_ptr(), plan.data ? nullptr : bt,
+                     plan.data ? nullptr : lens, plan.data ? plan.data->data_ptr() : nullptr,
+                     plan.data ? (size_t)plan.data->nbytes() : 0, plan.split, out.data_ptr(), wp, nbytes, sq.s, kns, vns,
+                     sk.s, sv.s, so.s, B, Hq, Hk, Lq, D, nb, bs, w, m, (float)scale, causal, dt, rope.cos, rope.sin,
+                     rope.rows, rope.dt, stream);
+  });
+}
+
+// paged(prefill, q, k_cache, v_cache, block_tables, context_lens, causal, scale | None, max_context, cos, sin, out | None)
+PyObject* paged(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  CIE_PY_BEGIN
+  if (n != 12) Py_RETURN_NONE;
+  const bool prefill = a[0] == Py_True;
+  const Tensor* q = tensor(a[1]);
+  bool ok = q != nullptr;
+  const Tensor* o = tensor_or_none(a[11], &ok);
+  if (!ok || !on_gpu(*q) || q->dim() != 4 || dtype_code(*q) < 0 || !head_dim_ok(q->size(3)) || !kernel_layout(*q))
+    Py_RETURN_NONE;
+  const int64_t B = q->size(0), Hq = q->size(1), Lq = q->size(2), D = q->size(3);
+  const Pools P(a[2], a[3], a[4], a[5], *q, B, D);
+  const int64_t mc = PyLong_Check(a[8]) ? PyLong_AsLongLong(a[8]) : -1;
+  if (!P.ok || Hq % P.Hk || !fits(mc) || !fits(B) || !fits(Hq) || !fits(Lq)) {
+    PyErr_Clear();
+    Py_RETURN_NONE;
+  }
+  if (o && (!on_gpu(*o) || o->sizes() != q->sizes() || o->scalar_type() != q->scalar_type() ||
+            o->device() != q->device() || !kernel_layout(*o)))
+    Py_RETURN_NONE;
+  const Rope rope(a[9], a[10], D, *q);
+  double scale = 1.0 / std::sqrt((double)D);
+  if (!rope.ok || (a[7] != Py_None && !number(a[7], &scale))) Py_RETURN_NONE;
+  const int causal = PyObject_IsTrue(a[6]);
+  if (causal < 0) return nullptr;
+  const c10::OptionalDeviceGuard guard(q->device());
+  const Tensor out = o ? *o : at::empty({B, Hq, Lq, D}, q->options());
+  const int64_t none3[3] = {0, 0, 1};
+  const Plan no_plan(Py_None, Py_None, Py_None, {}, *q);
+  return result(paged_launch(*q, P, out, rope, no_plan, mc, scale, causal, nullptr, nullptr, none3, none3, prefill), out);
+  CIE_PY_END
+}
+
+// One layer's fused decode / verify section:
+// section(q, k, v, k_cache, v_cache, block_tables, context_lens, max_context, cos, sin, plan data | None, split, key)
+// with q (B, Hq, L, D), k / v (B, Hk, L, D); returns (B, L, Hq * D).
+PyObject* section(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  CIE_PY_BEGIN
+  if (n != 13) Py_RETURN_NONE;
+  const Tensor *q = tensor(a[0]), *k = tensor(a[1]), *v = tensor(a[2]);
+  if (!q || !k || !v || !on_gpu(*q) || !on_gpu(*k) || !on_gpu(*v) || q->dim() != 4 || k->dim() != 4 ||
+      v->sizes() != k->sizes() || dtype_code(*q) < 0 || !head_dim_ok(q->size(3)) || !kernel_layout(*q) ||
+      !kernel_layout(*k) || !kernel_layout(*v))
+    Py_RETURN_NONE;
+  const int64_t B = q->size(0), Hq = q->size(1), L = q->size(2), D = q->size(3);
+  const Pools P(a[3], a[4], a[5], a[6], *q, B, D);
+  const int64_t mc = PyLong_Check(a[7]) ? PyLong_AsLongLong(a[7]) : -1;
+  if (!P.ok || Hq % P.Hk || !fits(mc) || !fits(B) || !fits(Hq) || !fits(L) || B * L == 0) {
+    PyErr_Clear();
+    Py_RETURN_NONE;
+  }
+  int64_t st[2][3];  // token row b * L + i of k / v: one stride over all of them
+  for (int x = 0; x < 2; ++x) {
+    const Tensor& t = x ? *v : *k;
+    if (t.size(0) != B || t.size(1) != P.Hk || t.size(2) != L || t.size(3) != D || t.scalar_type() != q->scalar_type() ||
+        t.device() != q->device() || (B > 1 && L > 1 && t.stride(0) != L * t.stride(2)))
+      Py_RETURN_NONE;
+    st[x][0] = L > 1 ? t.stride(2) : B > 1 ? t.stride(0) : 0;
+    st[x][1] = P.Hk > 1 ? t.stride(1) : 0;
+    st[x][2] = 1;
+  }
+  const Rope rope(a[8], a[9], D, *q);
+  const Plan plan(a[10], a[11], a[12], {B, Hq, P.Hk, L, D, P.num_blocks, P.block_size, P.width, mc, 1}, *q);
+  if (!rope.ok || !plan.ok) Py_RETURN_NONE;
+  const c10::OptionalDeviceGuard guard(q->device());
+  const Tensor rows = at::empty({B, L, Hq, D}, q->options());
+  const Tensor out = rows.transpose(1, 2);
+  const int rc = paged_launch(*q, P, out, rope, plan, mc, 1.0 / std::sqrt((double)D), 1, k->data_ptr(), v->data_ptr(),
+                              st[0], st[1], false);
+  return result(rc, rows.view({B, L, Hq * D}));
+  CIE_PY_END
+}
+
+// append(k_new, v_new, k_cache, v_cache, block_tables, cu_new, start, max_new, status | None, cos, sin, k_out | None);
+// returns True when done.
+PyObject* append(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  CIE_PY_BEGIN
+  if (n != 12) Py_RETURN_NONE;
+  const Tensor *k = tensor(a[0]), *v = tensor(a[1]), *cu = tensor(a[5]);
+  bool ok = k && v && cu;
+  const Tensor* status = tensor_or_none(a[8], &ok);
+  const Tensor* ko = tensor_or_none(a[11], &ok);
+  if (!ok || status || !on_gpu(*k) || !on_gpu(*v) || k->dim() != 3 || v->sizes() != k->sizes() || dtype_code(*k) < 0 ||
+      v->scalar_type() != k->scalar_type() || v->device() != k->device() || !kernel_layout(*k) || !kernel_layout(*v))
+    Py_RETURN_NONE;
+  const int64_t Hk = k->size(1), D = k->size(2), max_new = PyLong_Check(a[7]) ? PyLong_AsLongLong(a[7]) : -1;
+  if (!head_dim_ok(D) || cu->dim() != 1 || cu->size(0) < 2 || !fits(max_new)) {
+    PyErr_Clear();
+    Py_RETURN_NONE;
+  }
+  const int64_t B = cu->size(0) - 1, T = k->size(0);
+  const Pools P(a[2], a[3], a[4], a[6], *k, B, D);
+  const Rope rope(a[9], a[10], D, *k);
+  if (!P.ok || P.Hk != Hk || !fits(B) || !fits(T) || !rope.ok || !on_gpu(*cu) || cu->device() != k->device() ||
+      cu->scalar_type() != at::kInt || !cu->is_contiguous())
+    Py_RETURN_NONE;
+  if (ko && (!rope.cos || !on_gpu(*ko) || ko->sizes() != k->sizes() || ko->scalar_type() != k->scalar_type() ||
+             ko->device() != k->device() || !kernel_layout(*ko)))
+    Py_RETURN_NONE;
+  const c10::OptionalDeviceGuard guard(k->device());
+  const Strides sn(*k), sm(*v), sk(*P.kc), sv(*P.vc), so(ko ? *ko : *k);
+  void* stream = stream_of(*k);
+  const auto ip = [](const Tensor* t) { return static_cast<const int32_t*>(t->data_ptr()); };
+  const int dt = dtype_code(*k);
+  const int rc = launch(*k, [&] {
+    if (!rope.cos)
+      return api.append(k->data_ptr(), v->data_ptr(), P.kc->data_ptr(), P.vc->data_ptr(), sn.s, sm.s, sk.s, sv.s,
+                        ip(P.bt), ip(cu), ip(P.lens), nullptr, (int)B, (int)T, (int)max_new, (int)Hk, (int)D,
+                        (int)P.num_blocks, (int)P.block_size, (int)P.width, dt, stream);
+    return api.append_rope(k->data_ptr(), v->data_ptr(), P.kc->data_ptr(), P.vc->data_ptr(), sn.s, sm.s, sk.s, sv.s,
+                           ip(P.bt), ip(cu), ip(P.lens), nullptr, (int)B, (int)T, (int)max_new, (int)Hk, (int)D,
+                           (int)P.num_blocks, (int)P.block_size, (int)P.width, dt, rope.cos, rope.sin, rope.rows,
+                           rope.dt, ko ? ko->data_ptr() : nullptr, ko ? so.s : nullptr, stream);
+  });
+  if (rc) return PyLong_FromLong(rc);
+  Py_RETURN_TRUE;
+  CIE_PY_END
+}
+
+// int8(x, w_int8, scales, bias | None)
+PyObject* int8(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  CIE_PY_BEGIN
+  if (n != 4) Py_RETURN_NONE;
+  const Tensor *x = tensor(a[0]), *w = tensor(a[1]), *s = tensor(a[2]);
+  bool ok = x && w && s;
+  const Tensor* b = tensor_or_none(a[3], &ok);
+  if (!ok || !on_gpu(*x) || !on_gpu(*w) || !on_gpu(*s) || x->dim() < 1 || w->dim() != 2 || s->dim() != 1 ||
+      w->scalar_type() != at::kChar || dtype_code(*x) < 0 || any_code(*s) < 0 || w->device() != x->device() ||
+      s->device() != x->device())
+    Py_RETURN_NONE;
+  const int64_t N = w->size(0), K = w->size(1);
+  const auto aligned = [](const Tensor& t) { return !(reinterpret_cast<uintptr_t>(t.data_ptr()) & 15); };
+  if (K < 1 || x->size(-1) != K || s->size(0) != N || !s->is_contiguous() || !aligned(*x) || !aligned(*w) ||
+      w->stride(1) != 1 || w->stride(0) % 16 || w->stride(0) < K || !fits(N) || !fits(K))
+    Py_RETURN_NONE;
+  if (b && (!on_gpu(*b) || b->dim() != 1 || b->size(0) != N || b->device() != x->device() ||
+            b->scalar_type() != x->scalar_type() || !b->is_contiguous()))
+    Py_RETURN_NONE;
+  // rows of x: K apart when contiguous, or any 16-byte aligned stride of a matrix
+  int64_t xs = K;
+  if (!x->is_contiguous()) {
+    if (x->dim() != 2 || x->stride(1) != 1 || x->stride(0) < K) Py_RETURN_NONE;
+    xs = x->stride(0);
+  }
+  const int64_t M = x->numel() / K;
+  if (xs % 8 || M < 1 || N < 1 || !fits(M)) Py_RETURN_NONE;
+  const c10::OptionalDeviceGuard guard(x->device());
+  at::DimVector shape(x->sizes().begin(), x->sizes().end());
+  shape.back() = N;
+  const Tensor y = at::empty(shape, x->options());
+  const size_t nbytes = api.int8_ws((int)M, (int)N, (int)K);
+  const Tensor ws = nbytes ? bytes_like(nbytes, *x) : Tensor();
+  void* stream = stream_of(*x);
+  const int rc = launch(*x, [&] {
+    return api.int8(x->data_ptr(), static_cast<const int8_t*>(w->data_ptr()), s->data_ptr(), b ? b->data_ptr() : nullptr, y.data_ptr(), xs,
+                    w->stride(0), N, (int)M, (int)N, (int)K, dtype_code(*x), any_code(*s),
+                    nbytes ? ws.data_ptr() : nullptr, nbytes, stream);
+  });
+  return result(rc, y);
+  CIE_PY_END
+}
+
+// bind({name: address}): the library's entry points.
+PyObject* bind(PyObject*, PyObject* d) {
+  void** out = reinterpret_cast<void**>(&api);
+  for (size_t i = 0; i < kFns; ++i) {
+    PyObject* v = PyDict_GetItemString(d, kNames[i]);
+    if (!v) return PyErr_Format(PyExc_KeyError, "%s", kNames[i]);
+    out[i] = PyLong_AsVoidPtr(v);
+    if (PyErr_Occurred()) return nullptr;
+  }
+  Py_RETURN_NONE;
+}
+
+PyObject* names(PyObject*, PyObject*) {
+  PyObject* l = PyList_New(0);
+  for (const char* s : kNames) {
+    PyObject* u = PyUnicode_FromString(s);
+    PyList_Append(l, u);
+    Py_DECREF(u);
+  }
+  return l;
+}
+
+#define CIE_FAST(f) {#f, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(f)), METH_FASTCALL, nullptr}
+PyMethodDef methods[] = {CIE_FAST(flash), CIE_FAST(paged), CIE_FAST(section), CIE_FAST(append), CIE_FAST(int8),
+                         {"bind", bind, METH_O, nullptr},
+                         {"names", names, METH_NOARGS, nullptr},
+                         {nullptr, nullptr, 0, nullptr}};
+PyModuleDef module = {PyModuleDef_HEAD_INIT, "cie_host", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
+
+}  // namespace
+
+PyMODINIT_FUNC PyInit_cie_host() { return PyModule_Create(&module); }

@@ -9,12 +9,14 @@ library is missing or refuses a launch, the call raises.
 from __future__ import annotations
 
 import ctypes
+import importlib.util
 import os
 import threading
 
 import torch
 
 PKG_ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+HOST_PATH = os.path.join(PKG_ROOT, "cie_host.so")
 LIB_PATH = os.environ.get("CIE_ATTN_LIB", os.path.join(PKG_ROOT, "libcie_attn.so"))
 ABI_VERSION = 3
 
@@ -61,6 +63,7 @@ class NativeLibraryError(RuntimeError):
 
 
 _lib = None
+_host = None
 _lock = threading.Lock()
 
 _i64p = ctypes.POINTER(ctypes.c_int64)
@@ -163,6 +166,25 @@ def load() -> ctypes.CDLL:
     return _lib
 
 
+def host():
+    """Load (once) and return the extension module (``csrc/host.cpp``) that
+    makes the per-operation calls into the library."""
+    global _host
+    if _host is None:
+        lib = load()
+        with _lock:
+            if _host is None:
+                if not os.path.exists(HOST_PATH):
+                    raise NativeLibraryError(
+                        f"{HOST_PATH} is not built; run `python custom-inference-engine_amd/build_lib.py`")
+                spec = importlib.util.spec_from_file_location("cie_host", HOST_PATH)
+                mod = importlib.util.module_from_spec(spec)
+                spec.loader.exec_module(mod)
+                mod.bind({n: ctypes.cast(getattr(lib, n), ctypes.c_void_p).value for n in mod.names()})
+                _host = mod
+    return _host
+
+
 def last_error() -> str:
     return load().cie_last_error().decode()
 
@@ -175,6 +197,13 @@ def check(rc: int) -> None:
     if rc in (CIE_EHEADDIM, CIE_EDTYPE, CIE_EINVAL):
         raise ValueError(msg)
     raise NativeLibraryError(msg)
+
+
+def checked(done):
+    """The result of a ``host()`` call, or the exception of its status."""
+    if type(done) is int:
+        check(done)
+    return done
 
 
 def strides(t: torch.Tensor) -> ctypes.Array:

@@ -108,6 +108,11 @@ def flash_attention(
     unit last stride, e.g. the transposed view of a (B, M, H, D) buffer) to
     write instead of a new one.
     """
+    cos, sin = rope if rope is not None else (None, None)
+    done = _lib.host().flash(q, k, v, causal, scale, cos, sin, q_pos0 if rope is not None else None, out)
+    if done is not None:
+        return _lib.checked(done)
+    # arguments the kernels cannot take as they are: refuse, copy or convert
     if not q.is_cuda:
         raise RuntimeError("flash_attention requires CUDA tensors")
     if not (k.is_cuda and v.is_cuda) or k.device != q.device or v.device != q.device:
@@ -190,6 +195,11 @@ def paged_prefill(
     tokens, K and V read in place through the block tables. Arguments, result
     and treatment of invalid lengths and block ids as in
     :func:`paged_attention`, which is the faster one for few query rows."""
+    cos, sin = rope if rope is not None else (None, None)
+    done = _lib.host().paged(True, q, k_cache, v_cache, block_tables, context_lens, causal, scale, max_context or 0,
+                             cos, sin, out)
+    if done is not None:
+        return _lib.checked(done)
     for name, t in (("q", q), ("k_cache", k_cache), ("v_cache", v_cache),
                     ("block_tables", block_tables), ("context_lens", context_lens)):
         if not t.is_cuda or t.device != q.device:
@@ -431,6 +441,12 @@ def paged_attention(
     step's sequences (:meth:`PagedPlan.built_from` checks host copies). The
     shape is checked here (its key) and by the launch (the plan's header).
     """
+    if workspace is None and new_kv is None and plan is None:
+        cos, sin = rope if rope is not None else (None, None)
+        done = _lib.host().paged(False, q, k_cache, v_cache, block_tables, context_lens, causal, scale,
+                                 max_context or 0, cos, sin, out)
+        if done is not None:
+            return _lib.checked(done)
     for name, t in (("q", q), ("k_cache", k_cache), ("v_cache", v_cache),
                     ("block_tables", block_tables), ("context_lens", context_lens)):
         if not t.is_cuda or t.device != q.device:

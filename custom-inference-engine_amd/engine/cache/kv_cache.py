@@ -72,10 +72,20 @@ class StepBatch:
     plan: object = None          # engine.attention.PagedPlan of the step's paged launches, or None
     new_counts: tuple = ()       # new tokens per sequence (host)
     cache: dict = field(default_factory=dict, repr=False)  # device index tensors of ragged steps, built once
+    _host_flags: tuple | None = field(default=None, init=False, repr=False, compare=False)  # (fresh, aligned, total)
+
+    def _flags(self) -> tuple:
+        """(fresh, aligned, total new tokens) of the host copies, found once:
+        every layer of the step asks."""
+        if self._host_flags is None:
+            rows = list(zip(self.starts_host, self.lengths_host, self.new_counts))
+            self._host_flags = (all(s0 == 0 and n == c for s0, n, c in rows), all(s0 + c == n for s0, n, c in rows),
+                                sum(self.new_counts))
+        return self._host_flags
 
     @property
     def total_new(self) -> int:
-        return sum(self.new_counts)
+        return self._flags()[2]
 
     @property
     def max_new(self) -> int:
@@ -92,14 +102,14 @@ class StepBatch:
     def fresh(self) -> bool:
         """Every sequence holds exactly this step's tokens (a prefill from
         position 0): attention needs only the new K/V, no history."""
-        return all(s0 == 0 and n == c for s0, n, c in zip(self.starts_host, self.lengths_host, self.new_counts))
+        return self._flags()[0]
 
     @property
     def aligned(self) -> bool:
         """The new tokens are the newest of every sequence (start + count ==
         context length), so their positions are context_len - count + i, as
         the paged kernel's fused RoPE assumes."""
-        return all(s0 + c == n for s0, n, c in zip(self.starts_host, self.lengths_host, self.new_counts))
+        return self._flags()[1]
 
 
 def block_table_tensor(
@@ -147,6 +157,12 @@ def kv_append(k_new: torch.Tensor, v_new: torch.Tensor, k_cache: torch.Tensor, v
     """
     from engine import _lib
 
+    cos, sin = rope if rope is not None else (None, None)
+    done = _lib.host().append(k_new, v_new, k_cache, v_cache, block_tables, cu_new, start, max_new, status, cos, sin,
+                              k_out)
+    if done is not None:
+        _lib.checked(done)
+        return
     for name, t in (("k_new", k_new), ("v_new", v_new), ("k_cache", k_cache), ("v_cache", v_cache),
                     ("block_tables", block_tables), ("cu_new", cu_new), ("start", start)):
         if not t.is_cuda or t.device != k_cache.device:

@@ -38,6 +38,7 @@ import math
 
 import torch
 
+from engine import _lib
 from engine.attention import flash_attention, paged_attention, paged_max_rows, paged_prefill
 from engine.cache import PagedKVCache, StepBatch
 
@@ -63,6 +64,15 @@ def attention_section(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, layer_i
         raise ValueError(f"step of {step.context_lens.shape[0]} sequences x {step.num_new} tokens "
                          f"for q of shape {tuple(q.shape)}")
     Hk = k.shape[1]
+    fused = fuse_append and not step.fresh and step.aligned and (Hq // Hk) * L <= paged_max_rows(D)
+    if fused:  # decode / verify: append and attention in one call
+        plan = step.plan_for(True)
+        cos, sin = rope if rope is not None else (None, None)
+        done = _lib.host().section(q, k, v, cache.k[layer_idx], cache.v[layer_idx], step.block_tables,
+                                   step.context_lens, step.max_context, cos, sin,
+                                   *((plan.data, plan.split, plan.key) if plan is not None else (None, None, None)))
+        if done is not None:
+            return _lib.checked(done)
     scale = 1.0 / math.sqrt(D)
     # the kernels write (B, L, Hq, D) directly: the reference's
     # transpose(1, 2).contiguous() of the output (block.py:72-74) is free
@@ -83,7 +93,7 @@ def attention_section(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, layer_i
             cache.append_step(layer_idx, step, k_rows, v_rows, rope=rope, k_out=k_rot)
             flash_attention(q, k_rot.view(B, L, Hk, D).transpose(1, 2), v, causal=True, scale=scale, rope=rope,
                             out=out)  # positions 0..L-1
-    elif (Hq // Hk) * L <= paged_max_rows(D) and fuse_append and step.aligned:
+    elif fused:
         cache._validate(k_rows)
         cache._validate(v_rows)
         paged_attention(q, cache.k[layer_idx], cache.v[layer_idx], step.block_tables, step.context_lens,

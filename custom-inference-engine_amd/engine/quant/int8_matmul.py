@@ -55,6 +55,10 @@ def int8_matmul(x: torch.Tensor, w_int8: torch.Tensor, scales: torch.Tensor,
                 bias: torch.Tensor | None = None) -> torch.Tensor:
     """Per-channel INT8 x FP16/BF16 matmul: x (..., K), w_int8 (N, K) int8,
     scales (N,), optional bias (N,). Returns (..., N) in x's dtype."""
+    done = _lib.host().int8(x, w_int8, scales, bias)
+    if done is not None:
+        return _lib.checked(done)
+    # arguments the kernels cannot take as they are: refuse, copy or convert
     if not x.is_cuda:
         raise RuntimeError("int8_matmul requires CUDA tensors")
     if scales.ndim != 1:

@@ -1,0 +1,144 @@
+"""The compiled call layer (csrc/host.cpp) against the Python path it stands in
+for: the same call with the extension's functions handing everything back gives
+the same bits, over the layouts both accept (views, offsets, size-1 dimensions,
+padded rows, every table type) and those the extension hands back (misaligned,
+odd strides), in the output, the pools and the errors."""
+
+from __future__ import annotations
+
+import math
+import types
+
+import pytest
+import torch
+
+from engine import _lib
+from engine.attention import flash_attention, paged_attention, paged_prefill
+from engine.cache import KVCacheConfig, PagedKVCache
+from engine.model import attention_section, attention_section_rows
+from engine.model.rope import build_rope_cache
+from engine.quant import int8_matmul
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def _both(monkeypatch, call):
+    """call() through the extension and through Python alone: the same tensors,
+    or the same refusal (an append of rows with odd strides)."""
+
+    def outcome():
+        try:
+            return call()
+        except ValueError as e:
+            return str(e)
+
+    a = outcome()
+    back = types.SimpleNamespace(**{n: (lambda *args: None) for n in ("flash", "paged", "section", "append", "int8")})
+    with monkeypatch.context() as m:
+        m.setattr(_lib, "host", lambda: back)
+        b = outcome()
+    assert type(a) is type(b)
+    if isinstance(a, str):
+        assert a == b
+        return
+    for x, y in zip(a, b):
+        assert x.shape == y.shape and x.stride() == y.stride() and x.dtype == y.dtype
+        assert torch.equal(x.nan_to_num(7.0), y.nan_to_num(7.0)) and torch.equal(x.isnan(), y.isnan())
+
+
+def _views(g, B, H, L, D, dtype):
+    """One (B, H, L, D) tensor in the layouts callers hold."""
+    base = torch.randn(B, H, L, D, generator=g).to(dtype).to(DEV)
+    padded = torch.empty(B, H, L, D + 8, dtype=dtype, device=DEV)[..., :D]
+    padded.copy_(base)
+    odd = torch.empty(B, H, L, D + 1, dtype=dtype, device=DEV)[..., :D]
+    odd.copy_(base)
+    shifted = torch.empty(base.numel() + 1, dtype=dtype, device=DEV)[1:].view(B, H, L, D)
+    shifted.copy_(base)
+    return [base, base.transpose(1, 2).contiguous().transpose(1, 2), padded, odd, shifted,
+            base.transpose(2, 3).contiguous().transpose(2, 3)]
+
+
+@pytest.mark.parametrize("B,H,Hk,M,N,D", [(1, 4, 2, 5, 700, 64), (2, 2, 1, 130, 130, 128), (1, 1, 1, 1, 1, 32),
+                                          (2, 4, 4, 3, 0, 64), (0, 4, 2, 3, 9, 64)])
+def test_flash(monkeypatch, B, H, Hk, M, N, D):
+    g = torch.Generator().manual_seed(B + M)
+    cos, sin = (t.to(DEV) for t in build_rope_cache(2048, D))
+    pos = torch.full((B,), 7, dtype=torch.int32, device=DEV)
+    for q, k, v in zip(*(_views(g, B, h, n, D, torch.float16) for h, n in ((H, M), (Hk, N), (Hk, N)))):
+        for kw in ({}, {"causal": True, "scale": -0.3}, {"rope": (cos, sin)}, {"rope": (cos.half(), sin.half()), "q_pos0": pos},
+                   {"causal": 1, "out": torch.empty(B, M, H, D, dtype=torch.float16, device=DEV).transpose(1, 2)}):
+            _both(monkeypatch, lambda: (flash_attention(q, k, v, **kw).clone(),))
+
+
+@pytest.mark.parametrize("L,D,dtype", [(1, 64, torch.float16), (5, 128, torch.bfloat16), (90, 64, torch.float16)])
+@pytest.mark.parametrize("rope", [None, "f32", "x"])
+def test_sections(monkeypatch, L, D, dtype, rope):
+    Hq, Hk, hist = 8, 2, [70, 0, 33, 400]
+    g = torch.Generator().manual_seed(L)
+    cos, sin = build_rope_cache(1024, D)
+    tabs = None if rope is None else tuple(t.to(DEV, torch.float32 if rope == "f32" else dtype) for t in (cos, sin))
+    data = [torch.randn(400, 16, Hk, D, generator=g).to(dtype).to(DEV) for _ in range(2)]
+    B = len(hist)
+    qs, ks, vs = (_views(g, B, h, L, D, dtype) for h in (Hq, Hk, Hk))
+
+    def run(q, k, v, plan, rows):
+        cache = PagedKVCache(KVCacheConfig(1, Hk, D, 400, 16, dtype, DEV))
+        cache.k[0].copy_(data[0]), cache.v[0].copy_(data[1])
+        tables = [cache.new_sequence() for _ in hist]
+        for t, n in zip(tables, hist):
+            t.length = n
+        step = cache.prepare_step(tables, L, num_heads=Hq if plan else None)
+        if rows:
+            q, k, v = (x.transpose(1, 2).reshape(B * L, -1, D) for x in (q, k, v))
+            o = attention_section_rows(q, k, v, 0, cache, step, rope=tabs)
+        else:
+            o = attention_section(q, k, v, 0, cache, step, rope=tabs)
+        return o, cache.k[0], cache.v[0]
+
+    for q, k, v in zip(qs, ks, vs):
+        for plan, rows in ((False, False), (True, False), (False, True)):
+            _both(monkeypatch, lambda: run(q, k, v, plan, rows))
+
+
+def test_paged(monkeypatch):
+    g = torch.Generator().manual_seed(3)
+    kp, vp = (torch.randn(40, 16, 2, 64, generator=g).half().to(DEV) for _ in range(2))
+    bt = torch.randperm(40, generator=g).view(2, 20).int().to(DEV)
+    lens = torch.tensor([300, 17], dtype=torch.int32, device=DEV)
+    for q in _views(g, 2, 4, 3, 64, torch.float16):
+        for t, n in ((bt, lens), (bt.long(), lens.long()), (bt.repeat(1, 2)[:, :20], lens)):
+            for kw in ({}, {"max_context": 310, "scale": 0.2}, {"causal": False}, {"max_context": 16}):
+                _both(monkeypatch, lambda: (paged_attention(q, kp, vp, t, n, **kw), paged_prefill(q, kp, vp, t, n, **kw)))
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 24, 64), (3, 40, 100), (130, 136, 192), (0, 8, 64)])
+def test_int8(monkeypatch, M, N, K):
+    g = torch.Generator().manual_seed(M + K)
+    w = torch.randint(-127, 128, (N, K), generator=g).to(torch.int8).to(DEV)
+    wp = torch.empty(N, K + 16 - K % 16, dtype=torch.int8, device=DEV)[:, :K]
+    wp.copy_(w)
+    s = torch.rand(N, generator=g).to(DEV)
+    for dtype in (torch.float16, torch.bfloat16):
+        x = torch.randn(M, K, generator=g).to(dtype).to(DEV)
+        xp = torch.empty(M, K + 8, dtype=dtype, device=DEV)[:, :K]
+        xp.copy_(x)
+        for xx in (x, xp, x.view(1, M, K), x.t().contiguous().t()):
+            for ww in (w, wp):
+                for ss in (s, s.half(), s.double()):
+                    for b in (None, s.to(dtype), s.half()):
+                        _both(monkeypatch, lambda: (int8_matmul(xx, ww, ss, bias=b),))
+
+
+def test_errors_keep_their_types():
+    q = torch.zeros(1, 2, 4, 64, dtype=torch.float16, device=DEV)
+    for bad in (q.float(), q[..., :48], q.cpu()):
+        with pytest.raises((ValueError, RuntimeError)):
+            flash_attention(bad, bad, bad)
+    with pytest.raises(ValueError):
+        flash_attention(q, q, q, scale=math.inf)  # refused by the library
+    with pytest.raises(ValueError):
+        flash_attention(q, q, q, out=torch.empty(1, 2, 4, 65, dtype=torch.float16, device=DEV)[..., :64])
+    with pytest.raises(ValueError):
+        flash_attention(q, q, q, rope=(torch.zeros(4, 32, device=DEV), torch.zeros(5, 32, device=DEV)))
