@@ -174,7 +174,7 @@ int cie_prefill_kernel(int B, int Hq, int Hk, int Lq, int Lk, int D, int causal,
 static int flash_set_splits(cie::FlashParams* p, int D, int splits, void* workspace, size_t workspace_bytes) {
   if (splits < 0 || splits > cie::kFlashMaxSplits)
     return fail(CIE_EINVAL, "splits must be in [0, %d], got %d", cie::kFlashMaxSplits, splits);
-  p->splits = splits ? splits : cie::flash_splits(*p, D);
+  p->splits = splits ? splits : cie::flash_splits(*p, D, p->bt != nullptr);
   const size_t need = cie::flash_part_bytes(*p, D, p->splits);
   if (need == 0) return CIE_OK;
   if ((int64_t)p->n_wg * p->splits > 0x7fffffff / (4 * 32))  // workgroups of the merge pass
@@ -247,9 +247,7 @@ static int paged_ctx_limit(int max_context, int block_size, int max_blocks_per_s
   return (int)(max_context > 0 ? std::min<int64_t>(max_context, bound) : bound);
 }
 
-extern "C" {
-
-size_t cie_flash_workspace_bytes(int B, int Hq, int Hk, int Lq, int Lk, int D, int causal, int splits) {
+static size_t flash_workspace(int B, int Hq, int Hk, int Lq, int Lk, int D, int causal, int splits, bool paged) {
   if (B <= 0 || Hq <= 0 || Hk <= 0 || Lq <= 0 || Lk <= 0 || Hq % Hk || !head_dim_ok(D) || splits < 0 ||
       splits > cie::kFlashMaxSplits)
     return 0;
@@ -261,7 +259,13 @@ size_t cie_flash_workspace_bytes(int B, int Hq, int Hk, int Lq, int Lk, int D, i
   p.n_wg = (int)(n_mt * B * Hq);
   p.causal = causal ? 1 : 0;
   p.cus = cie::device_shape().cus;
-  return cie::flash_part_bytes(p, D, splits ? splits : cie::flash_splits(p, D));
+  return cie::flash_part_bytes(p, D, splits ? splits : cie::flash_splits(p, D, paged));
+}
+
+extern "C" {
+
+size_t cie_flash_workspace_bytes(int B, int Hq, int Hk, int Lq, int Lk, int D, int causal, int splits) {
+  return flash_workspace(B, Hq, Hk, Lq, Lk, D, causal, splits, false);
 }
 
 int cie_flash_fwd_ex(const void* q, const void* k, const void* v, void* o,
@@ -283,8 +287,7 @@ int cie_flash_fwd_ex(const void* q, const void* k, const void* v, void* o,
 size_t cie_flash_paged_workspace_bytes(int B, int Hq, int Hk, int Lq, int D, int max_context, int block_size,
                                        int max_blocks_per_seq, int splits) {
   if (block_size <= 0 || max_blocks_per_seq <= 0 || (int64_t)max_blocks_per_seq * block_size > 0x7fffffff) return 0;
-  return cie_flash_workspace_bytes(B, Hq, Hk, Lq, paged_ctx_limit(max_context, block_size, max_blocks_per_seq), D, 1,
-                                   splits);
+  return flash_workspace(B, Hq, Hk, Lq, paged_ctx_limit(max_context, block_size, max_blocks_per_seq), D, 1, splits, true);
 }
 
 int cie_flash_paged(const void* q, const void* k_cache, const void* v_cache, const int32_t* block_tables,
@@ -787,6 +790,76 @@ int cie_kv_append_rope(const void* k_new, const void* v_new, void* k_cache, void
   return append_impl(k_new, v_new, k_cache, v_cache, new_stride, v_new_stride, kc_stride, vc_stride, block_tables,
                      cu_new, start, status, B, T, max_new, Hk, D, num_blocks, block_size, max_blocks_per_seq, dtype,
                      stream, cie::RopeTables{rope_cos, rope_sin, rope_rows, rope_dtype}, k_out, k_out_stride);
+}
+
+// Strides in bytes. `start`: position of the first row, ids[0] the block of
+// position 0. Launches of at most kMoveIds blocks each.
+static int move_impl(const char* what, bool gather, void* k_dense, void* v_dense, void* k_cache, void* v_cache,
+                     const int64_t* dense_stride, const int64_t* pool_stride, const int32_t* ids, int n_ids,
+                     int64_t start, int64_t L, int heads, int64_t head_bytes, int num_blocks, int block_size,
+                     void* stream) {
+  if (L < 0 || start < 0 || heads < 1 || head_bytes < 16 || head_bytes % 16 || block_size < 1 || num_blocks < 0 ||
+      n_ids < 0 || start + L > 0x7fffffff)
+    return fail(CIE_EINVAL, "%s: invalid sizes", what);
+  if (L == 0) {
+    g_err.clear();
+    return CIE_OK;
+  }
+  if (!ids || !dense_stride || !pool_stride) return fail(CIE_EINVAL, "%s: NULL pointer", what);
+  CIE_TRY(check_ptr("k", k_dense));
+  CIE_TRY(check_ptr("v", v_dense));
+  CIE_TRY(check_ptr("k_cache", k_cache));
+  CIE_TRY(check_ptr("v_cache", v_cache));
+  if ((start + L + block_size - 1) / block_size > n_ids)
+    return fail(CIE_EINVAL, "%s: %lld positions need more than %d blocks", what, (long long)(start + L), n_ids);
+  for (int i = 0; i < 4; ++i)
+    if (dense_stride[i] < 0 || dense_stride[i] % 16) return fail(CIE_EINVAL, "%s: rows must be 16-byte aligned", what);
+  for (int i = 0; i < 6; ++i)
+    if (pool_stride[i] < 0 || pool_stride[i] % 16) return fail(CIE_EINVAL, "%s: pool rows must be 16-byte aligned", what);
+  if (gather)  // every id is read
+    for (int64_t b = start / block_size; b <= (start + L - 1) / block_size; ++b)
+      if (ids[b] < 0 || ids[b] >= num_blocks)
+        return fail(CIE_EINVAL, "%s: block id %d is outside the pool of %d blocks", what, ids[b], num_blocks);
+  cie::MoveParams p;
+  const int64_t cph = head_bytes / 16, cpr = cph * heads;
+  if (cpr > 0x3fffffff) return fail(CIE_EINVAL, "%s: token rows too large", what);
+  p.cpr = (uint32_t)cpr, p.cph = (uint32_t)cph;
+  p.cprdiv = cie::make_fastdiv(p.cpr), p.cphdiv = cie::make_fastdiv(p.cph);
+  p.bsdiv = cie::make_fastdiv((uint32_t)block_size);
+  p.block_size = block_size, p.num_blocks = num_blocks;
+  p.pool[0] = static_cast<char*>(k_cache), p.pool[1] = static_cast<char*>(v_cache);
+  for (int t = 0; t < 2; ++t) {
+    p.pool_block[t] = pool_stride[3 * t], p.pool_token[t] = pool_stride[3 * t + 1], p.pool_head[t] = pool_stride[3 * t + 2];
+    p.dense_token[t] = dense_stride[2 * t], p.dense_head[t] = dense_stride[2 * t + 1];
+  }
+  for (int64_t done = 0; done < L;) {
+    const int64_t pos = start + done, b0 = pos / block_size;
+    const int64_t n = std::min<int64_t>({L - done, (b0 + cie::kMoveIds) * block_size - pos, 0x7fffffff / cpr});
+    const int64_t nb = (pos + n - 1) / block_size - b0 + 1;
+    std::copy(ids + b0, ids + b0 + nb, p.ids);
+    std::fill(p.ids + nb, p.ids + cie::kMoveIds, -1);
+    p.start = (int)(pos - b0 * block_size);
+    p.total = (uint32_t)(n * cpr);
+    p.dense[0] = static_cast<char*>(k_dense) + done * dense_stride[0];
+    p.dense[1] = static_cast<char*>(v_dense) + done * dense_stride[2];
+    CIE_TRY(launch_status(cie::launch_kv_move(p, gather, static_cast<hipStream_t>(stream))));
+    done += n;
+  }
+  return CIE_OK;
+}
+
+int cie_kv_append_seq(const void* k_new, const void* v_new, void* k_cache, void* v_cache, const int64_t* new_stride,
+                      const int64_t* pool_stride, const int32_t* block_ids, int n_blocks, int64_t start, int64_t L,
+                      int heads, int64_t head_bytes, int num_blocks, int block_size, void* stream) {
+  return move_impl("append", false, const_cast<void*>(k_new), const_cast<void*>(v_new), k_cache, v_cache, new_stride,
+                   pool_stride, block_ids, n_blocks, start, L, heads, head_bytes, num_blocks, block_size, stream);
+}
+
+int cie_kv_gather(const void* k_cache, const void* v_cache, void* k, void* v, const int64_t* out_stride,
+                  const int64_t* pool_stride, const int32_t* block_ids, int n_blocks, int64_t L, int heads,
+                  int64_t head_bytes, int num_blocks, int block_size, void* stream) {
+  return move_impl("gather", true, k, v, const_cast<void*>(k_cache), const_cast<void*>(v_cache), out_stride,
+                   pool_stride, block_ids, n_blocks, 0, L, heads, head_bytes, num_blocks, block_size, stream);
 }
 
 size_t cie_int8_matmul_workspace_bytes(int M, int N, int K) {

@@ -1577,19 +1577,19 @@ FlashKernel flash_kernel_choice(const FlashParams& p, int D) {
 // keys alone; with them every partial state is written and read once more. The
 // estimate, in microseconds: a workgroup walks its tiles at kStep each (25 %
 // slower when the waves of two workgroups share a CU; one wave of a short query
-// tile does not notice), launches in rounds of the workgroup slots, and a
+// tile does not notice; 15 % slower over a paged history), launches in rounds of the workgroup slots, and a
 // split launch pays 4.2 us and 0.3 us per split for its second pass plus its
 // partial states at 1.6 MB/us. Measured, splits: us (B x Hq x Lq x Lk, D, causal):
 //   1x32x5x3001 D=64      1: 35.3  2: 22.5  4: 14.8  8: 11.9  16: 13.3
 //   1x32x5x300 D=64       1: 6.7   2: 8.4   4: 8.1
 //   1x32x5x16384 D=128    1: 260   4: 71.6  8: 40.7  16: 28.1
-//   1x32x300x1500 D=64    1: 21.9  2: 19.3  4: 18.9  8: 24.8
+//   1x32x300x1500 D=64    1: 21.9  2: 19.3  4: 18.9  8: 24.8 (paged 1: 24.8  2: 21.3  4: 20.1)
 //   1x32x1000x4600 D=128  1: 87.4  2: 78.2  3: 88.4  4: 84.6
 //   1x16x512x512 D=64     1: 10.0  2: 11.8  4: 13.3
 //   1x32x500x500 D=128    1: 14.6  2: 22.7
-int flash_splits(const FlashParams& p, int D) {
+int flash_splits(const FlashParams& p, int D, bool paged) {
   const int bn = D <= 32 ? 128 : (D == 64 ? 64 : 32);
-  const double kStep = D == 256 ? 1.35 : D == 128 ? 0.6 : D == 64 ? 0.75 : 1.05;
+  const double kStep = (paged ? 1.15 : 1.0) * (D == 256 ? 1.35 : D == 128 ? 0.6 : D == 64 ? 0.75 : 1.05);
   const int64_t items = p.n_wg, per_cu = D <= 128 ? 2 : 1, slots = per_cu * p.cus;
   const int64_t nt = ((int64_t)p.Lk + bn - 1) / bn;  // tiles of the longest item
   if (items < 1 || items >= slots) return 1;

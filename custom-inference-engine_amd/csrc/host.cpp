@@ -21,6 +21,7 @@
 #include <torch/csrc/autograd/python_variable.h>
 
 #include <cmath>
+#include <vector>
 
 #include "cie_attn.h"
 
@@ -35,12 +36,14 @@ struct Api {
   decltype(&cie_paged_fwd_ex) paged;
   decltype(&cie_kv_append) append;
   decltype(&cie_kv_append_rope) append_rope;
+  decltype(&cie_kv_append_seq) append_seq;
+  decltype(&cie_kv_gather) gather;
   decltype(&cie_int8_matmul_workspace_bytes) int8_ws;
   decltype(&cie_int8_matmul) int8;
 } api;
 const char* const kNames[] = {"cie_flash_workspace_bytes", "cie_flash_fwd_ex", "cie_flash_paged_workspace_bytes",
                               "cie_flash_paged", "cie_paged_workspace_bytes", "cie_paged_fwd_ex", "cie_kv_append",
-                              "cie_kv_append_rope", "cie_int8_matmul_workspace_bytes", "cie_int8_matmul"};
+                              "cie_kv_append_rope", "cie_kv_append_seq", "cie_kv_gather", "cie_int8_matmul_workspace_bytes", "cie_int8_matmul"};
 constexpr size_t kFns = sizeof(kNames) / sizeof(kNames[0]);
 static_assert(sizeof(Api) == kFns * sizeof(void*), "one name per function, in order");
 
@@ -375,6 +378,111 @@ PyObject* append(PyObject*, PyObject* const* a, Py_ssize_t n) {
   CIE_PY_END
 }
 
+// Block ids of a BlockTable's list.
+bool id_list(PyObject* o, std::vector<int32_t>* ids) {
+  if (!PyList_CheckExact(o)) return false;
+  const Py_ssize_t n = PyList_GET_SIZE(o);
+  ids->resize((size_t)n);
+  for (Py_ssize_t i = 0; i < n; ++i) {
+    PyObject* x = PyList_GET_ITEM(o, i);
+    const long long v = PyLong_CheckExact(x) ? PyLong_AsLongLong(x) : -2;
+    if (v < 0 || v > 0x7fffffff) {
+      PyErr_Clear();
+      return false;
+    }
+    (*ids)[(size_t)i] = (int32_t)v;
+  }
+  return true;
+}
+
+// The two pools of a layer, (num_blocks, block_size, heads, D) of any element
+// type, head rows of a multiple of 16 bytes, 16-byte aligned.
+struct SeqPools {
+  int64_t strides[6];
+  int64_t head_bytes = 0;
+  bool ok;
+  SeqPools(const Tensor* k, const Tensor* v) {
+    ok = k && v && on_gpu(*k) && on_gpu(*v) && k->dim() == 4 && k->sizes() == v->sizes() && k->device() == v->device() &&
+         k->scalar_type() == v->scalar_type() && k->numel() > 0;
+    if (!ok) return;
+    const int64_t e = k->element_size();
+    head_bytes = k->size(3) * e;
+    ok = head_bytes % 16 == 0;
+    for (const Tensor* t : {k, v}) {
+      ok = ok && t->stride(3) == 1 && !(reinterpret_cast<uintptr_t>(t->data_ptr()) & 15);
+      for (int i = 0; i < 3; ++i) {
+        const int64_t st = t->size(i) == 1 ? 0 : t->stride(i) * e;
+        strides[(t == v ? 3 : 0) + i] = st;
+        ok = ok && st >= 0 && st % 16 == 0;
+      }
+      ok = ok && fits(t->size(0)) && fits(t->size(1)) && fits(t->size(2));
+    }
+  }
+};
+
+// append_seq(k_new, v_new, k_cache, v_cache, blocks, start): (L, heads, D) rows
+// to positions start ..; True when done.
+PyObject* append_seq(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  CIE_PY_BEGIN
+  if (n != 6) Py_RETURN_NONE;
+  const Tensor *k = tensor(a[0]), *v = tensor(a[1]), *kc = tensor(a[2]), *vc = tensor(a[3]);
+  std::vector<int32_t> ids;
+  // (the engine's 16-bit caches only, as the append through device tables)
+  if (!k || !v || !on_gpu(*k) || !on_gpu(*v) || k->dim() != 3 || v->sizes() != k->sizes() || dtype_code(*k) < 0 ||
+      k->size(0) < 1 || !id_list(a[4], &ids) || !PyLong_Check(a[5]))
+    Py_RETURN_NONE;
+  const SeqPools P(kc, vc);
+  if (!P.ok || !head_dim_ok(k->size(2)) || kc->size(2) != k->size(1) || kc->size(3) != k->size(2) ||
+      kc->device() != k->device() || v->device() != k->device() || kc->scalar_type() != k->scalar_type() ||
+      v->scalar_type() != k->scalar_type() || !kernel_layout(*k) || !kernel_layout(*v))
+    Py_RETURN_NONE;
+  const int64_t start = PyLong_AsLongLong(a[5]), L = k->size(0);
+  if (PyErr_Occurred() || start < 0 || start + L > (int64_t)ids.size() * kc->size(1)) {
+    PyErr_Clear();
+    Py_RETURN_NONE;
+  }
+  const Strides sk(*k), sv(*v);
+  const int64_t dense[4] = {2 * sk.s[0], 2 * sk.s[1], 2 * sv.s[0], 2 * sv.s[1]};
+  const c10::OptionalDeviceGuard guard(k->device());
+  void* stream = stream_of(*k);
+  const int rc = launch(*k, [&] {
+    return api.append_seq(k->data_ptr(), v->data_ptr(), kc->data_ptr(), vc->data_ptr(), dense, P.strides, ids.data(),
+                          (int)ids.size(), start, L, (int)kc->size(2), P.head_bytes, (int)kc->size(0),
+                          (int)kc->size(1), stream);
+  });
+  if (rc) return PyLong_FromLong(rc);
+  Py_RETURN_TRUE;
+  CIE_PY_END
+}
+
+// gather(k_cache, v_cache, blocks, L): dense (L, heads, D) copies of both
+PyObject* gather(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  CIE_PY_BEGIN
+  if (n != 4) Py_RETURN_NONE;
+  const Tensor *kc = tensor(a[0]), *vc = tensor(a[1]);
+  std::vector<int32_t> ids;
+  if (!kc || !vc || !id_list(a[2], &ids) || !PyLong_Check(a[3])) Py_RETURN_NONE;
+  const SeqPools P(kc, vc);
+  const int64_t L = PyLong_AsLongLong(a[3]);
+  if (!P.ok || PyErr_Occurred() || L < 1 || !fits(L) || L > (int64_t)ids.size() * kc->size(1)) {
+    PyErr_Clear();
+    Py_RETURN_NONE;
+  }
+  const c10::OptionalDeviceGuard guard(kc->device());
+  const int64_t heads = kc->size(2);
+  const Tensor k = at::empty({L, heads, kc->size(3)}, kc->options()), v = at::empty_like(k);
+  const int64_t dense[4] = {heads * P.head_bytes, P.head_bytes, heads * P.head_bytes, P.head_bytes};
+  void* stream = stream_of(*kc);
+  const int rc = launch(*kc, [&] {
+    return api.gather(kc->data_ptr(), vc->data_ptr(), k.data_ptr(), v.data_ptr(), dense, P.strides, ids.data(),
+                      (int)ids.size(), L, (int)heads, P.head_bytes, (int)kc->size(0), (int)kc->size(1), stream);
+  });
+  if (rc) return PyLong_FromLong(rc);
+  PyObject *pk = THPVariable_Wrap(k), *pv = THPVariable_Wrap(v);
+  return pk && pv ? Py_BuildValue("(NN)", pk, pv) : nullptr;
+  CIE_PY_END
+}
+
 // int8(x, w_int8, scales, bias | None)
 PyObject* int8(PyObject*, PyObject* const* a, Py_ssize_t n) {
   CIE_PY_BEGIN
@@ -441,7 +549,8 @@ PyObject* names(PyObject*, PyObject*) {
 }
 
 #define CIE_FAST(f) {#f, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(f)), METH_FASTCALL, nullptr}
-PyMethodDef methods[] = {CIE_FAST(flash), CIE_FAST(paged), CIE_FAST(section), CIE_FAST(append), CIE_FAST(int8),
+PyMethodDef methods[] = {CIE_FAST(flash), CIE_FAST(paged), CIE_FAST(section), CIE_FAST(append), CIE_FAST(append_seq),
+                         CIE_FAST(gather), CIE_FAST(int8),
                          {"bind", bind, METH_O, nullptr},
                          {"names", names, METH_NOARGS, nullptr},
                          {nullptr, nullptr, 0, nullptr}};

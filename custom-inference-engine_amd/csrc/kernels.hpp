@@ -70,7 +70,7 @@ struct FlashParams {
 constexpr int kFlashIds = 1024;       // block ids of a workgroup's key range staged in LDS
 constexpr int kFlashMaxSplits = 32;
 // Splits of a launch (p.n_wg = B * Hq * n_mt, p.Lk the most keys a row sees) and the bytes of its partial states.
-int flash_splits(const FlashParams& p, int D);
+int flash_splits(const FlashParams& p, int D, bool paged);
 size_t flash_part_bytes(const FlashParams& p, int D, int splits);
 
 // Prefill kernel a launch takes (launch_flash); cie_prefill_kernel reports it.
@@ -248,6 +248,22 @@ struct AppendParams {
   int64_t os0, os1;       // k_out strides (token, head)
 };
 
+// One sequence's token rows between dense (L, ...) tensors and the pool, its
+// block ids in the argument block (kv_move_kernel). All strides in bytes.
+constexpr int kMoveIds = 768;  // block ids of one launch (12288 tokens of 16-token blocks; 4 KB of arguments)
+struct MoveParams {
+  char* pool[2];          // K, V
+  char* dense[2];
+  int64_t pool_block[2], pool_token[2], pool_head[2];
+  int64_t dense_token[2], dense_head[2];
+  uint32_t total;         // 16-byte chunks of one tensor: L * cpr
+  uint32_t cpr, cph;      // chunks per token row, per head row
+  FastDiv cprdiv, cphdiv, bsdiv;
+  int start;              // position of row 0 relative to the first id's block
+  int block_size, num_blocks;
+  int32_t ids[kMoveIds];
+};
+
 // Standalone RoPE of x (B, H, L, D) into out (may be x itself).
 struct RopeParams {
   const uint16_t* x;
@@ -305,6 +321,7 @@ hipError_t set_dynamic_lds(const void* kernel, int bytes);
 hipError_t launch_flash(const FlashParams& p, int dtype, int D, hipStream_t stream);
 hipError_t launch_int8_gemm(const I8GemmParams& p, const I8Geom& g, int dtype, hipStream_t stream);
 hipError_t launch_kv_append(const AppendParams& p, int B, int max_new, int dtype, int D, hipStream_t stream);
+hipError_t launch_kv_move(const MoveParams& p, bool gather, hipStream_t stream);
 hipError_t launch_rope(const RopeParams& p, int dtype, int D, hipStream_t stream);
 // merge: launch the merge pass of split sequences (false only when a plan
 // says no sequence is split)

@@ -161,6 +161,57 @@ __global__ __launch_bounds__(256) void kv_append_rope_kernel(const AppendParams 
   }
 }
 
+// One sequence's rows between dense tensors and the pool (PagedKVCache.append
+// and gather), one 16-byte chunk of K or of V per thread and trip. The block
+// ids travel in the argument block: staged in device memory they took a
+// host-to-device copy per call, which holds the host up until the stream has
+// drained (append + gather of 3001 tokens of 8 x 64 heads: 3 copies and
+// kernels plus two waits, 45 us of host time; now two launches).
+// Launched with the chunks of K in blockIdx.y = 0 and of V in 1. Ids outside
+// the pool are skipped.
+constexpr int kMoveUnroll = 2;
+
+template <bool GATHER>
+__global__ __launch_bounds__(256) void kv_move_kernel(const MoveParams p) {
+  const int t = blockIdx.y;
+  char* const pool = p.pool[t];
+  char* const dense = p.dense[t];
+  const uint32_t stride = gridDim.x * 256u;
+  for (uint32_t c0 = blockIdx.x * 256u + threadIdx.x; c0 < p.total; c0 += kMoveUnroll * stride) {
+    u32x4 v[kMoveUnroll];
+    char* dst[kMoveUnroll];
+    bool ok[kMoveUnroll];
+#pragma unroll
+    for (int u = 0; u < kMoveUnroll; ++u) {
+      const uint32_t c = c0 + u * stride;
+      const uint32_t cc = c < p.total ? c : c0;
+      const uint32_t i = fdiv(cc, p.cprdiv), ch = cc - i * p.cpr;
+      const uint32_t h = fdiv(ch, p.cphdiv), d = ch - h * p.cph;
+      const uint32_t pos = (uint32_t)p.start + i;
+      const uint32_t blk = fdiv(pos, p.bsdiv), off = pos - blk * (uint32_t)p.block_size;
+      const int id = p.ids[blk];
+      ok[u] = c < p.total && (uint32_t)id < (uint32_t)p.num_blocks;
+      char* const a = pool + (ok[u] ? id : 0) * p.pool_block[t] + off * p.pool_token[t] + h * p.pool_head[t] + 16 * d;
+      char* const b = dense + i * p.dense_token[t] + h * p.dense_head[t] + 16 * d;
+      v[u] = u32x4{0u, 0u, 0u, 0u};
+      if (ok[u]) v[u] = *reinterpret_cast<const u32x4*>(GATHER ? a : b);
+      dst[u] = GATHER ? b : a;
+    }
+#pragma unroll
+    for (int u = 0; u < kMoveUnroll; ++u)
+      if (ok[u]) *reinterpret_cast<u32x4*>(dst[u]) = v[u];
+  }
+}
+
+hipError_t launch_kv_move(const MoveParams& p, bool gather, hipStream_t stream) {
+  const unsigned gx = (unsigned)std::min<uint32_t>(1024u, (p.total + 256u * kMoveUnroll - 1) / (256u * kMoveUnroll));
+  if (gather)
+    hipLaunchKernelGGL(kv_move_kernel<true>, dim3(gx, 2), dim3(256), 0, stream, p);
+  else
+    hipLaunchKernelGGL(kv_move_kernel<false>, dim3(gx, 2), dim3(256), 0, stream, p);
+  return hipGetLastError();
+}
+
 hipError_t launch_kv_append(const AppendParams& p, int B, int max_new, int dtype, int D, hipStream_t stream) {
   if (B <= 0 || max_new <= 0) return hipSuccess;
   (void)D;

@@ -47,6 +47,8 @@ EXPORTED_SYMBOLS = (
     "cie_paged_plan",
     "cie_paged_fwd_ex",
     "cie_kv_append",
+    "cie_kv_append_seq",
+    "cie_kv_gather",
     "cie_rope_apply",
     "cie_flash_fwd_rope",
     "cie_paged_fwd_rope",
@@ -119,6 +121,12 @@ def _declare(lib: ctypes.CDLL) -> None:
     lib.cie_kv_append.argtypes = [_vp, _vp, _vp, _vp, _i64p, _i64p, _i64p, _i64p, _vp, _vp, _vp, _vp,
                                   _i, _i, _i, _i, _i, _i, _i, _i, _i, _vp]
     lib.cie_kv_append.restype = _i
+    lib.cie_kv_append_seq.argtypes = [_vp, _vp, _vp, _vp, _i64p, _i64p, _vp, _i, ctypes.c_int64, ctypes.c_int64,
+                                      _i, ctypes.c_int64, _i, _i, _vp]
+    lib.cie_kv_append_seq.restype = _i
+    lib.cie_kv_gather.argtypes = [_vp, _vp, _vp, _vp, _i64p, _i64p, _vp, _i, ctypes.c_int64, _i, ctypes.c_int64,
+                                  _i, _i, _vp]
+    lib.cie_kv_gather.restype = _i
     lib.cie_rope_apply.argtypes = [_vp, _vp, _i64p, _i64p, _vp, ctypes.c_int64, _vp, _vp, _i, _i, _vp,
                                    _i, _i, _i, _i, _i, _vp]
     lib.cie_rope_apply.restype = _i

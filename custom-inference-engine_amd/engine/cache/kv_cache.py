@@ -279,6 +279,14 @@ class PagedKVCache:
         while len(table.blocks) < table.num_blocks_needed(end):
             table.blocks.append(self._alloc_block())
         if L and self.device.type == "cuda":
+            from engine import _lib
+
+            # one launch, the block ids among its arguments
+            done = _lib.host().append_seq(k, v, self.k[layer], self.v[layer], table.blocks, start)
+            if done is not None:
+                _lib.checked(done)
+                table.length = max(table.length, end)
+                return
             # one launch; block ids, row offsets and start travel in one small copy
             first = start // self.cfg.block_size
             ids = table.blocks[first:table.num_blocks_needed(end)]
@@ -426,6 +434,13 @@ class PagedKVCache:
         if L == 0:
             empty = self.k[layer].new_zeros((0, Hk, D))
             return empty, empty.clone()
+        if self.device.type == "cuda":
+            from engine import _lib
+
+            # one launch, the block ids among its arguments
+            done = _lib.host().gather(self.k[layer], self.v[layer], table.blocks, L)
+            if done is not None:
+                return _lib.checked(done)
         idx = torch.tensor(table.blocks, dtype=torch.long, device=self.device)
         k = self.k[layer].index_select(0, idx).reshape(-1, Hk, D)[:L]
         v = self.v[layer].index_select(0, idx).reshape(-1, Hk, D)[:L]

@@ -258,6 +258,24 @@ int cie_kv_append(const void* k_new, const void* v_new, void* k_cache, void* v_c
                   int num_blocks, int block_size, int max_blocks_per_seq, int dtype, void* stream);
 
 /*
+ * One sequence's rows into, or out of, one layer's pools, its block ids given
+ * in HOST memory (read during the call; they reach the kernel as arguments, so
+ * nothing is copied to the device first). Row i of k / v is position start + i
+ * (gather: i), in block block_ids[position / block_size]. A token row is
+ * `heads` rows of head_bytes bytes (any element type; a multiple of 16).
+ * Strides in bytes, multiples of 16: dense {k token, k head, v token, v head},
+ * pool {k block, k token, k head, v block, v token, v head}. The append skips
+ * tokens whose block id lies outside the pool, the gather refuses them.
+ * Reference: engine/cache/kv_cache.py:102-139 (append), :141-165 (gather).
+ */
+int cie_kv_append_seq(const void* k_new, const void* v_new, void* k_cache, void* v_cache, const int64_t* new_stride,
+                      const int64_t* pool_stride, const int32_t* block_ids, int n_blocks, int64_t start, int64_t L,
+                      int heads, int64_t head_bytes, int num_blocks, int block_size, void* stream);
+int cie_kv_gather(const void* k_cache, const void* v_cache, void* k, void* v, const int64_t* out_stride,
+                  const int64_t* pool_stride, const int32_t* block_ids, int n_blocks, int64_t L, int heads,
+                  int64_t head_bytes, int num_blocks, int block_size, void* stream);
+
+/*
  * Rotary position embedding (RoPE).
  *
  * rope_cos, rope_sin: device tables of shape (rope_rows, D/2), row-major and

@@ -15,7 +15,8 @@ def test_binds_exported_entry_points():
     assert set(_lib.host().names()) <= set(_lib.EXPORTED_SYMBOLS)
 
 
-@pytest.mark.parametrize("name,n", [("flash", 9), ("paged", 12), ("section", 13), ("append", 12), ("int8", 4)])
+@pytest.mark.parametrize("name,n", [("flash", 9), ("paged", 12), ("section", 13), ("append", 12), ("append_seq", 6), ("gather", 4),
+                                    ("int8", 4)])
 def test_other_arguments_are_handed_back(name, n):
     fn = getattr(_lib.host(), name)
     t = torch.zeros(1, 2, 4, 16, dtype=torch.float16)

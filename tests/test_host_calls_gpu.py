@@ -34,7 +34,8 @@ def _both(monkeypatch, call):
             return str(e)
 
     a = outcome()
-    back = types.SimpleNamespace(**{n: (lambda *args: None) for n in ("flash", "paged", "section", "append", "int8")})
+    back = types.SimpleNamespace(**{n: (lambda *args: None) for n in ("flash", "paged", "section", "append", "append_seq",
+                                                                   "gather", "int8")})
     with monkeypatch.context() as m:
         m.setattr(_lib, "host", lambda: back)
         b = outcome()
@@ -142,3 +143,44 @@ def test_errors_keep_their_types():
         flash_attention(q, q, q, out=torch.empty(1, 2, 4, 65, dtype=torch.float16, device=DEV)[..., :64])
     with pytest.raises(ValueError):
         flash_attention(q, q, q, rope=(torch.zeros(4, 32, device=DEV), torch.zeros(5, 32, device=DEV)))
+
+
+@pytest.mark.parametrize("Hk,D,bs,dtype", [(8, 64, 16, torch.float16), (2, 128, 5, torch.bfloat16), (3, 16, 1, torch.float16),
+                                           (2, 256, 32, torch.bfloat16)])
+def test_append_and_gather_of_one_sequence(monkeypatch, Hk, D, bs, dtype):
+    """Rows to and from scattered blocks, starts inside a block, and (one-token
+    blocks) more block ids than one launch's arguments hold."""
+    g = torch.Generator().manual_seed(D + bs)
+    N = 1700
+    data = [torch.randn(N // bs + 9, bs, Hk, D, generator=g).to(dtype).to(DEV) for _ in range(2)]
+    order = torch.randperm(N // bs + 9, generator=g).tolist()
+
+    def run(rows, start, shape):
+        cache = PagedKVCache(KVCacheConfig(1, Hk, D, N // bs + 9, bs, dtype, DEV))
+        cache.k[0].copy_(data[0]), cache.v[0].copy_(data[1])
+        cache._free = list(order)
+        t = cache.new_sequence()
+        t.blocks = [cache._alloc_block() for _ in range(-(-start // bs))]
+        t.length = start
+        gg = torch.Generator().manual_seed(rows)
+        k, v = (shape(torch.randn(rows, Hk, D, generator=gg).to(dtype).to(DEV)) for _ in range(2))
+        cache.append(0, t, k, v)
+        assert t.length == start + rows
+        return (*cache.gather(0, t), cache.k[0], cache.v[0])
+
+    views = (lambda x: x, lambda x: x.transpose(0, 1).contiguous().transpose(0, 1),
+             lambda x: torch.cat([x, x], dim=2)[:, :, :D])
+    for rows, start in ((1, 0), (5, 700), (33, 31), (1000, 3), (1, 1600)):
+        for shape in views:
+            _both(monkeypatch, lambda: run(rows, start, shape))
+
+
+def test_gather_of_other_caches(monkeypatch):
+    """An fp32 cache (gathered, never attended over) and an empty sequence."""
+    for dtype, D in ((torch.float32, 24), (torch.float16, 12)):
+        cache = PagedKVCache(KVCacheConfig(1, 2, D, 6, 4, dtype, DEV))
+        cache.k[0].normal_(), cache.v[0].normal_()
+        t = cache.new_sequence()
+        assert cache.gather(0, t)[0].shape == (0, 2, D)
+        t.blocks, t.length = [5, 0, 3], 10
+        _both(monkeypatch, lambda: cache.gather(0, t))
