@@ -6,7 +6,7 @@
 //
 // Arithmetic. int8 values are exact in fp16 and bf16, so the weights are
 // converted in registers (fp16: byte | 0x6400 is 1024 + byte, minus 1152;
-// bf16: byte -> f32 -> bf16) and multiplied against x on the matrix cores
+// bf16: sign-extended byte -> f32 -> bf16) and multiplied against x on the matrix cores
 // (v_mfma_f32_32x32x16_{f16,bf16}) with fp32 accumulation: the products are
 // exact, as in the reference, which up-casts both operands to fp32 before
 // tl.dot (:47-53). The scale multiplies the fp32 sum once per output
@@ -116,9 +116,11 @@ template <> __device__ __forceinline__ void dequant16<1>(u32x4 q, u32x4& a0, u32
   uint32_t o[8];
 #pragma unroll
   for (int d = 0; d < 4; ++d) {
-    const uint32_t u = q[d] ^ 0x80808080u;
-    const float f0 = (float)(u & 0xffu) - 128.0f, f1 = (float)((u >> 8) & 0xffu) - 128.0f;
-    const float f2 = (float)((u >> 16) & 0xffu) - 128.0f, f3 = (float)(u >> 24) - 128.0f;
+    // sign-extending conversions: one instruction a byte (biasing the bytes and
+    // subtracting 128 took two; 512 x 4096 x 4096 33.7 -> 30.4 us, 1999 rows 95 -> 87)
+    const int u = (int)q[d];
+    const float f0 = (float)(int8_t)u, f1 = (float)(int8_t)(u >> 8);
+    const float f2 = (float)(int8_t)(u >> 16), f3 = (float)(u >> 24);
     o[2 * d] = Elt<1>::pack2(f0, f1);
     o[2 * d + 1] = Elt<1>::pack2(f2, f3);
   }
