@@ -81,7 +81,10 @@ struct I8Cfg {
   static constexpr int BM = 32 * MT;
   static constexpr int NST = NST_;  // LDS ring stages
   static constexpr int NT = 256 * KW;                    // threads
-  static constexpr int X_BYTES = BM * kI8BK * 2;        // x tile per stage
+  // x rows staged: BM, or 128 at MT = 3 (whose 96 rows do not split over eight
+  // waves; the last 32 are copied and never read)
+  static constexpr int XROWS = MT == 3 ? 128 : BM;
+  static constexpr int X_BYTES = XROWS * kI8BK * 2;     // x tile per stage
   static constexpr int W_BYTES = kI8BN * kI8BK;         // w tile per stage
   static constexpr int STAGE = X_BYTES + W_BYTES;
   static constexpr int XI = X_BYTES / (NT * 16);        // x copies per lane per stage
@@ -883,14 +886,18 @@ I8Geom int8_gemm_geometry(int M, int N, int K, DeviceShape dev) {
   const int64_t cus = dev.cus;
   const int64_t t128 = (int64_t)g.n_tiles * ((M + 127) / 128), t64 = (int64_t)g.n_tiles * ((M + 63) / 64);
   g.mt = t128 >= 2 * cus ? 4 : (t64 >= 2 * cus ? 2 : (t128 >= cus ? 4 : 2));
+  // More 64-row tiles than CUs gives some CUs two and others one; 96 rows then
+  // still give every CU at most one tile, at 3/4 of the longest CU's work
+  // (1400 x 2048 x 2048 fp16: 352 tiles of 64 rows 26.5 us, 240 of 96 24.7).
+  if (g.mt == 2 && t64 > cus && t64 < 2 * cus && (int64_t)g.n_tiles * ((M + 95) / 96) <= cus) g.mt = 3;
   // 3-4 ring stages let two workgroups share a CU
-  g.nst = g.mt >= 4 ? 3 : 4;
+  g.nst = g.mt >= 3 ? 3 : 4;
   const int bm = 32 * g.mt;
   g.m_tiles = (M + bm - 1) / bm;
   const int64_t tiles = (int64_t)g.m_tiles * g.n_tiles;
   // split K only as far as needed for one workgroup per CU, keeping >= 4 k steps per split
   int s = 1;
-  if (tiles < cus) s = (int)std::min<int64_t>((cus + tiles - 1) / tiles, std::max(1, g.ksteps / 4));
+  if (tiles < cus && g.mt != 3) s = (int)std::min<int64_t>((cus + tiles - 1) / tiles, std::max(1, g.ksteps / 4));
   g.splits = std::max(1, std::min(s, kI8MaxSplits));
   // one workgroup per CU or fewer: eight waves (two k halves) so every SIMD
   // holds two waves (512 x 4096 x 4096: 31.9 -> 30.1 us); else four waves and
@@ -900,7 +907,7 @@ I8Geom int8_gemm_geometry(int M, int N, int K, DeviceShape dev) {
   g.m_pad = g.m_tiles * bm;
   g.n_pad = g.n_tiles * kI8BN;
   g.workspace_bytes = g.splits > 1 ? (size_t)g.splits * g.m_pad * g.n_pad * sizeof(float) : 0;
-  g.lds_bytes = (size_t)g.nst * (bm * kI8BK * 2 + kI8BN * kI8BK);
+  g.lds_bytes = (size_t)g.nst * ((g.mt == 3 ? 128 : bm) * kI8BK * 2 + kI8BN * kI8BK);  // (I8Cfg::XROWS)
   return g;
 }
 
@@ -954,6 +961,7 @@ static hipError_t launch_i8_d(const I8GemmParams& p, const I8Geom& g, hipStream_
     return launch_ws_t<DTYPE, 64, 2, 4>(p, stream);
   }
   if (g.mt == 2 && g.nst == 4) return launch_i8_t<DTYPE, 2, 4>(p, g.lds_bytes, g.kw2, stream);
+  if (g.mt == 3 && g.nst == 3) return launch_i8_t<DTYPE, 3, 3>(p, g.lds_bytes, g.kw2, stream);
   if (g.mt == 4 && g.nst == 3) return launch_i8_t<DTYPE, 4, 3>(p, g.lds_bytes, g.kw2, stream);
   return hipErrorInvalidValue;
 }
