@@ -33,9 +33,10 @@
 // Any K. The reference masks the K tail of its last tile
 // (kernels/int8_matmul.py:43-50). Here each kernel's main loop covers the
 // largest prefix of K its step divides (64 for the tiled kernel, 32 for the
-// streaming one, 16 for the dot kernel) and never reads past it; the
-// remaining k < 64 terms of every output are added in the epilogue, in fp32
-// with exact products and in ascending k, before the scale is applied.
+// streaming one, 16 for the dot kernel) and never reads past it. The tiled
+// kernel takes the rest as one more step with zeros behind K; in the others
+// the remaining k < 32 terms of every output are added in the epilogue, in
+// fp32 with exact products and in ascending k, before the scale is applied.
 //
 // Split K. When the (n, m) tiles alone cannot occupy the GPU, the K steps
 // are cut into `splits` contiguous ranges; each
@@ -281,16 +282,8 @@ __global__ __launch_bounds__(256 * KW, KW == 1 ? 2 : 1) void int8_gemm_kernel(co
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt) acc[mt] = f32x16{};
 
-  // One barrier per step: it publishes step t and, as every wave has left
-  // step t-1, frees that step's stage, which is refilled at once with step
-  // t + NST - 1 (NST - 1 steps in flight during the compute of step t).
-  const int pro = min(C::NST - 1, T);
-  for (int t = 0; t < pro; ++t) issue(t);
-  for (int t = 0; t < T; ++t) {
-    wait_steps_ahead<C::PER, C::NST - 2>(min(C::NST - 2, T - 1 - t));  // steps issued after step t
-    __syncthreads();  // step t is in LDS for every wave; the stage of step t-1 is free
-    if (t + C::NST - 1 < T) issue(t + C::NST - 1);
-    const uint8_t* st = smem + (t % C::NST) * C::STAGE;
+  // One step from the stage at st: this wave's k halves of it.
+  auto compute = [&](const uint8_t* st) CIE_GV_INLINE {
     // every fragment of the step is read first, so the LDS latency is paid
     // once per step rather than in front of each MFMA
     // (this wave's k halves g2 = kh G2 .. kh G2 + G2 - 1 of the step)
@@ -314,6 +307,55 @@ __global__ __launch_bounds__(256 * KW, KW == 1 ? 2 : 1) void int8_gemm_kernel(co
         acc[mt] = E::mfma(a1, xb[mt][i][1], acc[mt]);
       }
     }
+  };
+
+  // One barrier per step: it publishes step t and, as every wave has left
+  // step t-1, frees that step's stage, which is refilled at once with step
+  // t + NST - 1 (NST - 1 steps in flight during the compute of step t).
+  const int pro = min(C::NST - 1, T);
+  for (int t = 0; t < pro; ++t) issue(t);
+  for (int t = 0; t < T; ++t) {
+    wait_steps_ahead<C::PER, C::NST - 2>(min(C::NST - 2, T - 1 - t));  // steps issued after step t
+    __syncthreads();  // step t is in LDS for every wave; the stage of step t-1 is free
+    if (t + C::NST - 1 < T) issue(t + C::NST - 1);
+    compute(smem + (t % C::NST) * C::STAGE);
+  }
+  // The K tail past the last whole step, as one more step of the last split:
+  // staged by plain loads with zeros behind K (a tail of 40 k added on the
+  // vector pipe, one byte load per weight and k, took longer than the 15 steps
+  // before it: 3000 x 1000 x 1000 bf16 86 us, now 25, the padding
+  // copies of unaligned rows included).
+  const int k_main = p.ksteps * kI8BK;
+  if (k_main < p.K && split == p.splits - 1) {
+    __syncthreads();  // no wave reads the ring any more
+    for (int P = threadIdx.x; P < C::XROWS * 8; P += C::NT) {
+      const int r = P >> 3, c = P & 7, k = k_main + 8 * c;
+      const uint16_t* src = p.x + (int64_t)min(m0 + r, p.M - 1) * p.xs + k;
+      u32x4 v = {0u, 0u, 0u, 0u};
+      if (k + 8 <= p.K) {
+        v = load16_clamped(src);
+      } else {
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+          if (k + e < p.K) v[e >> 1] |= (uint32_t)src[e] << (16 * (e & 1));
+      }
+      *reinterpret_cast<u32x4*>(smem + r * 128 + 16 * (c ^ chunk_swizzle<8>(r))) = v;
+    }
+    for (int P = threadIdx.x; P < kI8BN * 4; P += C::NT) {
+      const int r = P >> 2, c = P & 3, k = k_main + 16 * c;
+      const uint8_t* src = reinterpret_cast<const uint8_t*>(p.w) + (int64_t)min(n0 + r, p.N - 1) * p.wsr + k;
+      u32x4 v = {0u, 0u, 0u, 0u};
+      if (k + 16 <= p.K) {
+        v = *reinterpret_cast<const u32x4*>(src);
+      } else {
+#pragma unroll
+        for (int e = 0; e < 16; ++e)
+          if (k + e < p.K) v[e >> 2] |= (uint32_t)src[e] << (8 * (e & 3));
+      }
+      *reinterpret_cast<u32x4*>(smem + C::X_BYTES + r * 64 + 16 * (c ^ chunk_swizzle<4>(r))) = v;
+    }
+    __syncthreads();
+    compute(smem);
   }
   if constexpr (KW == 2) {
     // the k-half-1 sums join the k-half-0 ones through LDS (fixed order:
@@ -336,39 +378,6 @@ __global__ __launch_bounds__(256 * KW, KW == 1 ? 2 : 1) void int8_gemm_kernel(co
 
   // C[i][j] of a 32x32 tile: lane j + 32 * ((i / 4) % 2), element (i / 8) * 4 + i % 4;
   // here i = weight row (n), j = activation row (m)
-  const int k_main = p.ksteps * kI8BK;  // k of the MFMA steps; the last split adds the tail
-  if (k_main < p.K && split == p.splits - 1) {
-    // this lane's MT activation rows and 16 weight rows, clamped into the
-    // tensors (rows past M / N are never stored); each tail k loads every
-    // row's element once
-    const uint16_t* xr[MT];
-    const int8_t* wr[16];
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt) xr[mt] = p.x + (int64_t)min(m0 + mt * 32 + r32, p.M - 1) * p.xs;
-#pragma unroll
-    for (int el = 0; el < 16; ++el)
-      wr[el] = p.w + (int64_t)min(n0 + w * 32 + 8 * (el >> 2) + 4 * hk + (el & 3), p.N - 1) * p.wsr;
-    float ta[MT][16];
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-      for (int el = 0; el < 16; ++el) ta[mt][el] = 0.f;
-    for (int k = k_main; k < p.K; ++k) {
-      float xv[MT], wv[16];
-#pragma unroll
-      for (int mt = 0; mt < MT; ++mt) xv[mt] = elt_to_f32<DTYPE>(xr[mt][k]);
-#pragma unroll
-      for (int el = 0; el < 16; ++el) wv[el] = (float)wr[el][k];
-#pragma unroll
-      for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-        for (int el = 0; el < 16; ++el) ta[mt][el] = fmaf(xv[mt], wv[el], ta[mt][el]);
-    }
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-      for (int el = 0; el < 16; ++el) acc[mt][el] += ta[mt][el];
-  }
   if (p.splits == 1) {
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) {

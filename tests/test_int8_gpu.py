@@ -182,3 +182,32 @@ def test_repeated_calls_are_deterministic():
     a = int8_matmul(xr, wd, sd)
     for _ in range(3):
         assert torch.equal(int8_matmul(xr, wd, sd), a)
+
+
+@pytest.mark.parametrize("M,N,K", [(65, 128, 63), (96, 130, 64), (97, 96, 65), (130, 300, 100), (200, 130, 1000),
+                                   (700, 4096, 200), (1400, 2048, 129), (1343, 2050, 96), (256, 8192, 40)])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_tiled_kernel_tails_and_tile_heights(M, N, K, dtype):
+    """K tails of 1..63 behind no, one or several whole steps, with and without
+    a K split, and 64-, 96- and 128-row tiles (700 x 4096 and 1400 x 2048 take
+    96 rows on 256 CUs), with exact arithmetic: products and sums of small
+    integers are exact in fp32 in any order, so the result is bit-exact. Every
+    byte value from -128 to 127 is among the weights; an infinity in a row of x
+    reaches that row alone, and no value behind K reaches anything."""
+    g = torch.Generator().manual_seed(M + K)
+    x = torch.randint(-4, 5, (M, K), generator=g).to(dtype)
+    w = torch.randint(-128, 128, (N, K), generator=g).to(torch.int8)
+    w.view(-1)[:256] = torch.arange(-128, 128).to(torch.int8)
+    s = (2.0 ** -torch.randint(6, 10, (N,), generator=g).float()).half()
+    want = (x.double() @ w.double().t() * s.double()).to(dtype)
+    # rows padded with values that would show: huge activations, full-scale weights
+    xp = torch.full((M, -(-K // 8) * 8 + 8), float("inf"), dtype=dtype, device=DEV)
+    wp = torch.full((N, -(-K // 16) * 16 + 16), 127, dtype=torch.int8, device=DEV)
+    xp[:, :K], wp[:, :K] = x.to(DEV), w.to(DEV)
+    for xd, wd in ((x.to(DEV), w.to(DEV)), (xp[:, :K], wp[:, :K])):
+        assert torch.equal(int8_matmul(xd, wd, s.to(DEV)).cpu(), want)
+    xi = x.to(DEV)
+    xi[M // 2, K - 1] = float("inf")
+    y = int8_matmul(xi, w.to(DEV), s.to(DEV)).cpu()
+    keep = torch.arange(M) != M // 2
+    assert torch.equal(y[keep], want[keep]) and not torch.isfinite(y[M // 2]).all()
