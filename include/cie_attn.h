@@ -396,9 +396,9 @@ int cie_paged_fwd_rope(const void* q, const void* k_cache, const void* v_cache,
  * already counts them, as after the reference's append). k_new, v_new:
  * (B * Lq, Hk, D), row b * Lq + i = new token i of sequence b, strides
  * {token, head} in elements (multiples of 8), unit head_dim stride,
- * 16-byte aligned. Attention reads those rows straight from k_new / v_new;
- * each is also written into the pool at position context_lens[b] - Lq + i
- * through the block table, so the pool afterwards equals what cie_kv_append
+ * 16-byte aligned. Each row is written into the pool at position
+ * context_lens[b] - Lq + i through the block table, by the workgroup that
+ * attends over it and before it does, so the pool afterwards equals what cie_kv_append
  * leaves, and o equals cie_kv_append then cie_paged_fwd bit for bit.
  * A context shorter than Lq is invalid here (NaN output, nothing written);
  * a token whose block id is out of range is not written (its sequence's
