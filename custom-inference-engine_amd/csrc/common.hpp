@@ -46,6 +46,11 @@ template <> struct Elt<0> {
   static __device__ __forceinline__ uint32_t pack2(float lo, float hi) {
     return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{lo, hi}, f16x2));
   }
+  // What pack2 rounded off, packed: pack2(lo, hi) + rest2(...) is lo, hi to twice the digits.
+  static __device__ __forceinline__ uint32_t rest2(uint32_t pk, float lo, float hi) {
+    const f16x2 h = __builtin_bit_cast(f16x2, pk);
+    return pack2(lo - (float)h[0], hi - (float)h[1]);
+  }
   // acc + lo + hi of a packed pair (v_dot2c_f32_f16 against ones).
   static __device__ __forceinline__ float sum2(uint32_t pk, float acc) {
     return __builtin_amdgcn_fdot2(__builtin_bit_cast(f16x2, pk), f16x2{(_Float16)1.f, (_Float16)1.f}, acc, false);
@@ -75,6 +80,9 @@ template <> struct Elt<1> {
   }
   static __device__ __forceinline__ uint32_t pack2(float lo, float hi) {
     return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{lo, hi}, bf16x2));
+  }
+  static __device__ __forceinline__ uint32_t rest2(uint32_t pk, float lo, float hi) {
+    return pack2(lo - __uint_as_float(pk << 16), hi - __uint_as_float(pk & 0xffff0000u));
   }
   static __device__ __forceinline__ float sum2(uint32_t pk, float acc) {
     return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, pk), bf16x2{(__bf16)1.f, (__bf16)1.f}, acc,

@@ -105,6 +105,18 @@ struct FlashCfg {
 //             through the int32 block table, with or without splits.
 enum KvMode { kKvDense = 0, kKvSplit = 1, kKvPaged = 2 };
 
+// Paged launches keep P in two 16-bit parts, the rounded p and what the
+// rounding left (Elt::rest2), with a P.V product for each, and sum the fp32 p:
+// a chunk over a history must not be less precise than paged_fwd_kernel's
+// launches over it, whose ranges of a tile or two have a reference max of their
+// own (the largest p of every tile is exactly 1 there). Relative error against
+// 64 bits, paged_fwd_kernel's launches / one part / two parts (32/8 heads):
+// 1000 on 4600 at D=128 bf16 2.17e-3 / 2.32e-3 / 1.66e-3, 300 on 1500 at D=64
+// fp16 2.52e-4 / 2.86e-4 / 2.07e-4 (1.66e-3 and 2.07e-4 are the rounding of
+// the output alone); time 888 / 94 / 115 us and 248 / 32 / 33 us.
+template <int MODE>
+constexpr bool kTwoPartP = MODE == kKvPaged;
+
 // The work item of a workgroup. Workgroups are dispatched round-robin over
 // the XCDs; each XCD gets a contiguous run of logical items so the query heads
 // of a kv head (and its neighbouring query tiles) share one L2. Within a kv
@@ -488,7 +500,7 @@ __global__ __launch_bounds__(256, FlashCfg<D>::OCC) void flash_fwd_kernel(const 
     // turning S(t) into P(t) next to its QK MFMAs issues first and the other
     // wave's P.V phase fills the gaps (measured 4-5 % faster at D=64).
     __builtin_amdgcn_s_setprio(1);
-    u32x4 pb[2 * C::MT];
+    u32x4 pb[2 * C::MT], pr[kTwoPartP<MODE> ? 2 * C::MT : 1];  // P(t), its rest
     f32x4 tsm[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};  // this lane's sums of the tile's p
     {
       const uint16_t* ks = ring + st1 * C::STAGE;
@@ -516,10 +528,16 @@ __global__ __launch_bounds__(256, FlashCfg<D>::OCC) void flash_fwd_kernel(const 
             const uint32_t pk = E::pack2(sc[m2][ee - 1], sc[m2][ee]);
             asm volatile("" ::"v"(pk));  // pin the work of this chunk next to its MFMA
             pb[2 * m2 + (ee >> 3)][(ee & 7) >> 1] = pk;
+            if constexpr (kTwoPartP<MODE>) {
+              const uint32_t rs = E::rest2(pk, sc[m2][ee - 1], sc[m2][ee]);
+              asm volatile("" ::"v"(rs));
+              pr[2 * m2 + (ee >> 3)][(ee & 7) >> 1] = rs;
+              tsm[(ee >> 1) & 1][0] += sc[m2][ee - 1] + sc[m2][ee];
+            }
           }
           // four p of P(t) are packed: their sum on the matrix pipe (a DOT
           // instruction per pair would wait for the pipe to drain)
-          if ((ee & 3) == 3) {
+          if (!kTwoPartP<MODE> && (ee & 3) == 3) {
             const int cb = 2 * m2 + (ee >> 3), w = (ee & 7) >> 1;
             tsm[(ee >> 2) & 1] = E::mfma4(sum_ones, u32x2{pb[cb][w - 1], pb[cb][w]}, tsm[(ee >> 2) & 1]);
           }
@@ -543,15 +561,20 @@ __global__ __launch_bounds__(256, FlashCfg<D>::OCC) void flash_fwd_kernel(const 
       l *= alpha;
 #pragma unroll
       for (int dt = 0; dt < C::DT; ++dt) acc[dt] *= alpha;
+      tsm[0] = tsm[1] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int e = 0; e < 16 * C::MT; e += 2) {
         const int m2 = e / 16, ee = e % 16;
-        pb[2 * m2 + (ee >> 3)][(ee & 7) >> 1] =
-            E::pack2(exp2_fast(fmaf(sc[m2][ee], c, nm)), exp2_fast(fmaf(sc[m2][ee + 1], c, nm)));
+        const float p0 = exp2_fast(fmaf(sc[m2][ee], c, nm)), p1 = exp2_fast(fmaf(sc[m2][ee + 1], c, nm));
+        const uint32_t pk = E::pack2(p0, p1);
+        pb[2 * m2 + (ee >> 3)][(ee & 7) >> 1] = pk;
+        if constexpr (kTwoPartP<MODE>) {
+          pr[2 * m2 + (ee >> 3)][(ee & 7) >> 1] = E::rest2(pk, p0, p1);
+          tsm[(ee >> 1) & 1][0] += p0 + p1;
+        }
       }
-      tsm[0] = tsm[1] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int cc = 0; cc < 2 * C::MT; ++cc) {
+      for (int cc = 0; cc < (kTwoPartP<MODE> ? 0 : 2 * C::MT); ++cc) {
         tsm[0] = E::mfma4(sum_ones, u32x2{pb[cc][0], pb[cc][1]}, tsm[0]);
         tsm[1] = E::mfma4(sum_ones, u32x2{pb[cc][2], pb[cc][3]}, tsm[1]);
       }
@@ -582,6 +605,7 @@ __global__ __launch_bounds__(256, FlashCfg<D>::OCC) void flash_fwd_kernel(const 
       for (int i = 0; i < C::NPV; ++i) {
         const int dt = i % C::DT, cc = i / C::DT;  // alternate accumulators
         acc[dt] = E::mfma(va[dt * 2 * C::MT + cc], pb[cc], acc[dt]);
+        if constexpr (kTwoPartP<MODE>) acc[dt] = E::mfma(va[dt * 2 * C::MT + cc], pr[cc], acc[dt]);
       }
     }
   };
@@ -857,6 +881,8 @@ __global__ __launch_bounds__(256, 2) void flash_fwd_il_kernel(const FlashParams 
 
   f32x16 sA[C::MT], sB[C::MT];
   u32x4 pA[C::NCC], pB[C::NCC];
+  constexpr int NR = kTwoPartP<MODE> ? C::NCC : 1;
+  u32x4 rA[NR], rB[NR];  // the rests of pA, pB
   if (n_tiles > 0) {
     wait_tiles<C::PER_TILE, C::AHEAD>(pro - 1);
     __syncthreads();
@@ -870,7 +896,7 @@ __global__ __launch_bounds__(256, 2) void flash_fwd_il_kernel(const FlashParams 
   // 16-bit P.V operand; always the case for a row that had no visible key
   // before) recomputes S(tc) from the resident K tile, raises m to its row
   // max, rescales O and l, and redoes its p; the other rows keep theirs.
-  auto check = [&](const int tc, const uint16_t* kst, u32x4* pq, float ts) CIE_INLINE {
+  auto check = [&](const int tc, const uint16_t* kst, u32x4* pq, u32x4* rq2, float ts) CIE_INLINE {
     const bool trig = !(ts <= kSumTrigger);
     if (__builtin_amdgcn_ballot_w64(trig)) {
       f32x16 s2[C::MT];
@@ -883,16 +909,21 @@ __global__ __launch_bounds__(256, 2) void flash_fwd_il_kernel(const FlashParams 
       l *= alpha;
 #pragma unroll
       for (int dt = 0; dt < C::DT; ++dt) acc[dt] *= alpha;
+      f32x4 t2[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
 #pragma unroll
       for (int e = 0; e < C::NE; e += 2) {
         const int m2 = e / 16, ee = e % 16;
-        const uint32_t w = pq[2 * m2 + (ee >> 3)][(ee & 7) >> 1];
-        pq[2 * m2 + (ee >> 3)][(ee & 7) >> 1] =
-            trig ? E::pack2(exp2_fast(fmaf(s2[m2][ee], c, nm)), exp2_fast(fmaf(s2[m2][ee + 1], c, nm))) : w;
+        const float p0 = exp2_fast(fmaf(s2[m2][ee], c, nm)), p1 = exp2_fast(fmaf(s2[m2][ee + 1], c, nm));
+        const int cb = 2 * m2 + (ee >> 3), w = (ee & 7) >> 1;
+        const uint32_t pk = E::pack2(p0, p1);
+        if (trig) pq[cb][w] = pk;
+        if constexpr (kTwoPartP<MODE>) {
+          if (trig) rq2[cb][w] = E::rest2(pk, p0, p1);
+          t2[(ee >> 1) & 1][0] += p0 + p1;
+        }
       }
-      f32x4 t2[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
 #pragma unroll
-      for (int cc = 0; cc < C::NCC; ++cc) {
+      for (int cc = 0; cc < (kTwoPartP<MODE> ? 0 : C::NCC); ++cc) {
         t2[0] = E::mfma4(sum_ones, u32x2{pq[cc][0], pq[cc][1]}, t2[0]);
         t2[1] = E::mfma4(sum_ones, u32x2{pq[cc][2], pq[cc][3]}, t2[1]);
       }
@@ -903,8 +934,9 @@ __global__ __launch_bounds__(256, 2) void flash_fwd_il_kernel(const FlashParams 
   };
 
   // One pipeline step t: ST = t % NST, PV = t > 0. sc = S(t), sn receives
-  // S(t+1), pb receives P(t), pp holds P(t-1).
-  auto step = [&](auto ST, auto PV, const int t, f32x16* sc, f32x16* sn, u32x4* pb, u32x4* pp) CIE_INLINE {
+  // S(t+1), pb receives P(t), pp holds P(t-1); rb and rp their rests.
+  auto step = [&](auto ST, auto PV, const int t, f32x16* sc, f32x16* sn, u32x4* pb, u32x4* pp, u32x4* rb,
+                  u32x4* rp) CIE_INLINE {
     constexpr int st = decltype(ST)::value;
     constexpr int st1 = (st + 1) % C::NST, stp = (st + C::NST - 1) % C::NST;
     constexpr bool has_pv = decltype(PV)::value;
@@ -946,8 +978,14 @@ __global__ __launch_bounds__(256, 2) void flash_fwd_il_kernel(const FlashParams 
           const uint32_t pk = E::pack2(sc[m2][ee - 1], sc[m2][ee]);
           asm volatile("" ::"v"(pk));  // pin the work of this chunk next to its MFMA
           pb[2 * m2 + (ee >> 3)][(ee & 7) >> 1] = pk;
+          if constexpr (kTwoPartP<MODE>) {
+            const uint32_t rs = E::rest2(pk, sc[m2][ee - 1], sc[m2][ee]);
+            asm volatile("" ::"v"(rs));
+            rb[2 * m2 + (ee >> 3)][(ee & 7) >> 1] = rs;
+            tsum[(ee >> 1) & 1][0] += sc[m2][ee - 1] + sc[m2][ee];
+          }
         }
-        if ((ee & 3) == 3) {
+        if (!kTwoPartP<MODE> && (ee & 3) == 3) {
           const int cb = 2 * m2 + (ee >> 3), w = (ee & 7) >> 1;
           tsum[(ee >> 2) & 1] = E::mfma4(sum_ones, u32x2{pb[cb][w - 1], pb[cb][w]}, tsum[(ee >> 2) & 1]);
         }
@@ -968,13 +1006,17 @@ __global__ __launch_bounds__(256, 2) void flash_fwd_il_kernel(const FlashParams 
       __builtin_amdgcn_sched_barrier(0);
       chunk(std::integral_constant<int, 2 * i + 1>{});
       __builtin_amdgcn_sched_barrier(0);
+      if constexpr (has_pv && kTwoPartP<MODE>) {
+        acc[i % C::DT] = E::mfma(va[i], rp[i / C::DT], acc[i % C::DT]);
+        __builtin_amdgcn_sched_barrier(0);
+      }
     });
     __builtin_amdgcn_s_setprio(0);
-    check(t, ring + st * C::STAGE, pb, xhalf_sum(tsum[0][0] + tsum[1][0]));
+    check(t, ring + st * C::STAGE, pb, rb, xhalf_sum(tsum[0][0] + tsum[1][0]));
     mask(t + 1, sn);
   };
 
-  if (n_tiles > 0) step(std::integral_constant<int, 0>{}, std::false_type{}, 0, sA, sB, pA, pB);
+  if (n_tiles > 0) step(std::integral_constant<int, 0>{}, std::false_type{}, 0, sA, sB, pA, pB, rA, rB);
   constexpr int U = 2 * C::NST;  // stage and buffer parity repeat
   for (int t = 1; t < n_tiles; t += U) {
     static_for<U>([&](auto I) CIE_INLINE {
@@ -982,9 +1024,9 @@ __global__ __launch_bounds__(256, 2) void flash_fwd_il_kernel(const FlashParams 
       constexpr int st = (1 + i) % C::NST;
       if (t + i < n_tiles) {
         if constexpr ((1 + i) % 2 == 1)
-          step(std::integral_constant<int, st>{}, std::true_type{}, t + i, sB, sA, pB, pA);
+          step(std::integral_constant<int, st>{}, std::true_type{}, t + i, sB, sA, pB, pA, rB, rA);
         else
-          step(std::integral_constant<int, st>{}, std::true_type{}, t + i, sA, sB, pA, pB);
+          step(std::integral_constant<int, st>{}, std::true_type{}, t + i, sA, sB, pA, pB, rA, rB);
       }
     });
   }
@@ -992,15 +1034,18 @@ __global__ __launch_bounds__(256, 2) void flash_fwd_il_kernel(const FlashParams 
   if (wave_nt > 0 && wave_nt == n_tiles) {
     const int tl = n_tiles - 1;
     const uint16_t* vs = ring + (tl % C::NST) * C::STAGE + C::TILE;
-    auto fin = [&](const u32x4* pq) CIE_INLINE {
+    auto fin = [&](const u32x4* pq, const u32x4* rq2) CIE_INLINE {
       u32x4 va[C::NPV];
 #pragma unroll
       for (int i = 0; i < C::NPV; ++i) va[i] = vfrag(vs, i % C::DT, i / C::DT);
 #pragma unroll
-      for (int i = 0; i < C::NPV; ++i) acc[i % C::DT] = E::mfma(va[i], pq[i / C::DT], acc[i % C::DT]);
+      for (int i = 0; i < C::NPV; ++i) {
+        acc[i % C::DT] = E::mfma(va[i], pq[i / C::DT], acc[i % C::DT]);
+        if constexpr (kTwoPartP<MODE>) acc[i % C::DT] = E::mfma(va[i], rq2[i / C::DT], acc[i % C::DT]);
+      }
     };
-    if (tl & 1) fin(pB);
-    else fin(pA);
+    if (tl & 1) fin(pB, rB);
+    else fin(pA, rA);
   }
 
   // Epilogue: rows with keys but none visible give 0 * inf = NaN like the

@@ -137,3 +137,30 @@ def test_paged_prefill_matches_oracle(D, bs, dtype, rope):
                 _close(o, want, TOL[dtype], f"splits={splits}")
             else:
                 assert torch.isnan(o[5]).all() and torch.isnan(o[4, :, Lq - 1]).all()
+
+
+@pytest.mark.parametrize("D", [16, 32, 64, 128, 256])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("rising", [False, True])
+def test_paged_prefill_error_is_the_rounding_of_its_output(D, dtype, rising):
+    """P in two 16-bit parts leaves about 16 (bf16) to 22 (fp16) of its bits and
+    the row sums stay in fp32, so against 64 bits the result is off by its one
+    rounding to 16 bits and little else (with P rounded to 16 bits it would be
+    1.4 times that). rising: scores that grow along the keys past 2^10 take the
+    recompute of the running max."""
+    Hq, Hk, Lq, n, bs = 4, 2, 150, 1203, 16
+    g = torch.Generator().manual_seed(D)
+    nb = -(-n // bs)
+    kp, vp = (_randn(g, nb, bs, Hk, D, dtype=dtype) for _ in range(2))
+    q = _randn(g, 1, Hq, Lq, D, dtype=dtype)
+    if rising:
+        q = q.abs()
+        kp = (kp.abs() * torch.linspace(0, 24 / D ** 0.5, nb).view(-1, 1, 1, 1)).to(dtype)
+    bt = torch.randperm(nb, generator=g).view(1, nb).int()
+    kh, vh = (gather_ref(p, bt[0].tolist(), n).transpose(0, 1).double().repeat_interleave(Hq // Hk, 0) for p in (kp, vp))
+    s = q[0].double() @ kh.transpose(1, 2).contiguous() / math.sqrt(D)
+    s.masked_fill_(torch.arange(n) > torch.arange(Lq).unsqueeze(1) + n - Lq, -math.inf)
+    ref = torch.softmax(s, -1) @ vh
+    rel = lambda x: ((x.double() - ref).norm() / ref.norm()).item()  # noqa: E731
+    out = paged_prefill(q.to(DEV), kp.to(DEV), vp.to(DEV), bt.to(DEV), torch.tensor([n], dtype=torch.int32, device=DEV))
+    assert rel(out[0].cpu()) <= 1.05 * rel(ref.to(dtype))
