@@ -83,7 +83,12 @@ def _build_host() -> None:
     inc += [f"-isystem{d}" for d in include_paths()]
     libs = [x for d in library_paths() for x in (f"-L{d}", f"-Wl,-rpath,{d}")]
     tmp = HOST_PATH + ".tmp"
-    _run(["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+    # NDEBUG: without it the headers bring a thread-local counter, and a library
+    # with thread-local storage that no call touches keeps glibc's per-thread
+    # table out of date: every thread-local access of the process (each torch
+    # call makes some) then takes the slow lookup (torch.empty 1.07 -> 1.31 us,
+    # Tensor.view 0.58 -> 0.66)
+    _run(["g++", "-O2", "-DNDEBUG", "-std=c++17", "-fPIC", "-shared", "-Wall", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", *inc, os.path.join(CSRC, "host.cpp"),
           "-o", tmp, *libs, "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_python"])
     os.replace(tmp, HOST_PATH)

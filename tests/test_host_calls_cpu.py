@@ -4,6 +4,8 @@ Python functions (None), which refuse it with their own errors."""
 
 from __future__ import annotations
 
+import struct
+
 import pytest
 import torch
 
@@ -13,6 +15,17 @@ from engine.quant import int8_matmul
 
 def test_binds_exported_entry_points():
     assert set(_lib.host().names()) <= set(_lib.EXPORTED_SYMBOLS)
+
+
+def test_extension_has_no_thread_local_storage():
+    """A library loaded with thread-local storage that no call touches slows
+    every thread-local access of the process (see build_lib.py)."""
+    with open(_lib.HOST_PATH, "rb") as f:
+        elf = f.read()
+    phoff, = struct.unpack_from("<Q", elf, 32)
+    size, count = struct.unpack_from("<HH", elf, 54)
+    kinds = [struct.unpack_from("<I", elf, phoff + i * size)[0] for i in range(count)]
+    assert 1 in kinds and 7 not in kinds  # PT_LOAD, PT_TLS
 
 
 @pytest.mark.parametrize("name,n", [("flash", 9), ("paged", 12), ("section", 13), ("append", 12), ("append_seq", 6), ("gather", 4),
