@@ -18,6 +18,7 @@
 #include <ATen/ATen.h>
 #include <c10/core/DeviceGuard.h>
 #include <c10/hip/HIPStream.h>
+#include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 
 #include <cmath>
@@ -114,25 +115,17 @@ void* stream_of(const Tensor& t) { return c10::hip::getCurrentHIPStream(t.device
 
 Tensor bytes_like(size_t n, const Tensor& t) { return at::empty({(int64_t)n}, t.options().dtype(at::kByte)); }
 
-// Runs f without the GIL (as ctypes does), on the tensor's device; f returns a status.
+// Runs f without the GIL (as ctypes does); f returns a status.
 template <typename F>
-int launch(const Tensor& t, F&& f) {
-  int rc;
-  Py_BEGIN_ALLOW_THREADS;
-  rc = f();
-  Py_END_ALLOW_THREADS;
-  return rc;
+int launch(F&& f) {
+  struct Released {
+    PyThreadState* s = PyEval_SaveThread();
+    ~Released() { PyEval_RestoreThread(s); }
+  } released;
+  return f();
 }
 
 PyObject* result(int rc, const Tensor& out) { return rc ? PyLong_FromLong(rc) : THPVariable_Wrap(out); }
-
-#define CIE_PY_BEGIN try {
-#define CIE_PY_END                                    \
-  }                                                   \
-  catch (const std::exception& e) {                   \
-    PyErr_SetString(PyExc_RuntimeError, e.what());    \
-    return nullptr;                                   \
-  }
 
 bool number(PyObject* o, double* v) {
   *v = PyFloat_AsDouble(o);
@@ -143,7 +136,7 @@ bool number(PyObject* o, double* v) {
 
 // flash(q, k, v, causal, scale | None, cos | None, sin | None, q_pos0 | None, out | None)
 PyObject* flash(PyObject*, PyObject* const* a, Py_ssize_t n) {
-  CIE_PY_BEGIN
+  HANDLE_TH_ERRORS  // torch's own translation: an allocator failure is torch.OutOfMemoryError
   if (n != 9) Py_RETURN_NONE;
   const Tensor *q = tensor(a[0]), *k = tensor(a[1]), *v = tensor(a[2]);
   bool ok = q && k && v;
@@ -175,14 +168,14 @@ PyObject* flash(PyObject*, PyObject* const* a, Py_ssize_t n) {
   const Tensor ws = nbytes ? bytes_like(nbytes, *q) : Tensor();
   const Strides sq(*q), sk(*k), sv(*v), so(out);
   void* stream = stream_of(*q);
-  const int rc = launch(*q, [&] {
+  const int rc = launch([&] {
     return api.flash(q->data_ptr(), k->data_ptr(), v->data_ptr(), out.data_ptr(), sq.s, sk.s, sv.s, so.s, (int)B,
                      (int)H, (int)Hk, (int)M, (int)N, (int)D, (float)scale, causal, dt, rope.cos, rope.sin, rope.rows,
                      rope.dt, pos ? static_cast<const int32_t*>(pos->data_ptr()) : nullptr, 0,
                      nbytes ? ws.data_ptr() : nullptr, nbytes, stream);
   });
   return result(rc, out);
-  CIE_PY_END
+  END_HANDLE_TH_ERRORS
 }
 
 // A launch over one layer's pools; the tables are int32 and contiguous.
@@ -246,7 +239,7 @@ int paged_launch(const Tensor& q, const Pools& P, const Tensor& out, const Rope&
   void* const wp = nbytes ? ws.data_ptr() : nullptr;
   void* stream = stream_of(q);
   const int32_t *bt = static_cast<const int32_t*>(P.bt->data_ptr()), *lens = static_cast<const int32_t*>(P.lens->data_ptr());
-  return launch(q, [&] {
+  return launch([&] {
     if (prefill)
       return api.flash_paged(q.data_ptr(), P.kc->data_ptr(), P.vc->data_ptr(), bt, lens, out.data_ptr(), sq.s, sk.s,
                              sv.s, so.s, B, Hq, Hk, Lq, D, nb, bs, w, m, (float)scale, causal, dt, rope.cos, rope.sin,
@@ -261,7 +254,7 @@ int paged_launch(const Tensor& q, const Pools& P, const Tensor& out, const Rope&
 
 // paged(prefill, q, k_cache, v_cache, block_tables, context_lens, causal, scale | None, max_context, cos, sin, out | None)
 PyObject* paged(PyObject*, PyObject* const* a, Py_ssize_t n) {
-  CIE_PY_BEGIN
+  HANDLE_TH_ERRORS
   if (n != 12) Py_RETURN_NONE;
   const bool prefill = a[0] == Py_True;
   const Tensor* q = tensor(a[1]);
@@ -289,14 +282,14 @@ PyObject* paged(PyObject*, PyObject* const* a, Py_ssize_t n) {
   const int64_t none3[3] = {0, 0, 1};
   const Plan no_plan(Py_None, Py_None, Py_None, {}, *q);
   return result(paged_launch(*q, P, out, rope, no_plan, mc, scale, causal, nullptr, nullptr, none3, none3, prefill), out);
-  CIE_PY_END
+  END_HANDLE_TH_ERRORS
 }
 
 // One layer's fused decode / verify section:
 // section(q, k, v, k_cache, v_cache, block_tables, context_lens, max_context, cos, sin, plan data | None, split, key)
 // with q (B, Hq, L, D), k / v (B, Hk, L, D); returns (B, L, Hq * D).
 PyObject* section(PyObject*, PyObject* const* a, Py_ssize_t n) {
-  CIE_PY_BEGIN
+  HANDLE_TH_ERRORS
   if (n != 13) Py_RETURN_NONE;
   const Tensor *q = tensor(a[0]), *k = tensor(a[1]), *v = tensor(a[2]);
   if (!q || !k || !v || !on_gpu(*q) || !on_gpu(*k) || !on_gpu(*v) || q->dim() != 4 || k->dim() != 4 ||
@@ -329,13 +322,13 @@ PyObject* section(PyObject*, PyObject* const* a, Py_ssize_t n) {
   const int rc = paged_launch(*q, P, out, rope, plan, mc, 1.0 / std::sqrt((double)D), 1, k->data_ptr(), v->data_ptr(),
                               st[0], st[1], false);
   return result(rc, rows.view({B, L, Hq * D}));
-  CIE_PY_END
+  END_HANDLE_TH_ERRORS
 }
 
 // append(k_new, v_new, k_cache, v_cache, block_tables, cu_new, start, max_new, status | None, cos, sin, k_out | None);
 // returns True when done.
 PyObject* append(PyObject*, PyObject* const* a, Py_ssize_t n) {
-  CIE_PY_BEGIN
+  HANDLE_TH_ERRORS
   if (n != 12) Py_RETURN_NONE;
   const Tensor *k = tensor(a[0]), *v = tensor(a[1]), *cu = tensor(a[5]);
   bool ok = k && v && cu;
@@ -363,7 +356,7 @@ PyObject* append(PyObject*, PyObject* const* a, Py_ssize_t n) {
   void* stream = stream_of(*k);
   const auto ip = [](const Tensor* t) { return static_cast<const int32_t*>(t->data_ptr()); };
   const int dt = dtype_code(*k);
-  const int rc = launch(*k, [&] {
+  const int rc = launch([&] {
     if (!rope.cos)
       return api.append(k->data_ptr(), v->data_ptr(), P.kc->data_ptr(), P.vc->data_ptr(), sn.s, sm.s, sk.s, sv.s,
                         ip(P.bt), ip(cu), ip(P.lens), nullptr, (int)B, (int)T, (int)max_new, (int)Hk, (int)D,
@@ -375,7 +368,7 @@ PyObject* append(PyObject*, PyObject* const* a, Py_ssize_t n) {
   });
   if (rc) return PyLong_FromLong(rc);
   Py_RETURN_TRUE;
-  CIE_PY_END
+  END_HANDLE_TH_ERRORS
 }
 
 // Block ids of a BlockTable's list.
@@ -423,7 +416,7 @@ struct SeqPools {
 // append_seq(k_new, v_new, k_cache, v_cache, blocks, start): (L, heads, D) rows
 // to positions start ..; True when done.
 PyObject* append_seq(PyObject*, PyObject* const* a, Py_ssize_t n) {
-  CIE_PY_BEGIN
+  HANDLE_TH_ERRORS
   if (n != 6) Py_RETURN_NONE;
   const Tensor *k = tensor(a[0]), *v = tensor(a[1]), *kc = tensor(a[2]), *vc = tensor(a[3]);
   std::vector<int32_t> ids;
@@ -445,19 +438,19 @@ PyObject* append_seq(PyObject*, PyObject* const* a, Py_ssize_t n) {
   const int64_t dense[4] = {2 * sk.s[0], 2 * sk.s[1], 2 * sv.s[0], 2 * sv.s[1]};
   const c10::OptionalDeviceGuard guard(k->device());
   void* stream = stream_of(*k);
-  const int rc = launch(*k, [&] {
+  const int rc = launch([&] {
     return api.append_seq(k->data_ptr(), v->data_ptr(), kc->data_ptr(), vc->data_ptr(), dense, P.strides, ids.data(),
                           (int)ids.size(), start, L, (int)kc->size(2), P.head_bytes, (int)kc->size(0),
                           (int)kc->size(1), stream);
   });
   if (rc) return PyLong_FromLong(rc);
   Py_RETURN_TRUE;
-  CIE_PY_END
+  END_HANDLE_TH_ERRORS
 }
 
 // gather(k_cache, v_cache, blocks, L): dense (L, heads, D) copies of both
 PyObject* gather(PyObject*, PyObject* const* a, Py_ssize_t n) {
-  CIE_PY_BEGIN
+  HANDLE_TH_ERRORS
   if (n != 4) Py_RETURN_NONE;
   const Tensor *kc = tensor(a[0]), *vc = tensor(a[1]);
   std::vector<int32_t> ids;
@@ -473,19 +466,19 @@ PyObject* gather(PyObject*, PyObject* const* a, Py_ssize_t n) {
   const Tensor k = at::empty({L, heads, kc->size(3)}, kc->options()), v = at::empty_like(k);
   const int64_t dense[4] = {heads * P.head_bytes, P.head_bytes, heads * P.head_bytes, P.head_bytes};
   void* stream = stream_of(*kc);
-  const int rc = launch(*kc, [&] {
+  const int rc = launch([&] {
     return api.gather(kc->data_ptr(), vc->data_ptr(), k.data_ptr(), v.data_ptr(), dense, P.strides, ids.data(),
                       (int)ids.size(), L, (int)heads, P.head_bytes, (int)kc->size(0), (int)kc->size(1), stream);
   });
   if (rc) return PyLong_FromLong(rc);
   PyObject *pk = THPVariable_Wrap(k), *pv = THPVariable_Wrap(v);
   return pk && pv ? Py_BuildValue("(NN)", pk, pv) : nullptr;
-  CIE_PY_END
+  END_HANDLE_TH_ERRORS
 }
 
 // int8(x, w_int8, scales, bias | None)
 PyObject* int8(PyObject*, PyObject* const* a, Py_ssize_t n) {
-  CIE_PY_BEGIN
+  HANDLE_TH_ERRORS
   if (n != 4) Py_RETURN_NONE;
   const Tensor *x = tensor(a[0]), *w = tensor(a[1]), *s = tensor(a[2]);
   bool ok = x && w && s;
@@ -517,13 +510,13 @@ PyObject* int8(PyObject*, PyObject* const* a, Py_ssize_t n) {
   const size_t nbytes = api.int8_ws((int)M, (int)N, (int)K);
   const Tensor ws = nbytes ? bytes_like(nbytes, *x) : Tensor();
   void* stream = stream_of(*x);
-  const int rc = launch(*x, [&] {
+  const int rc = launch([&] {
     return api.int8(x->data_ptr(), static_cast<const int8_t*>(w->data_ptr()), s->data_ptr(), b ? b->data_ptr() : nullptr, y.data_ptr(), xs,
                     w->stride(0), N, (int)M, (int)N, (int)K, dtype_code(*x), any_code(*s),
                     nbytes ? ws.data_ptr() : nullptr, nbytes, stream);
   });
   return result(rc, y);
-  CIE_PY_END
+  END_HANDLE_TH_ERRORS
 }
 
 // bind({name: address}): the library's entry points.

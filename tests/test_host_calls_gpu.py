@@ -23,6 +23,12 @@ pytestmark = pytest.mark.gpu
 DEV = "cuda"
 
 
+def _python_only(m):
+    back = types.SimpleNamespace(**{n: (lambda *args: None) for n in ("flash", "paged", "section", "append", "append_seq",
+                                                                   "gather", "int8")})
+    m.setattr(_lib, "host", lambda: back)
+
+
 def _both(monkeypatch, call):
     """call() through the extension and through Python alone: the same tensors,
     or the same refusal (an append of rows with odd strides)."""
@@ -34,10 +40,8 @@ def _both(monkeypatch, call):
             return str(e)
 
     a = outcome()
-    back = types.SimpleNamespace(**{n: (lambda *args: None) for n in ("flash", "paged", "section", "append", "append_seq",
-                                                                   "gather", "int8")})
     with monkeypatch.context() as m:
-        m.setattr(_lib, "host", lambda: back)
+        _python_only(m)
         b = outcome()
     assert type(a) is type(b)
     if isinstance(a, str):
@@ -184,3 +188,57 @@ def test_gather_of_other_caches(monkeypatch):
         assert cache.gather(0, t)[0].shape == (0, 2, D)
         t.blocks, t.length = [5, 0, 3], 10
         _both(monkeypatch, lambda: cache.gather(0, t))
+
+
+@pytest.fixture
+def no_memory():
+    """Nothing over 20 MB can be allocated while it is entered (the caching
+    allocator's own limit: the driver is never asked)."""
+    import contextlib
+
+    @contextlib.contextmanager
+    def limit():
+        torch.cuda.synchronize()
+        torch.cuda.empty_cache()
+        total = torch.cuda.get_device_properties(0).total_memory
+        torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + 1024) / total)
+        try:
+            yield
+        finally:
+            torch.cuda.set_per_process_memory_fraction(1.0)
+
+    return limit
+
+
+@pytest.mark.parametrize("path", ["compiled", "python"])
+def test_out_of_memory_is_torch_out_of_memory(monkeypatch, no_memory, path):
+    """A result that does not fit raises torch.OutOfMemoryError on both paths
+    (what a serving loop catches to preempt a sequence), and the next call
+    that fits works."""
+    f16 = torch.float16
+    z = torch.zeros(1, 1, 1, 64, dtype=f16, device=DEV)
+    q = z.expand(64, 64, 128, 64)
+    kp = torch.zeros(2048, 16, 64, 64, dtype=f16, device=DEV)
+    bt, lens = torch.zeros(64, 16, dtype=torch.int32, device=DEV), torch.full((64,), 200, dtype=torch.int32, device=DEV)
+    cache = PagedKVCache(KVCacheConfig(1, 8, 256, 1024, 16, f16, DEV))
+    tables = [cache.new_sequence() for _ in range(64)]
+    for t in tables:
+        t.length = 100
+    step = cache.prepare_step(tables, 32, num_heads=32)
+    qs, ks = (torch.zeros(1, 1, 1, 256, dtype=f16, device=DEV).expand(64, h, 32, 256) for h in (32, 8))
+    ks = ks.contiguous()
+    one = cache.new_sequence()
+    one.blocks, one.length = list(range(1000)), 16000
+    x, w, s = (torch.zeros(16384, 16, dtype=f16, device=DEV), torch.zeros(2048, 16, dtype=torch.int8, device=DEV),
+               torch.zeros(2048, dtype=f16, device=DEV))
+    calls = {"flash": lambda: flash_attention(q, q, q), "paged": lambda: paged_attention(q, kp, kp, bt, lens),
+             "prefill": lambda: paged_prefill(q, kp, kp, bt, lens),
+             "section": lambda: attention_section(qs, ks, ks, 0, cache, step),
+             "gather": lambda: cache.gather(0, one), "int8": lambda: int8_matmul(x, w, s)}
+    with monkeypatch.context() as m:
+        if path == "python":
+            _python_only(m)
+        for name, call in calls.items():
+            with no_memory(), pytest.raises(torch.OutOfMemoryError):
+                call()
+            assert call() is not None, name
