@@ -5,17 +5,21 @@
 // and device context took 17-24 us of host time per operation, more than most
 // of the kernels it launches; here it takes 4-7.
 //
-// Every function handles the arguments a kernel can take as they are (exact
-// tensors on one GPU, supported dtypes and shapes, rows the kernels can read in
-// place) and returns None for everything else, before any side effect: the
-// Python function then copies, converts or raises as the case needs. A
-// non-zero status of the library comes back as an int.
+// Every function handles exact tensors on one GPU of supported dtypes and
+// shapes, making the copies the Python functions make where a kernel cannot
+// read an operand in place (misaligned rows, int64 tables, a bias of another
+// type: handing those back cost the refused call on top of the Python path,
+// Int8Linear of a bf16 model with its fp16 bias 18.9 -> 20.9 us at 16 x 4096 x
+// 4096). It returns None for everything else, before any side effect: the
+// Python function then raises or converts as the case needs. A non-zero status
+// of the library comes back as an int.
 //
 // The library's functions are bound by address (bind), so the extension works
 // with whichever build of the library the package loaded.
 #include <Python.h>
 
 #include <ATen/ATen.h>
+#include <ATen/core/grad_mode.h>
 #include <c10/core/DeviceGuard.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/Exceptions.h>
@@ -80,6 +84,19 @@ bool kernel_layout(const Tensor& t) {
     if (t.size(i) != 1 && (t.stride(i) % 8 || t.stride(i) < 0)) return false;
   return true;
 }
+
+// t, or a contiguous copy when the kernels cannot read it in place.
+Tensor laid_out(const Tensor& t) { return kernel_layout(t) ? t : t.clone(at::MemoryFormat::Contiguous); }
+
+// Block tables, lengths and the like: int32 or int64 on the device of `like`,
+// converted where the kernels need it.
+bool index_ok(const Tensor* t, const Tensor& like) {
+  return t && on_gpu(*t) && t->device() == like.device() && (t->scalar_type() == at::kInt || t->scalar_type() == at::kLong);
+}
+Tensor index32(const Tensor& t) {
+  return t.scalar_type() == at::kInt && t.is_contiguous() ? t : t.to(at::kInt).contiguous();
+}
+const int32_t* ip(const Tensor& t) { return static_cast<const int32_t*>(t.data_ptr()); }
 
 struct Strides {
   int64_t s[4];
@@ -147,8 +164,7 @@ PyObject* flash(PyObject*, PyObject* const* a, Py_ssize_t n) {
   const int64_t B = q->size(0), H = q->size(1), M = q->size(2), D = q->size(3), Hk = k->size(1), N = k->size(2);
   if (dt < 0 || k->scalar_type() != q->scalar_type() || v->scalar_type() != q->scalar_type() ||
       k->device() != q->device() || v->device() != q->device() || !head_dim_ok(D) || v->sizes() != k->sizes() ||
-      k->size(0) != B || k->size(3) != D || Hk < 1 || H % Hk || !fits(B) || !fits(H) || !fits(M) || !fits(N) ||
-      !kernel_layout(*q) || !kernel_layout(*k) || !kernel_layout(*v))
+      k->size(0) != B || k->size(3) != D || Hk < 1 || H % Hk || !fits(B) || !fits(H) || !fits(M) || !fits(N))
     Py_RETURN_NONE;
   if (o && (!on_gpu(*o) || o->sizes() != q->sizes() || o->scalar_type() != q->scalar_type() ||
             o->device() != q->device() || !kernel_layout(*o)))
@@ -166,10 +182,11 @@ PyObject* flash(PyObject*, PyObject* const* a, Py_ssize_t n) {
   const Tensor out = o ? *o : at::empty({B, H, M, D}, q->options());
   const size_t nbytes = api.flash_ws((int)B, (int)H, (int)Hk, (int)M, (int)N, (int)D, causal, 0);
   const Tensor ws = nbytes ? bytes_like(nbytes, *q) : Tensor();
-  const Strides sq(*q), sk(*k), sv(*v), so(out);
+  const Tensor qc = laid_out(*q), kc = laid_out(*k), vc = laid_out(*v);
+  const Strides sq(qc), sk(kc), sv(vc), so(out);
   void* stream = stream_of(*q);
   const int rc = launch([&] {
-    return api.flash(q->data_ptr(), k->data_ptr(), v->data_ptr(), out.data_ptr(), sq.s, sk.s, sv.s, so.s, (int)B,
+    return api.flash(qc.data_ptr(), kc.data_ptr(), vc.data_ptr(), out.data_ptr(), sq.s, sk.s, sv.s, so.s, (int)B,
                      (int)H, (int)Hk, (int)M, (int)N, (int)D, (float)scale, causal, dt, rope.cos, rope.sin, rope.rows,
                      rope.dt, pos ? static_cast<const int32_t*>(pos->data_ptr()) : nullptr, 0,
                      nbytes ? ws.data_ptr() : nullptr, nbytes, stream);
@@ -178,9 +195,9 @@ PyObject* flash(PyObject*, PyObject* const* a, Py_ssize_t n) {
   END_HANDLE_TH_ERRORS
 }
 
-// A launch over one layer's pools; the tables are int32 and contiguous.
+// A launch over one layer's pools.
 struct Pools {
-  const Tensor *kc, *vc, *bt, *lens;
+  const Tensor *kc, *vc, *bt, *lens;  // block table and lengths as given; index32() of them for a kernel
   int64_t num_blocks = 0, block_size = 0, Hk = 0, width = 0;
   bool ok;
   Pools(PyObject* k, PyObject* v, PyObject* t, PyObject* l, const Tensor& like, int64_t B, int64_t D)
@@ -190,8 +207,7 @@ struct Pools {
     for (const Tensor* x : {kc, vc})
       ok = ok && on_gpu(*x) && x->device() == like.device() && x->dim() == 4 && x->scalar_type() == like.scalar_type() &&
            x->size(3) == D && kernel_layout(*x);
-    for (const Tensor* x : {bt, lens})
-      ok = ok && on_gpu(*x) && x->device() == like.device() && x->scalar_type() == at::kInt && x->is_contiguous();
+    for (const Tensor* x : {bt, lens}) ok = ok && index_ok(x, like);
     ok = ok && kc->sizes() == vc->sizes() && bt->dim() == 2 && bt->size(0) == B && lens->dim() == 1 && lens->size(0) == B;
     if (!ok) return;
     num_blocks = kc->size(0), block_size = kc->size(1), Hk = kc->size(2), width = bt->size(1);
@@ -238,14 +254,15 @@ int paged_launch(const Tensor& q, const Pools& P, const Tensor& out, const Rope&
   const Strides sq(q), sk(*P.kc), sv(*P.vc), so(out);
   void* const wp = nbytes ? ws.data_ptr() : nullptr;
   void* stream = stream_of(q);
-  const int32_t *bt = static_cast<const int32_t*>(P.bt->data_ptr()), *lens = static_cast<const int32_t*>(P.lens->data_ptr());
+  // (a plan carries both)
+  const Tensor bt_c = plan.data ? Tensor() : index32(*P.bt), lens_c = plan.data ? Tensor() : index32(*P.lens);
+  const int32_t *bt = plan.data ? nullptr : ip(bt_c), *lens = plan.data ? nullptr : ip(lens_c);
   return launch([&] {
     if (prefill)
       return api.flash_paged(q.data_ptr(), P.kc->data_ptr(), P.vc->data_ptr(), bt, lens, out.data_ptr(), sq.s, sk.s,
                              sv.s, so.s, B, Hq, Hk, Lq, D, nb, bs, w, m, (float)scale, causal, dt, rope.cos, rope.sin,
                              rope.rows, rope.dt, 0, wp, nbytes, stream);
-    return api.paged(q.data_ptr(), kn, vn, P.kc->data_ptr(), P.vc->data_ptr(), plan.data ? nullptr : bt,
-                     plan.data ? nullptr : lens, plan.data ? plan.data->data_ptr() : nullptr,
+    return api.paged(q.data_ptr(), kn, vn, P.kc->data_ptr(), P.vc->data_ptr(), bt, lens, plan.data ? plan.data->data_ptr() : nullptr,
                      plan.data ? (size_t)plan.data->nbytes() : 0, plan.split, out.data_ptr(), wp, nbytes, sq.s, kns, vns,
                      sk.s, sv.s, so.s, B, Hq, Hk, Lq, D, nb, bs, w, m, (float)scale, causal, dt, rope.cos, rope.sin,
                      rope.rows, rope.dt, stream);
@@ -260,8 +277,7 @@ PyObject* paged(PyObject*, PyObject* const* a, Py_ssize_t n) {
   const Tensor* q = tensor(a[1]);
   bool ok = q != nullptr;
   const Tensor* o = tensor_or_none(a[11], &ok);
-  if (!ok || !on_gpu(*q) || q->dim() != 4 || dtype_code(*q) < 0 || !head_dim_ok(q->size(3)) || !kernel_layout(*q))
-    Py_RETURN_NONE;
+  if (!ok || !on_gpu(*q) || q->dim() != 4 || dtype_code(*q) < 0 || !head_dim_ok(q->size(3))) Py_RETURN_NONE;
   const int64_t B = q->size(0), Hq = q->size(1), Lq = q->size(2), D = q->size(3);
   const Pools P(a[2], a[3], a[4], a[5], *q, B, D);
   const int64_t mc = PyLong_Check(a[8]) ? PyLong_AsLongLong(a[8]) : -1;
@@ -281,7 +297,7 @@ PyObject* paged(PyObject*, PyObject* const* a, Py_ssize_t n) {
   const Tensor out = o ? *o : at::empty({B, Hq, Lq, D}, q->options());
   const int64_t none3[3] = {0, 0, 1};
   const Plan no_plan(Py_None, Py_None, Py_None, {}, *q);
-  return result(paged_launch(*q, P, out, rope, no_plan, mc, scale, causal, nullptr, nullptr, none3, none3, prefill), out);
+  return result(paged_launch(laid_out(*q), P, out, rope, no_plan, mc, scale, causal, nullptr, nullptr, none3, none3, prefill), out);
   END_HANDLE_TH_ERRORS
 }
 
@@ -293,8 +309,7 @@ PyObject* section(PyObject*, PyObject* const* a, Py_ssize_t n) {
   if (n != 13) Py_RETURN_NONE;
   const Tensor *q = tensor(a[0]), *k = tensor(a[1]), *v = tensor(a[2]);
   if (!q || !k || !v || !on_gpu(*q) || !on_gpu(*k) || !on_gpu(*v) || q->dim() != 4 || k->dim() != 4 ||
-      v->sizes() != k->sizes() || dtype_code(*q) < 0 || !head_dim_ok(q->size(3)) || !kernel_layout(*q) ||
-      !kernel_layout(*k) || !kernel_layout(*v))
+      v->sizes() != k->sizes() || dtype_code(*q) < 0 || !head_dim_ok(q->size(3)))
     Py_RETURN_NONE;
   const int64_t B = q->size(0), Hq = q->size(1), L = q->size(2), D = q->size(3);
   const Pools P(a[3], a[4], a[5], a[6], *q, B, D);
@@ -303,24 +318,29 @@ PyObject* section(PyObject*, PyObject* const* a, Py_ssize_t n) {
     PyErr_Clear();
     Py_RETURN_NONE;
   }
-  int64_t st[2][3];  // token row b * L + i of k / v: one stride over all of them
-  for (int x = 0; x < 2; ++x) {
-    const Tensor& t = x ? *v : *k;
-    if (t.size(0) != B || t.size(1) != P.Hk || t.size(2) != L || t.size(3) != D || t.scalar_type() != q->scalar_type() ||
-        t.device() != q->device() || (B > 1 && L > 1 && t.stride(0) != L * t.stride(2)))
+  for (const Tensor* t : {k, v})
+    if (t->size(0) != B || t->size(1) != P.Hk || t->size(2) != L || t->size(3) != D ||
+        t->scalar_type() != q->scalar_type() || t->device() != q->device())
       Py_RETURN_NONE;
-    st[x][0] = L > 1 ? t.stride(2) : B > 1 ? t.stride(0) : 0;
-    st[x][1] = P.Hk > 1 ? t.stride(1) : 0;
-    st[x][2] = 1;
-  }
   const Rope rope(a[8], a[9], D, *q);
   const Plan plan(a[10], a[11], a[12], {B, Hq, P.Hk, L, D, P.num_blocks, P.block_size, P.width, mc, 1}, *q);
   if (!rope.ok || !plan.ok) Py_RETURN_NONE;
   const c10::OptionalDeviceGuard guard(q->device());
+  Tensor kv[2];
+  int64_t st[2][3];  // token row b * L + i of k / v: one stride over all of them, else copied
+  for (int x = 0; x < 2; ++x) {
+    Tensor& t = kv[x];
+    t = x ? *v : *k;
+    if (!kernel_layout(t) || (B > 1 && L > 1 && t.stride(0) != L * t.stride(2)))
+      t = t.transpose(1, 2).clone(at::MemoryFormat::Contiguous).transpose(1, 2);
+    st[x][0] = L > 1 ? t.stride(2) : B > 1 ? t.stride(0) : 0;
+    st[x][1] = P.Hk > 1 ? t.stride(1) : 0;
+    st[x][2] = 1;
+  }
   const Tensor rows = at::empty({B, L, Hq, D}, q->options());
   const Tensor out = rows.transpose(1, 2);
-  const int rc = paged_launch(*q, P, out, rope, plan, mc, 1.0 / std::sqrt((double)D), 1, k->data_ptr(), v->data_ptr(),
-                              st[0], st[1], false);
+  const int rc = paged_launch(laid_out(*q), P, out, rope, plan, mc, 1.0 / std::sqrt((double)D), 1, kv[0].data_ptr(),
+                              kv[1].data_ptr(), st[0], st[1], false);
   return result(rc, rows.view({B, L, Hq * D}));
   END_HANDLE_TH_ERRORS
 }
@@ -334,7 +354,7 @@ PyObject* append(PyObject*, PyObject* const* a, Py_ssize_t n) {
   bool ok = k && v && cu;
   const Tensor* status = tensor_or_none(a[8], &ok);
   const Tensor* ko = tensor_or_none(a[11], &ok);
-  if (!ok || status || !on_gpu(*k) || !on_gpu(*v) || k->dim() != 3 || v->sizes() != k->sizes() || dtype_code(*k) < 0 ||
+  if (!ok || !on_gpu(*k) || !on_gpu(*v) || k->dim() != 3 || v->sizes() != k->sizes() || dtype_code(*k) < 0 ||
       v->scalar_type() != k->scalar_type() || v->device() != k->device() || !kernel_layout(*k) || !kernel_layout(*v))
     Py_RETURN_NONE;
   const int64_t Hk = k->size(1), D = k->size(2), max_new = PyLong_Check(a[7]) ? PyLong_AsLongLong(a[7]) : -1;
@@ -345,8 +365,9 @@ PyObject* append(PyObject*, PyObject* const* a, Py_ssize_t n) {
   const int64_t B = cu->size(0) - 1, T = k->size(0);
   const Pools P(a[2], a[3], a[4], a[6], *k, B, D);
   const Rope rope(a[9], a[10], D, *k);
-  if (!P.ok || P.Hk != Hk || !fits(B) || !fits(T) || !rope.ok || !on_gpu(*cu) || cu->device() != k->device() ||
-      cu->scalar_type() != at::kInt || !cu->is_contiguous())
+  if (!P.ok || P.Hk != Hk || !fits(B) || !fits(T) || !rope.ok || !index_ok(cu, *k)) Py_RETURN_NONE;
+  if (status && (!on_gpu(*status) || status->device() != k->device() || status->numel() < 1 ||
+                 (status->scalar_type() != at::kInt && status->scalar_type() != at::kUInt32)))
     Py_RETURN_NONE;
   if (ko && (!rope.cos || !on_gpu(*ko) || ko->sizes() != k->sizes() || ko->scalar_type() != k->scalar_type() ||
              ko->device() != k->device() || !kernel_layout(*ko)))
@@ -354,15 +375,16 @@ PyObject* append(PyObject*, PyObject* const* a, Py_ssize_t n) {
   const c10::OptionalDeviceGuard guard(k->device());
   const Strides sn(*k), sm(*v), sk(*P.kc), sv(*P.vc), so(ko ? *ko : *k);
   void* stream = stream_of(*k);
-  const auto ip = [](const Tensor* t) { return static_cast<const int32_t*>(t->data_ptr()); };
+  const Tensor bt = index32(*P.bt), cu_new = index32(*cu), start = index32(*P.lens);
+  uint32_t* const sp = status ? static_cast<uint32_t*>(status->data_ptr()) : nullptr;
   const int dt = dtype_code(*k);
   const int rc = launch([&] {
     if (!rope.cos)
       return api.append(k->data_ptr(), v->data_ptr(), P.kc->data_ptr(), P.vc->data_ptr(), sn.s, sm.s, sk.s, sv.s,
-                        ip(P.bt), ip(cu), ip(P.lens), nullptr, (int)B, (int)T, (int)max_new, (int)Hk, (int)D,
+                        ip(bt), ip(cu_new), ip(start), sp, (int)B, (int)T, (int)max_new, (int)Hk, (int)D,
                         (int)P.num_blocks, (int)P.block_size, (int)P.width, dt, stream);
     return api.append_rope(k->data_ptr(), v->data_ptr(), P.kc->data_ptr(), P.vc->data_ptr(), sn.s, sm.s, sk.s, sv.s,
-                           ip(P.bt), ip(cu), ip(P.lens), nullptr, (int)B, (int)T, (int)max_new, (int)Hk, (int)D,
+                           ip(bt), ip(cu_new), ip(start), sp, (int)B, (int)T, (int)max_new, (int)Hk, (int)D,
                            (int)P.num_blocks, (int)P.block_size, (int)P.width, dt, rope.cos, rope.sin, rope.rows,
                            rope.dt, ko ? ko->data_ptr() : nullptr, ko ? so.s : nullptr, stream);
   });
@@ -419,16 +441,17 @@ PyObject* append_seq(PyObject*, PyObject* const* a, Py_ssize_t n) {
   HANDLE_TH_ERRORS
   if (n != 6) Py_RETURN_NONE;
   const Tensor *k = tensor(a[0]), *v = tensor(a[1]), *kc = tensor(a[2]), *vc = tensor(a[3]);
-  std::vector<int32_t> ids;
   // (the engine's 16-bit caches only, as the append through device tables)
   if (!k || !v || !on_gpu(*k) || !on_gpu(*v) || k->dim() != 3 || v->sizes() != k->sizes() || dtype_code(*k) < 0 ||
-      k->size(0) < 1 || !id_list(a[4], &ids) || !PyLong_Check(a[5]))
+      k->size(0) < 1 || !PyLong_Check(a[5]))
     Py_RETURN_NONE;
   const SeqPools P(kc, vc);
   if (!P.ok || !head_dim_ok(k->size(2)) || kc->size(2) != k->size(1) || kc->size(3) != k->size(2) ||
       kc->device() != k->device() || v->device() != k->device() || kc->scalar_type() != k->scalar_type() ||
       v->scalar_type() != k->scalar_type() || !kernel_layout(*k) || !kernel_layout(*v))
     Py_RETURN_NONE;
+  std::vector<int32_t> ids;
+  if (!id_list(a[4], &ids)) Py_RETURN_NONE;
   const int64_t start = PyLong_AsLongLong(a[5]), L = k->size(0);
   if (PyErr_Occurred() || start < 0 || start + L > (int64_t)ids.size() * kc->size(1)) {
     PyErr_Clear();
@@ -453,11 +476,11 @@ PyObject* gather(PyObject*, PyObject* const* a, Py_ssize_t n) {
   HANDLE_TH_ERRORS
   if (n != 4) Py_RETURN_NONE;
   const Tensor *kc = tensor(a[0]), *vc = tensor(a[1]);
-  std::vector<int32_t> ids;
-  if (!kc || !vc || !id_list(a[2], &ids) || !PyLong_Check(a[3])) Py_RETURN_NONE;
   const SeqPools P(kc, vc);
+  std::vector<int32_t> ids;
+  if (!P.ok || !PyLong_Check(a[3]) || !id_list(a[2], &ids)) Py_RETURN_NONE;
   const int64_t L = PyLong_AsLongLong(a[3]);
-  if (!P.ok || PyErr_Occurred() || L < 1 || !fits(L) || L > (int64_t)ids.size() * kc->size(1)) {
+  if ( PyErr_Occurred() || L < 1 || !fits(L) || L > (int64_t)ids.size() * kc->size(1)) {
     PyErr_Clear();
     Py_RETURN_NONE;
   }
@@ -476,6 +499,17 @@ PyObject* gather(PyObject*, PyObject* const* a, Py_ssize_t n) {
   END_HANDLE_TH_ERRORS
 }
 
+// t (rows, K) itself when its rows start 16-byte aligned (a row stride of a
+// multiple of `elems` elements), else a copy with padded rows.
+Tensor aligned_rows(const Tensor& t, int64_t elems) {
+  const int64_t K = t.size(1);
+  if (t.stride(1) == 1 && t.stride(0) % elems == 0 && t.stride(0) >= K && !(reinterpret_cast<uintptr_t>(t.data_ptr()) & 15))
+    return t;
+  const Tensor rows = at::empty({t.size(0), (K + elems - 1) / elems * elems}, t.options()).narrow(1, 0, K);
+  rows.copy_(t);
+  return rows;
+}
+
 // int8(x, w_int8, scales, bias | None)
 PyObject* int8(PyObject*, PyObject* const* a, Py_ssize_t n) {
   HANDLE_TH_ERRORS
@@ -484,26 +518,21 @@ PyObject* int8(PyObject*, PyObject* const* a, Py_ssize_t n) {
   bool ok = x && w && s;
   const Tensor* b = tensor_or_none(a[3], &ok);
   if (!ok || !on_gpu(*x) || !on_gpu(*w) || !on_gpu(*s) || x->dim() < 1 || w->dim() != 2 || s->dim() != 1 ||
-      w->scalar_type() != at::kChar || dtype_code(*x) < 0 || any_code(*s) < 0 || w->device() != x->device() ||
-      s->device() != x->device())
+      w->scalar_type() != at::kChar || dtype_code(*x) < 0 || w->device() != x->device() || s->device() != x->device() ||
+      (any_code(*s) < 0 && s->scalar_type() != at::kDouble))
     Py_RETURN_NONE;
   const int64_t N = w->size(0), K = w->size(1);
-  const auto aligned = [](const Tensor& t) { return !(reinterpret_cast<uintptr_t>(t.data_ptr()) & 15); };
-  if (K < 1 || x->size(-1) != K || s->size(0) != N || !s->is_contiguous() || !aligned(*x) || !aligned(*w) ||
-      w->stride(1) != 1 || w->stride(0) % 16 || w->stride(0) < K || !fits(N) || !fits(K))
+  if (K < 1 || N < 1 || x->size(-1) != K || x->numel() < 1 || s->size(0) != N || !fits(N) || !fits(K) ||
+      !fits(x->numel() / K))
     Py_RETURN_NONE;
-  if (b && (!on_gpu(*b) || b->dim() != 1 || b->size(0) != N || b->device() != x->device() ||
-            b->scalar_type() != x->scalar_type() || !b->is_contiguous()))
+  if (b && (!on_gpu(*b) || b->dim() != 1 || b->size(0) != N || b->device() != x->device() || any_code(*b) < 0))
     Py_RETURN_NONE;
-  // rows of x: K apart when contiguous, or any 16-byte aligned stride of a matrix
-  int64_t xs = K;
-  if (!x->is_contiguous()) {
-    if (x->dim() != 2 || x->stride(1) != 1 || x->stride(0) < K) Py_RETURN_NONE;
-    xs = x->stride(0);
-  }
-  const int64_t M = x->numel() / K;
-  if (xs % 8 || M < 1 || N < 1 || !fits(M)) Py_RETURN_NONE;
   const c10::OptionalDeviceGuard guard(x->device());
+  const at::NoGradGuard no_grad;  // (the copies of a Parameter need no graph)
+  const Tensor xr = aligned_rows(x->dim() == 2 ? *x : x->reshape({-1, K}), 8), wr = aligned_rows(*w, 16);
+  const Tensor sr = (any_code(*s) < 0 ? s->to(at::kFloat) : *s).contiguous();
+  const Tensor br = b ? b->to(x->scalar_type()).contiguous() : Tensor();
+  const int64_t M = xr.size(0);
   at::DimVector shape(x->sizes().begin(), x->sizes().end());
   shape.back() = N;
   const Tensor y = at::empty(shape, x->options());
@@ -511,8 +540,8 @@ PyObject* int8(PyObject*, PyObject* const* a, Py_ssize_t n) {
   const Tensor ws = nbytes ? bytes_like(nbytes, *x) : Tensor();
   void* stream = stream_of(*x);
   const int rc = launch([&] {
-    return api.int8(x->data_ptr(), static_cast<const int8_t*>(w->data_ptr()), s->data_ptr(), b ? b->data_ptr() : nullptr, y.data_ptr(), xs,
-                    w->stride(0), N, (int)M, (int)N, (int)K, dtype_code(*x), any_code(*s),
+    return api.int8(xr.data_ptr(), static_cast<const int8_t*>(wr.data_ptr()), sr.data_ptr(), b ? br.data_ptr() : nullptr,
+                    y.data_ptr(), xr.stride(0), wr.stride(0), N, (int)M, (int)N, (int)K, dtype_code(*x), any_code(sr),
                     nbytes ? ws.data_ptr() : nullptr, nbytes, stream);
   });
   return result(rc, y);

@@ -112,7 +112,7 @@ def flash_attention(
     done = _lib.host().flash(q, k, v, causal, scale, cos, sin, q_pos0 if rope is not None else None, out)
     if done is not None:
         return _lib.checked(done)
-    # arguments the kernels cannot take as they are: refuse, copy or convert
+    # everything else: refuse, copy or convert
     if not q.is_cuda:
         raise RuntimeError("flash_attention requires CUDA tensors")
     if not (k.is_cuda and v.is_cuda) or k.device != q.device or v.device != q.device:

@@ -58,7 +58,7 @@ def int8_matmul(x: torch.Tensor, w_int8: torch.Tensor, scales: torch.Tensor,
     done = _lib.host().int8(x, w_int8, scales, bias)
     if done is not None:
         return _lib.checked(done)
-    # arguments the kernels cannot take as they are: refuse, copy or convert
+    # everything else: refuse, copy or convert
     if not x.is_cuda:
         raise RuntimeError("int8_matmul requires CUDA tensors")
     if scales.ndim != 1:

@@ -1,8 +1,9 @@
 """The compiled call layer (csrc/host.cpp) against the Python path it stands in
 for: the same call with the extension's functions handing everything back gives
 the same bits, over the layouts both accept (views, offsets, size-1 dimensions,
-padded rows, every table type) and those the extension hands back (misaligned,
-odd strides), in the output, the pools and the errors."""
+padded rows, every table type) and those both copy (misaligned, odd strides), in
+the output, the pools and the errors; and the extension takes these calls (one
+handed back pays for the refused call and then for all of the Python path)."""
 
 from __future__ import annotations
 
@@ -14,24 +15,25 @@ import torch
 
 from engine import _lib
 from engine.attention import flash_attention, paged_attention, paged_prefill
-from engine.cache import KVCacheConfig, PagedKVCache
+from engine.cache import KVCacheConfig, PagedKVCache, kv_append
 from engine.model import attention_section, attention_section_rows
 from engine.model.rope import build_rope_cache
 from engine.quant import int8_matmul
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
+NAMES = ("flash", "paged", "section", "append", "append_seq", "gather", "int8")
 
 
 def _python_only(m):
-    back = types.SimpleNamespace(**{n: (lambda *args: None) for n in ("flash", "paged", "section", "append", "append_seq",
-                                                                   "gather", "int8")})
+    back = types.SimpleNamespace(**{n: (lambda *args: None) for n in NAMES})
     m.setattr(_lib, "host", lambda: back)
 
 
-def _both(monkeypatch, call):
+def _both(monkeypatch, call, taken=True):
     """call() through the extension and through Python alone: the same tensors,
-    or the same refusal (an append of rows with odd strides)."""
+    or the same refusal (an append of rows with odd strides). taken: the
+    extension hands no call back (unless it is refused)."""
 
     def outcome():
         try:
@@ -39,7 +41,21 @@ def _both(monkeypatch, call):
         except ValueError as e:
             return str(e)
 
-    a = outcome()
+    host, back = _lib.host(), []
+
+    def noting(name):
+        def f(*args):
+            done = getattr(host, name)(*args)
+            if done is None:
+                back.append(name)
+            return done
+
+        return f
+
+    with monkeypatch.context() as m:
+        m.setattr(_lib, "host", lambda: types.SimpleNamespace(**{n: noting(n) for n in NAMES}))
+        a = outcome()
+    assert not (taken and back and not isinstance(a, str)), back
     with monkeypatch.context() as m:
         _python_only(m)
         b = outcome()
@@ -118,7 +134,7 @@ def test_paged(monkeypatch):
                 _both(monkeypatch, lambda: (paged_attention(q, kp, vp, t, n, **kw), paged_prefill(q, kp, vp, t, n, **kw)))
 
 
-@pytest.mark.parametrize("M,N,K", [(1, 24, 64), (3, 40, 100), (130, 136, 192), (0, 8, 64)])
+@pytest.mark.parametrize("M,N,K", [(1, 24, 64), (3, 40, 100), (130, 136, 192), (65, 40, 1000), (0, 8, 64)])
 def test_int8(monkeypatch, M, N, K):
     g = torch.Generator().manual_seed(M + K)
     w = torch.randint(-127, 128, (N, K), generator=g).to(torch.int8).to(DEV)
@@ -132,8 +148,8 @@ def test_int8(monkeypatch, M, N, K):
         for xx in (x, xp, x.view(1, M, K), x.t().contiguous().t()):
             for ww in (w, wp):
                 for ss in (s, s.half(), s.double()):
-                    for b in (None, s.to(dtype), s.half()):
-                        _both(monkeypatch, lambda: (int8_matmul(xx, ww, ss, bias=b),))
+                    for b in (None, s.to(dtype), s.half(), torch.nn.Parameter(s), s.repeat(2)[::2]):
+                        _both(monkeypatch, lambda: (int8_matmul(xx, ww, ss, bias=b),), taken=M > 0)
 
 
 def test_errors_keep_their_types():
@@ -187,12 +203,36 @@ def test_gather_of_other_caches(monkeypatch):
         t = cache.new_sequence()
         assert cache.gather(0, t)[0].shape == (0, 2, D)
         t.blocks, t.length = [5, 0, 3], 10
-        _both(monkeypatch, lambda: cache.gather(0, t))
+        _both(monkeypatch, lambda: cache.gather(0, t), taken=dtype == torch.float32)
+
+
+@pytest.mark.parametrize("rope", [False, True])
+def test_append_with_status_and_wide_indices(monkeypatch, rope):
+    """kv_append of int64 tables, counts and starts, with a status word of
+    either type: the pools and the status (a block id and, with rope, a
+    position out of range)."""
+    g = torch.Generator().manual_seed(4)
+    k, v = (torch.randn(9, 2, 64, generator=g).half().to(DEV) for _ in range(2))
+    tabs = tuple(t.to(DEV) for t in build_rope_cache(60, 64)) if rope else None
+    bt = torch.tensor([[3, 1, 99, 5], [0, 2, 4, 6]], device=DEV)
+    cu, start = torch.tensor([0, 5, 9], device=DEV), torch.tensor([29, 58], device=DEV)
+
+    def run(index, word):
+        kp, vp = (torch.zeros(8, 16, 2, 64, dtype=torch.float16, device=DEV) for _ in range(2))
+        status = None if word is None else torch.zeros(1, dtype=torch.int32, device=DEV).view(word)
+        kv_append(k, v, kp, vp, *(x.to(index) for x in (bt, cu, start)), 5, status, rope=tabs)
+        if word is not None:
+            assert status.view(torch.int32).item() == (3 if rope else 1)
+        return kp, vp
+
+    for index in (torch.int32, torch.int64):
+        for word in (None, torch.int32, torch.uint32):
+            _both(monkeypatch, lambda: run(index, word))
 
 
 @pytest.fixture
 def no_memory():
-    """Nothing over 20 MB can be allocated while it is entered (the caching
+    """Nothing over 4 MB can be allocated while it is entered (the caching
     allocator's own limit: the driver is never asked)."""
     import contextlib
 
@@ -202,9 +242,16 @@ def no_memory():
         torch.cuda.empty_cache()
         total = torch.cuda.get_device_properties(0).total_memory
         torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + 1024) / total)
+        held = []
         try:
+            try:
+                while True:  # what the allocator still holds in large blocks
+                    held.append(torch.empty(2 << 20, dtype=torch.uint8, device=DEV))
+            except torch.OutOfMemoryError:
+                pass
             yield
         finally:
+            held.clear()
             torch.cuda.set_per_process_memory_fraction(1.0)
 
     return limit
