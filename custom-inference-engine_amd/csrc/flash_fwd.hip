@@ -252,29 +252,39 @@ struct PagedTiles {
 
 // Partial state of one work item (p.part): the accumulator of each wave in
 // lane order (float4 slot x of lane l holds columns 8x + 4 (l / 32) .. +3 of
-// row l % 32: every store instruction writes 1 KiB in a row), then, after the
-// accumulators of all items, (reference max, row sum) of its 128 rows.
+// row l % 32: with 32 rows every store instruction writes 1 KiB in a row),
+// then, after the accumulators of all items, (reference max, row sum) of the
+// item's rows. Only rows a tile can hold have room: Lq of them up to 32, then
+// whole waves (128 for every item made it 34 MB where 0.3 are written: one row
+// of 32 heads over 16384 keys, D=128, 16 splits).
+__host__ __device__ inline int flash_part_rows(const FlashParams& p) {
+  return p.Lq <= 32 ? p.Lq : 32 * ((p.Lq < 128 ? p.Lq + 31 : 128) / 32);
+}
 __device__ __forceinline__ int64_t flash_part_item(const FlashParams& p, int b, int hq, int mt, int sp) {
   return (((int64_t)b * p.Hq + hq) * p.n_mt + mt) * p.splits + sp;
 }
+// The accumulator of a lane's row (below the rows that have room); slot x lies
+// flash_part_slot floats after slot x - 1.
+__device__ __forceinline__ int flash_part_slot(const FlashParams& p) { return 8 * min(p.Lq, 32); }
 template <int D>
-__device__ __forceinline__ float* flash_part_acc(const FlashParams& p, int64_t item) {
-  return p.part + item * (128 * D);
+__device__ __forceinline__ float* flash_part_acc(const FlashParams& p, int64_t item, int wave, int lane) {
+  return p.part + item * (flash_part_rows(p) * D) + wave * (32 * D) + 4 * ((lane >> 5) * min(p.Lq, 32) + (lane & 31));
 }
 template <int D>
 __device__ __forceinline__ float2* flash_part_ml(const FlashParams& p, int64_t item) {
-  const int64_t items = (int64_t)p.B * p.Hq * p.n_mt * p.splits;
-  return reinterpret_cast<float2*>(p.part + items * (128 * D)) + item * 128;
+  const int64_t items = (int64_t)p.B * p.Hq * p.n_mt * p.splits, rows = flash_part_rows(p);
+  return reinterpret_cast<float2*>(p.part + items * (rows * D)) + item * rows;
 }
 template <int D, typename Acc>
 __device__ __forceinline__ void flash_store_partial(const FlashParams& p, const FlashItem& w, int wave, int lane,
                                                     const Acc& acc, float m, float l) {
   const int64_t item = flash_part_item(p, w.b, w.hq, w.mt, w.sp);
-  float* sl = flash_part_acc<D>(p, item) + wave * (32 * D) + 4 * lane;
+  float* sl = flash_part_acc<D>(p, item, wave, lane);
+  const int slot = flash_part_slot(p);
 #pragma unroll
   for (int x = 0; x < D / 8; ++x) {
     const int dt = x / 4, g4 = x % 4;
-    *reinterpret_cast<float4*>(sl + 256 * x) =
+    *reinterpret_cast<float4*>(sl + slot * x) =
         float4{acc[dt][4 * g4], acc[dt][4 * g4 + 1], acc[dt][4 * g4 + 2], acc[dt][4 * g4 + 3]};
   }
   if (lane < 32) flash_part_ml<D>(p, item)[32 * wave + lane] = float2{m, l};
@@ -1094,7 +1104,8 @@ __global__ __launch_bounds__(256) void flash_merge_kernel(const FlashParams p) {
   const int row = mt * 128 + (int)wave * 32 + (lane & 31);
   if (row >= p.Lq) return;
   const int64_t item0 = flash_part_item(p, b, hq, mt, 0);
-  const float* sl = flash_part_acc<D>(p, item0) + wave * (32 * D) + 256 * x + 4 * lane;
+  const float* sl = flash_part_acc<D>(p, item0, wave, lane) + flash_part_slot(p) * x;
+  const int64_t rows = flash_part_rows(p);
   const float2* ml = flash_part_ml<D>(p, item0) + wave * 32 + (lane & 31);
   float M = -INFINITY, L = 0.f;
   float4 A = {0.f, 0.f, 0.f, 0.f};
@@ -1104,8 +1115,8 @@ __global__ __launch_bounds__(256) void flash_merge_kernel(const FlashParams p) {
 #pragma unroll
     for (int u = 0; u < kMergeAhead; ++u) {
       const int s = min(s0 + u, p.splits - 1);
-      a[u] = *reinterpret_cast<const float4*>(sl + (int64_t)s * (128 * D));
-      st[u] = ml[(int64_t)s * 128];
+      a[u] = *reinterpret_cast<const float4*>(sl + s * (rows * D));
+      st[u] = ml[s * rows];
     }
 #pragma unroll
     for (int u = 0; u < kMergeAhead; ++u) {
@@ -1653,7 +1664,7 @@ int flash_splits(const FlashParams& p, int D, bool paged) {
 
 size_t flash_part_bytes(const FlashParams& p, int D, int splits) {
   if (splits <= 1) return 0;
-  return (size_t)p.n_wg * splits * (128 * D + 256) * sizeof(float);  // p.n_wg = B * Hq * n_mt items
+  return (size_t)p.n_wg * splits * flash_part_rows(p) * (D + 2) * sizeof(float);  // p.n_wg = B * Hq * n_mt items
 }
 
 template <int DTYPE, int D, int MODE>

@@ -21,6 +21,7 @@
 #include <ATen/ATen.h>
 #include <ATen/core/grad_mode.h>
 #include <c10/core/DeviceGuard.h>
+#include <c10/util/Exception.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
@@ -132,6 +133,21 @@ void* stream_of(const Tensor& t) { return c10::hip::getCurrentHIPStream(t.device
 
 Tensor bytes_like(size_t n, const Tensor& t) { return at::empty({(int64_t)n}, t.options().dtype(at::kByte)); }
 
+// The partial states of a launch with key splits. When memory for them is short
+// the launch goes without splits, which needs none (*splits 0: the library's
+// rule, 1: none).
+Tensor split_workspace(size_t* nbytes, int* splits, const Tensor& like) {
+  *splits = 0;
+  if (!*nbytes) return Tensor();
+  try {
+    return bytes_like(*nbytes, like);
+  } catch (const c10::OutOfMemoryError&) {
+    *nbytes = 0;
+    *splits = 1;
+    return Tensor();
+  }
+}
+
 // Runs f without the GIL (as ctypes does); f returns a status.
 template <typename F>
 int launch(F&& f) {
@@ -180,15 +196,16 @@ PyObject* flash(PyObject*, PyObject* const* a, Py_ssize_t n) {
   if (causal < 0) return nullptr;
   const c10::OptionalDeviceGuard guard(q->device());
   const Tensor out = o ? *o : at::empty({B, H, M, D}, q->options());
-  const size_t nbytes = api.flash_ws((int)B, (int)H, (int)Hk, (int)M, (int)N, (int)D, causal, 0);
-  const Tensor ws = nbytes ? bytes_like(nbytes, *q) : Tensor();
+  size_t nbytes = api.flash_ws((int)B, (int)H, (int)Hk, (int)M, (int)N, (int)D, causal, 0);
+  int splits;
+  const Tensor ws = split_workspace(&nbytes, &splits, *q);
   const Tensor qc = laid_out(*q), kc = laid_out(*k), vc = laid_out(*v);
   const Strides sq(qc), sk(kc), sv(vc), so(out);
   void* stream = stream_of(*q);
   const int rc = launch([&] {
     return api.flash(qc.data_ptr(), kc.data_ptr(), vc.data_ptr(), out.data_ptr(), sq.s, sk.s, sv.s, so.s, (int)B,
                      (int)H, (int)Hk, (int)M, (int)N, (int)D, (float)scale, causal, dt, rope.cos, rope.sin, rope.rows,
-                     rope.dt, pos ? static_cast<const int32_t*>(pos->data_ptr()) : nullptr, 0,
+                     rope.dt, pos ? static_cast<const int32_t*>(pos->data_ptr()) : nullptr, splits,
                      nbytes ? ws.data_ptr() : nullptr, nbytes, stream);
   });
   return result(rc, out);
@@ -248,9 +265,10 @@ int paged_launch(const Tensor& q, const Pools& P, const Tensor& out, const Rope&
   const int B = (int)q.size(0), Hq = (int)q.size(1), Lq = (int)q.size(2), D = (int)q.size(3), dt = dtype_code(q);
   const int nb = (int)P.num_blocks, bs = (int)P.block_size, Hk = (int)P.Hk, w = (int)P.width, m = (int)mc;
   size_t nbytes = 0;
+  int splits = 0;
   if (prefill) nbytes = api.flash_paged_ws(B, Hq, Hk, Lq, D, m, bs, w, 0);
   else if (!plan.data || plan.split) nbytes = api.paged_ws(B, Hq, Hk, Lq, D, m, bs, w);
-  const Tensor ws = nbytes ? bytes_like(nbytes, q) : Tensor();
+  const Tensor ws = prefill ? split_workspace(&nbytes, &splits, q) : nbytes ? bytes_like(nbytes, q) : Tensor();
   const Strides sq(q), sk(*P.kc), sv(*P.vc), so(out);
   void* const wp = nbytes ? ws.data_ptr() : nullptr;
   void* stream = stream_of(q);
@@ -261,7 +279,7 @@ int paged_launch(const Tensor& q, const Pools& P, const Tensor& out, const Rope&
     if (prefill)
       return api.flash_paged(q.data_ptr(), P.kc->data_ptr(), P.vc->data_ptr(), bt, lens, out.data_ptr(), sq.s, sk.s,
                              sv.s, so.s, B, Hq, Hk, Lq, D, nb, bs, w, m, (float)scale, causal, dt, rope.cos, rope.sin,
-                             rope.rows, rope.dt, 0, wp, nbytes, stream);
+                             rope.rows, rope.dt, splits, wp, nbytes, stream);
     return api.paged(q.data_ptr(), kn, vn, P.kc->data_ptr(), P.vc->data_ptr(), bt, lens, plan.data ? plan.data->data_ptr() : nullptr,
                      plan.data ? (size_t)plan.data->nbytes() : 0, plan.split, out.data_ptr(), wp, nbytes, sq.s, kns, vns,
                      sk.s, sv.s, so.s, B, Hq, Hk, Lq, D, nb, bs, w, m, (float)scale, causal, dt, rope.cos, rope.sin,

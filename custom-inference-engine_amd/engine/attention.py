@@ -171,10 +171,14 @@ def _flash_workspace_bytes(device: int, B: int, H: int, Hk: int, M: int, N: int,
 
 def _split_workspace(nbytes: int, q: torch.Tensor) -> tuple[torch.Tensor | None, int]:
     """Partial states of a split launch: allocated for the call (the caching
-    allocator orders its reuse on the stream), nothing when not split."""
+    allocator orders its reuse on the stream); nothing when not split, or when
+    memory for them is short (the launch then goes without splits)."""
     if nbytes == 0:
         return None, 0
-    return torch.empty(nbytes, dtype=torch.uint8, device=q.device), nbytes
+    try:
+        return torch.empty(nbytes, dtype=torch.uint8, device=q.device), nbytes
+    except torch.OutOfMemoryError:
+        return None, 0
 
 
 def paged_prefill(
@@ -236,7 +240,7 @@ def paged_prefill(
             q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), bt.data_ptr(), lens.data_ptr(), out.data_ptr(),
             _lib.strides(q), _lib.strides(k_cache), _lib.strides(v_cache), _lib.strides(out),
             B, Hq, Hk, Lq, D, num_blocks, block_size, bt.shape[1], mc, float(scale), 1 if causal else 0,
-            _lib.DTYPE_CODES[q.dtype], *rp, 0, ws.data_ptr() if ws is not None else None, nbytes,
+            _lib.DTYPE_CODES[q.dtype], *rp, 0 if ws is not None else 1, ws.data_ptr() if ws is not None else None, nbytes,
             _lib.stream_handle(q.device))
     _lib.check(rc)
     return out

@@ -168,6 +168,18 @@ def test_paged_workspace_size():
     assert _paged(Lq=33, D=256, qs=_st(8448 * 4, 8448, 256, 1), os_=_st(8448 * 4, 8448, 256, 1)) == _lib.CIE_EINVAL
 
 
+@pytest.mark.parametrize("Lq,rows", [(1, 1), (5, 5), (32, 32), (33, 64), (100, 128), (128, 128), (300, 128)])
+def test_split_workspace_holds_the_rows_of_a_tile(Lq, rows):
+    """Partial states of 16 splits: D floats, a max and a sum per row that a
+    128-row query tile can hold, in whole waves above 32 rows."""
+    lib = _lib.load()
+    tiles = -(-Lq // 128)
+    want = 16 * 32 * tiles * rows * (128 + 2) * 4
+    assert lib.cie_flash_workspace_bytes(1, 32, 8, Lq, 16384, 128, 1, 16) == want
+    assert lib.cie_flash_paged_workspace_bytes(1, 32, 8, Lq, 128, 16384, 16, 1024, 16) == want
+    assert lib.cie_flash_workspace_bytes(1, 32, 8, Lq, 16384, 128, 1, 1) == 0
+
+
 def test_error_codes_map_to_reference_exception_types():
     with pytest.raises(ValueError):
         _lib.check(_lib.CIE_EDTYPE)

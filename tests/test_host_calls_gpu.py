@@ -289,3 +289,27 @@ def test_out_of_memory_is_torch_out_of_memory(monkeypatch, no_memory, path):
             with no_memory(), pytest.raises(torch.OutOfMemoryError):
                 call()
             assert call() is not None, name
+
+
+@pytest.mark.parametrize("path", ["compiled", "python"])
+def test_split_launches_go_without_their_workspace(monkeypatch, no_memory, path):
+    """Calls whose keys are split fit a full GPU: without room for the partial
+    states they run unsplit."""
+    g = torch.Generator().manual_seed(1)
+    f16 = torch.float16
+    q = torch.randn(1, 32, 300, 128, generator=g).to(DEV, f16)
+    kp, vp = (torch.randn(400, 16, 8, 128, generator=g).to(DEV, f16) for _ in range(2))
+    bt, lens = torch.arange(400, dtype=torch.int32, device=DEV).view(1, 400), torch.full((1,), 6400, dtype=torch.int32, device=DEV)
+    k, v = (p.view(1, 6400, 8, 128).transpose(1, 2) for p in (kp, vp))
+    out = torch.empty_like(q)
+    assert _lib.load().cie_flash_workspace_bytes(1, 32, 8, 300, 6400, 128, 1, 0) > 4 << 20
+    assert _lib.load().cie_flash_paged_workspace_bytes(1, 32, 8, 300, 128, 0, 16, 400, 0) > 4 << 20
+    with monkeypatch.context() as m:
+        if path == "python":
+            _python_only(m)
+        for call in (lambda: flash_attention(q, k, v, causal=True, out=out),
+                     lambda: paged_prefill(q, kp, vp, bt, lens, out=out)):
+            want = call().clone()
+            with no_memory():
+                got = call()
+            assert (got.float() - want.float()).abs().max().item() <= 2e-3
