@@ -1633,19 +1633,28 @@ FlashKernel flash_kernel_choice(const FlashParams& p, int D) {
 // keys alone; with them every partial state is written and read once more. The
 // estimate, in microseconds: a workgroup walks its tiles at kStep each (25 %
 // slower when the waves of two workgroups share a CU; one wave of a short query
-// tile does not notice; 15 % slower over a paged history), launches in rounds of the workgroup slots, and a
-// split launch pays 4.2 us and 0.3 us per split for its second pass plus its
-// partial states at 1.6 MB/us. Measured, splits: us (B x Hq x Lq x Lk, D, causal):
-//   1x32x5x3001 D=64      1: 35.3  2: 22.5  4: 14.8  8: 11.9  16: 13.3
-//   1x32x5x300 D=64       1: 6.7   2: 8.4   4: 8.1
-//   1x32x5x16384 D=128    1: 260   4: 71.6  8: 40.7  16: 28.1
-//   1x32x300x1500 D=64    1: 21.9  2: 19.3  4: 18.9  8: 24.8 (paged 1: 24.8  2: 21.3  4: 20.1)
-//   1x32x1000x4600 D=128  1: 87.4  2: 78.2  3: 88.4  4: 84.6
-//   1x16x512x512 D=64     1: 10.0  2: 11.8  4: 13.3
-//   1x32x500x500 D=128    1: 14.6  2: 22.7
+// tile does not notice; 45 % slower over a paged history, whose P.V products
+// are two), launches in rounds of the workgroup slots, and a split launch pays
+// 4.2 us and 0.3 us per split for its second pass plus its partial states at
+// 1.6 MB/us. A causal launch is costed by its longest tile. Measured over 17
+// dense and 11 paged shapes at each head_dim, the choice is never slower than no
+// splits and 2 % from the best count on average (up to 20 % on a few paged chunks
+// of 50-100 tiles of work). Splits: us (B x Hq / Hk x Lq x Lk, causal):
+//   D=16   1x32/8x5x3001       1: 23.6  4: 12.1  8: 11.1  16: 13.8
+//   D=16   1x4/4x2000x2000     1: 17.9  2: 14.0  4: 11.2  8: 12.1
+//   D=32   2x32/8x150x3000 paged  1: 44.4  2: 30.6  4: 28.9  8: 32.2
+//   D=64   1x32/8x5x3001       1: 35.7  4: 15.4  8: 12.5  12: 13.1  16: 13.7
+//   D=64   4x32/8x1x4096       1: 47.3  2: 29.6  4: 20.5  8: 24.7
+//   D=64   1x16/16x512x512     1: 10.4  2: 12.2  4: 13.8
+//   D=64   1x32/8x300x1500     1: 21.4  2: 19.4  4: 19.0  8: 25.2
+//   D=64   the same, paged     1: 30.1  2: 24.1  4: 23.1  8: 28.9
+//   D=128  1x16/2x1x16384      1: 260   4: 71.7  8: 41.6  16: 27.8  32: 26.0
+//   D=128  1x32/8x1000x4600 paged  1: 126  2: 113  3: 119  4: 118
+//   D=256  1x32/8x64x2048      1: 83.0  4: 33.2  6: 29.0  8: 29.6  16: 33.4
+//   D=256  1x8/8x1000x1000     1: 47.5  2: 37.9  3: 33.7  4: 30.0  8: 37.6
 int flash_splits(const FlashParams& p, int D, bool paged) {
   const int bn = D <= 32 ? 128 : (D == 64 ? 64 : 32);
-  const double kStep = (paged ? 1.15 : 1.0) * (D == 256 ? 1.35 : D == 128 ? 0.6 : D == 64 ? 0.75 : 1.05);
+  const double kStep = (paged ? 1.45 : 1.0) * (D == 256 ? 1.35 : D == 128 ? 0.6 : D == 64 ? 0.75 : 1.05);
   const int64_t items = p.n_wg, per_cu = D <= 128 ? 2 : 1, slots = per_cu * p.cus;
   const int64_t nt = ((int64_t)p.Lk + bn - 1) / bn;  // tiles of the longest item
   if (items < 1 || items >= slots) return 1;
