@@ -22,6 +22,7 @@
 #include <ATen/core/grad_mode.h>
 #include <c10/core/DeviceGuard.h>
 #include <c10/util/Exception.h>
+#include <c10/hip/HIPGraphsC10Utils.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
@@ -453,6 +454,13 @@ struct SeqPools {
   }
 };
 
+// A graph captured from either of the two below would replay with the block ids
+// and the position of the capture: handed back, to be refused like the copies
+// of the Python path.
+bool capturing() {
+  return c10::hip::currentStreamCaptureStatusMayInitCtx() != c10::hip::CaptureStatus::None;
+}
+
 // append_seq(k_new, v_new, k_cache, v_cache, blocks, start): (L, heads, D) rows
 // to positions start ..; True when done.
 PyObject* append_seq(PyObject*, PyObject* const* a, Py_ssize_t n) {
@@ -475,9 +483,10 @@ PyObject* append_seq(PyObject*, PyObject* const* a, Py_ssize_t n) {
     PyErr_Clear();
     Py_RETURN_NONE;
   }
+  const c10::OptionalDeviceGuard guard(k->device());
+  if (capturing()) Py_RETURN_NONE;
   const Strides sk(*k), sv(*v);
   const int64_t dense[4] = {2 * sk.s[0], 2 * sk.s[1], 2 * sv.s[0], 2 * sv.s[1]};
-  const c10::OptionalDeviceGuard guard(k->device());
   void* stream = stream_of(*k);
   const int rc = launch([&] {
     return api.append_seq(k->data_ptr(), v->data_ptr(), kc->data_ptr(), vc->data_ptr(), dense, P.strides, ids.data(),
@@ -503,6 +512,7 @@ PyObject* gather(PyObject*, PyObject* const* a, Py_ssize_t n) {
     Py_RETURN_NONE;
   }
   const c10::OptionalDeviceGuard guard(kc->device());
+  if (capturing()) Py_RETURN_NONE;
   const int64_t heads = kc->size(2);
   const Tensor k = at::empty({L, heads, kc->size(3)}, kc->options()), v = at::empty_like(k);
   const int64_t dense[4] = {heads * P.head_bytes, P.head_bytes, heads * P.head_bytes, P.head_bytes};

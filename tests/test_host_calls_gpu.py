@@ -313,3 +313,23 @@ def test_split_launches_go_without_their_workspace(monkeypatch, no_memory, path)
             with no_memory():
                 got = call()
             assert (got.float() - want.float()).abs().max().item() <= 2e-3
+
+
+def test_single_sequence_moves_are_not_captured():
+    """append / gather of one sequence put host block ids into the launch: a
+    graph would replay stale ones, so under capture the extension hands them
+    back (the Python path's copy to the device then refuses)."""
+    cache = PagedKVCache(KVCacheConfig(1, 2, 64, 8, 16, torch.float16, DEV))
+    k = torch.ones(3, 2, 64, dtype=torch.float16, device=DEV)
+    args = (k, k, cache.k[0], cache.v[0], [5], 0)
+    x = torch.zeros(1, device=DEV)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        x.add_(1)
+        assert _lib.host().append_seq(*args) is None
+        assert _lib.host().gather(cache.k[0], cache.v[0], [5], 3) is None
+    graph.replay()
+    torch.cuda.synchronize()
+    assert x.item() == 1 and not cache.k[0].any()
+    assert _lib.host().append_seq(*args) is True
+    assert torch.equal(_lib.host().gather(cache.k[0], cache.v[0], [5], 3)[0], k)
