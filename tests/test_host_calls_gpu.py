@@ -333,3 +333,81 @@ def test_single_sequence_moves_are_not_captured():
     assert x.item() == 1 and not cache.k[0].any()
     assert _lib.host().append_seq(*args) is True
     assert torch.equal(_lib.host().gather(cache.k[0], cache.v[0], [5], 3)[0], k)
+
+
+def _workspace_calls(seed):
+    """Calls that allocate a workspace each (key splits dense and paged, split
+    K, paged partial states), as closures over inputs of their own, and the
+    inputs to refill."""
+    g = torch.Generator().manual_seed(seed)
+    rand = lambda *shape: torch.randn(shape, generator=g).half().to(DEV)  # noqa: E731
+    q, qp, qd = rand(1, 32, 5, 64), rand(1, 16, 300, 64), rand(3, 16, 1, 64)
+    k, v = rand(1, 8, 3001, 64), rand(1, 8, 3001, 64)
+    kp, vp = rand(300, 16, 4, 64), rand(300, 16, 4, 64)
+    bt = torch.randperm(300, generator=g).int().to(DEV)
+    lens = torch.tensor([1500, 700, 33], dtype=torch.int32, device=DEV)
+    x, w = rand(96, 2048), torch.randint(-127, 128, (512, 2048), generator=g).to(torch.int8).to(DEV)
+    sc = torch.rand(512, generator=g).half().to(DEV)
+    lib = _lib.load()
+    assert min(lib.cie_flash_workspace_bytes(1, 32, 8, 5, 3001, 64, 1, 0),
+               lib.cie_flash_paged_workspace_bytes(1, 16, 4, 300, 64, 0, 16, 100, 0),
+               lib.cie_int8_matmul_workspace_bytes(96, 512, 2048)) > 0
+    calls = [lambda: flash_attention(q, k, v, causal=True),
+             lambda: paged_prefill(qp, kp, vp, bt[:100].view(1, 100), lens[:1]),
+             lambda: paged_attention(qd, kp, vp, bt.view(3, 100), lens),
+             lambda: int8_matmul(x, w, sc, bias=sc)]
+    return calls, (q, qp, qd, k, v, kp, vp, x)
+
+
+def test_workspaces_in_a_captured_graph():
+    """A graph of calls that allocate their workspaces, replayed with new
+    inputs and eager calls in between."""
+    calls, inputs = _workspace_calls(11)
+    g = torch.Generator().manual_seed(12)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        for call in calls:
+            call()
+    torch.cuda.current_stream().wait_stream(side)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        outs = [call() for call in calls]
+    for _ in range(3):
+        for t in inputs:
+            t.copy_(torch.randn(t.shape, generator=g).half())
+        graph.replay()
+        torch.cuda.synchronize()
+        got = [o.clone() for o in outs]
+        for a, call in zip(got, calls):
+            assert torch.isfinite(a.float()).all() and torch.equal(a, call())
+
+
+def test_two_threads_on_their_own_streams():
+    """The extension releases the GIL around a launch: two threads, each on a
+    stream of its own, get what one thread gets on the default stream."""
+    import threading
+
+    sets = [_workspace_calls(seed) for seed in (21, 22)]
+    want = [[call() for call in calls] for calls, _ in sets]
+    torch.cuda.synchronize()
+    bad, gate = [], threading.Barrier(2)
+
+    def work(i):
+        try:
+            stream = torch.cuda.Stream()
+            gate.wait(timeout=30)
+            with torch.cuda.stream(stream):
+                for _ in range(25):
+                    got = [call() for call in sets[i][0]]
+                    stream.synchronize()
+                    bad.extend((i, n) for n, (a, b) in enumerate(zip(got, want[i])) if not torch.equal(a, b))
+        except Exception as e:  # noqa: BLE001
+            bad.append((i, repr(e)))
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join(timeout=60)
+    assert not any(t.is_alive() for t in threads) and not bad, bad[:4]
