@@ -74,9 +74,14 @@ class StepBatch:
     cache: dict = field(default_factory=dict, repr=False)  # device index tensors of ragged steps, built once
     _host_flags: tuple | None = field(default=None, init=False, repr=False, compare=False)  # (fresh, aligned, total)
 
+    def __setattr__(self, name: str, value) -> None:
+        if name in ("starts_host", "lengths_host", "new_counts"):
+            object.__setattr__(self, "_host_flags", None)
+        object.__setattr__(self, name, value)
+
     def _flags(self) -> tuple:
-        """(fresh, aligned, total new tokens) of the host copies, found once:
-        every layer of the step asks."""
+        """(fresh, aligned, total new tokens) of the host copies, found once
+        (every layer of the step asks) and again when one of them is replaced."""
         if self._host_flags is None:
             rows = list(zip(self.starts_host, self.lengths_host, self.new_counts))
             self._host_flags = (all(s0 == 0 and n == c for s0, n, c in rows), all(s0 + c == n for s0, n, c in rows),

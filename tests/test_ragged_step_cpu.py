@@ -82,3 +82,16 @@ def test_chunked_causal_rows_equal_the_whole_block(c, hist, chunk):
                                 causal=True)
     if i1 - i0 > 1:
         assert not torch.allclose(wrong.nan_to_num(9.0), whole[:, :, i0:i1], atol=1e-3)
+
+
+def test_step_flags_follow_the_host_copies():
+    """fresh, aligned and total_new are found once per step, and again when a
+    program moves the step on by replacing its host copies."""
+    step = _step([4, 4], [4, 4])
+    assert step.fresh and step.aligned and step.total_new == 8
+    step.starts_host, step.lengths_host = (4, 4), (8, 8)
+    assert not step.fresh and step.aligned
+    step.lengths_host = (9, 8)
+    assert not step.aligned
+    step.new_counts = (4, 3)
+    assert step.total_new == 7
