@@ -170,8 +170,7 @@ def _paged_rows(q_rows: torch.Tensor, layer_idx: int, cache: PagedKVCache, step:
         rope = None
     key = ("launches",)
     if key not in step.cache:
-        step.cache[key] = [(*launch, *_group_span(step, launch[3]))
-                           for launch in _launches(step, max(1, step.max_new), dev)]
+        step.cache[key] = _launches(step, dev)
     for tables, rows, lens, L, r0, max_context in step.cache[key]:
         n = lens.shape[0]
         # (a group of more query heads per kv head than paged_attention takes is refused there)
@@ -184,42 +183,36 @@ def _paged_rows(q_rows: torch.Tensor, layer_idx: int, cache: PagedKVCache, step:
             out_rows[rows] = o.transpose(1, 2).reshape(-1, Hq, D)
 
 
-def _group_span(step: StepBatch, count: int) -> tuple[int | None, int]:
-    """First packed row of the sequences with ``count`` new tokens when their
-    rows are consecutive (else None), and their longest context."""
-    seqs = [b for b, c in enumerate(step.new_counts) if c == count]
+def _group_span(step: StepBatch, seqs: list[int], count: int) -> tuple[int | None, int]:
+    """First packed row of the sequences ``seqs`` with ``count`` new tokens
+    each when their rows are consecutive (else None), and their longest
+    context."""
     between = step.new_counts[seqs[0]:seqs[-1] + 1]
     contiguous = all(c in (count, 0) for c in between)
     return (sum(step.new_counts[:seqs[0]]) if contiguous else None), max(step.lengths_host[b] for b in seqs)
 
 
-def _launches(step: StepBatch, chunk: int, dev: torch.device) -> list:
-    """(block tables (B', max_blocks), packed row indices (B' * Lsub,),
-    context lengths (B',), Lsub) of every launch of a step; the indices are
-    uploaded in one copy."""
+def _launches(step: StepBatch, dev: torch.device) -> list:
+    """(block tables (B', max_blocks), packed row indices (B' * L,), context
+    lengths (B',), L, first packed row or None, longest context) per count L of
+    new tokens in the step; the indices are uploaded in one copy."""
     groups: dict[int, list[int]] = {}
     for b, c in enumerate(step.new_counts):
         if c > 0:
             groups.setdefault(c, []).append(b)
+    if not groups:
+        return []
     cu = [0]
     for c in step.new_counts:
         cu.append(cu[-1] + c)
-    parts, shapes = [], []
+    flat = []
     for c, seqs in sorted(groups.items()):
-        for i0 in range(0, c, chunk):
-            i1 = min(c, i0 + chunk)
-            rows = [cu[b] + i for b in seqs for i in range(i0, i1)]
-            lens = [step.lengths_host[b] - c + i1 for b in seqs]
-            parts += [seqs, rows, lens]
-            shapes.append((len(seqs), i1 - i0))
-    if not shapes:
-        return []
-    flat = torch.tensor([x for part in parts for x in part], dtype=torch.int64).to(dev)
+        flat += seqs + [cu[b] + i for b in seqs for i in range(c)] + [step.lengths_host[b] for b in seqs]
+    flat = torch.tensor(flat, dtype=torch.int64).to(dev)
     out, p = [], 0
-    for n, Lsub in shapes:
-        tables = step.block_tables[flat[p:p + n]]
-        rows = flat[p + n:p + n + n * Lsub]
-        lens = flat[p + n + n * Lsub:p + 2 * n + n * Lsub].to(torch.int32)
-        out.append((tables, rows, lens, Lsub))
-        p += 2 * n + n * Lsub
+    for c, seqs in sorted(groups.items()):
+        n = len(seqs)
+        out.append((step.block_tables[flat[p:p + n]], flat[p + n:p + n + n * c],
+                    flat[p + n + n * c:p + 2 * n + n * c].to(torch.int32), c, *_group_span(step, seqs, c)))
+        p += 2 * n + n * c
     return out

@@ -1,17 +1,17 @@
 """Host logic of the ragged / long-step attention section on the CPU.
 
-attention_section_rows and the long-chunk branch of attention_section run
-paged attention per group of sequences with equal counts of new tokens, in
-launches of at most 256 query rows per kv head: chunk [i0, i1) of a
-sequence's c new tokens is launched as the i1 - i0 newest tokens of a
-context of length ctx - c + i1. Checked here:
+attention_section_rows and the long-chunk branch of attention_section run one
+launch per count of new tokens, over the sequences with that count. Checked
+here:
 
 * the launch list covers every new-token row exactly once, with the block
-  table row of its own sequence and that context length;
-* the splitting identity itself on the oracle: the chunks' causal attention
-  (the reference's bottom-right mask, kernels/ref/flash_attention_ref.py:
-  35-39) equals the whole block's, row for row -- a wrong length (ctx - c +
-  i0, or ctx) fails it."""
+  table row and context length of its own sequence, and says which groups lie
+  in consecutive rows and how long their contexts are;
+* the oracle's causal rule (the reference's bottom-right mask,
+  kernels/ref/flash_attention_ref.py:35-39) gives a prompt prefilled in chunks
+  over several steps the rows of the whole prompt: chunk [i0, i1) of c new
+  tokens is the i1 - i0 newest tokens of a context of length ctx - c + i1, and
+  a wrong length (ctx - c + i0, or ctx) fails it."""
 
 from __future__ import annotations
 
@@ -36,30 +36,31 @@ def _step(counts, lengths, width=4):
                      lengths_host=tuple(lengths), new_counts=tuple(counts))
 
 
-@pytest.mark.parametrize("counts,chunk", [([300, 1, 1, 0, 5, 700, 64, 1], 64), ([4, 4, 4], 256), ([1], 1),
-                                          ([129, 128, 127, 0], 32), ([0, 0], 8)])
-def test_launches_cover_every_row_once(counts, chunk):
+@pytest.mark.parametrize("counts,spans", [
+    ([300, 1, 1, 0, 5, 700, 64, 1], {300: 0, 1: None, 5: 302, 700: 307, 64: 1007}),  # the last 1 is apart
+    ([4, 4, 4], {4: 0}), ([1], {1: 0}), ([0, 7, 0, 0, 7, 2], {7: 0, 2: 14}),  # zeros in between stay consecutive
+    ([2, 3, 2, 3], {2: None, 3: None}), ([129, 128, 127, 0], {129: 0, 128: 129, 127: 257}), ([0, 0], {}), ([], {})])
+def test_launches_cover_every_row_once(counts, spans):
     lengths = [c + 37 * b for b, c in enumerate(counts)]
-    step = _step(counts, lengths)
-    launches = _launches(step, chunk, torch.device("cpu"))
+    step = _step(counts, lengths or [0])
+    launches = _launches(step, torch.device("cpu"))
     cu = [0]
     for c in counts:
         cu.append(cu[-1] + c)
-    seen = {}
-    for tables, rows, lens, Lsub in launches:
-        assert 1 <= Lsub <= chunk and rows.numel() == tables.shape[0] * Lsub == lens.shape[0] * Lsub
-        for j in range(tables.shape[0]):
+    seen = []
+    for tables, rows, lens, L, r0, longest in launches:
+        n = tables.shape[0]
+        assert rows.numel() == n * L and lens.shape[0] == n and lens.dtype == torch.int32
+        for j in range(n):
             b = int(tables[j, 0]) // 4
-            assert torch.equal(tables[j], step.block_tables[b])
-            r = rows[j * Lsub:(j + 1) * Lsub].tolist()
-            i1 = r[-1] - cu[b] + 1
-            assert r == list(range(cu[b] + i1 - Lsub, cu[b] + i1))  # consecutive rows of sequence b
-            assert int(lens[j]) == lengths[b] - counts[b] + i1
-            for x in r:
-                seen[x] = seen.get(x, 0) + 1
-    assert sorted(seen) == list(range(sum(counts))) and all(n == 1 for n in seen.values())
-    # one launch per (count, chunk) pair
-    assert len(launches) == sum(-(-c // chunk) for c in set(counts) if c)
+            assert torch.equal(tables[j], step.block_tables[b]) and counts[b] == L
+            assert rows[j * L:(j + 1) * L].tolist() == list(range(cu[b], cu[b + 1]))
+            assert int(lens[j]) == lengths[b]
+        seen += rows.tolist()
+        assert r0 == spans[L] and longest == int(lens.max())
+        if r0 is not None:
+            assert rows.tolist() == list(range(r0, r0 + n * L))
+    assert sorted(seen) == list(range(sum(counts))) and sorted(launch[3] for launch in launches) == sorted(spans)
 
 
 @pytest.mark.parametrize("c,hist,chunk", [(300, 200, 64), (97, 0, 32), (5, 1000, 2)])
