@@ -37,7 +37,8 @@
 // max, raise m to it and redo the tile. Otherwise every p <= 2^10, exact to
 // fp16 / bf16 rounding. The final acc / l is unchanged by the choice of m. l
 // accumulates the probabilities as rounded for the P.V product, summed on
-// the matrix pipe (see sum_ones).
+// the matrix pipe (see sum_ones); launches over a paged history sum them in
+// fp32 and keep their rounding as a second operand (see kTwoPartP).
 //
 // The tile loop is unrolled by a multiple of the ring depth so that every
 // LDS stage offset is an immediate of the fragment reads.

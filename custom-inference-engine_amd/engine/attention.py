@@ -367,8 +367,9 @@ def paged_workspace_bytes(B: int, Hq: int, Hk: int, Lq: int, D: int, block_size:
         B, Hq, Hk, Lq, D, int(max_context or 0), block_size, max_blocks_per_seq))
 
 
-# Workspaces, one per (device, stream): calls on one stream run in order, so
-# they can share it. A workspace outgrown by a larger call is retired, never
+# Workspaces of the calls csrc/host.cpp does not take (new_kv or plan given
+# here; the others get one per call), one per (device, stream): calls on one
+# stream run in order, so they can share it. A workspace outgrown by a larger call is retired, never
 # freed: a HIP graph captured earlier may still hold its address, and its
 # replays must not write into memory the caching allocator has handed to
 # another tensor.
@@ -415,8 +416,9 @@ def paged_attention(
     upper bound of context_lens; a longer context yields NaN) lets the launch
     size its work split tighter than max_blocks * block_size. ``workspace``:
     a caller-owned uint8 device buffer of at least
-    :func:`paged_workspace_bytes` bytes; by default a cached per-(device,
-    stream) buffer is used. Equal to ``flash_attention`` over ``cache.gather``
+    :func:`paged_workspace_bytes` bytes; by default one is allocated for the
+    call (the caching allocator orders its reuse on the stream), or, with
+    ``new_kv`` or ``plan``, a buffer kept per (device, stream). Equal to ``flash_attention`` over ``cache.gather``
     per sequence. Returns (B, Hq, Lq, D) in q's dtype.
 
     ``rope``: (cos, sin) tables; q is then un-rotated and row i of sequence

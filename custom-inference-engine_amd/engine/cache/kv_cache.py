@@ -18,10 +18,11 @@ kernels read; :func:`kv_append`, the batched device write of new tokens
 many sequences; :meth:`PagedKVCache.prepare_step` / :meth:`append_step`,
 which upload a step's metadata once for all layers (:class:`StepBatch`);
 and :meth:`PagedKVCache.attend`, which runs
-``paged_attention`` on one layer's pools. On a CUDA device ``append`` writes
-through ``cie_kv_append`` (the reference's per-block slice loop,
-kv_cache.py:128-136, becomes one launch); a cache on the CPU device keeps the
-reference's slice copies, since no kernel runs there.
+``paged_attention`` on one layer's pools. On a CUDA device ``append`` and
+``gather`` are one launch each with the block ids among its arguments
+(``cie_kv_append_seq``, ``cie_kv_gather``; the reference's per-block slice
+loop, kv_cache.py:128-136, and its gather, :141-165); a cache on the CPU device
+keeps the reference's slice copies, since no kernel runs there.
 """
 
 from __future__ import annotations

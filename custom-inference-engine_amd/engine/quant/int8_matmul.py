@@ -14,7 +14,8 @@ import torch
 from engine import _lib
 
 _SCALE_CODES = {torch.float16: 0, torch.bfloat16: 1, torch.float32: 2}
-# One split-K workspace per (device, stream); an outgrown one is retired, not
+# Split-K workspace of the calls csrc/host.cpp does not take (the others get one
+# per call), one per (device, stream); an outgrown one is retired, not
 # freed, since a HIP graph captured earlier may still write to it.
 _WORKSPACES: dict[tuple[int, int], torch.Tensor] = {}
 _RETIRED_WORKSPACES: list[torch.Tensor] = []
