@@ -15,7 +15,7 @@ import pytest
 import torch
 
 from engine import _lib
-from engine.attention import flash_attention, paged_prefill
+from engine.attention import flash_attention, paged_attention, paged_prefill
 from engine.model.rope import build_rope_cache
 from oracle import flash_attention_ref, gather_ref, rope_ref
 
@@ -164,3 +164,28 @@ def test_paged_prefill_error_is_the_rounding_of_its_output(D, dtype, rising):
     rel = lambda x: ((x.double() - ref).norm() / ref.norm()).item()  # noqa: E731
     out = paged_prefill(q.to(DEV), kp.to(DEV), vp.to(DEV), bt.to(DEV), torch.tensor([n], dtype=torch.int32, device=DEV))
     assert rel(out[0].cpu()) <= 1.05 * rel(ref.to(dtype))
+
+
+@pytest.mark.parametrize("D,bs", [(16, 16), (64, 5), (128, 16), (256, 8)])
+@pytest.mark.parametrize("kw", [{}, {"causal": False}, {"max_context": 200}, {"scale": -0.4}, {"scale": 0.0}])
+@pytest.mark.parametrize("rope", [False, True])
+def test_paged_prefill_answers_as_paged_attention(D, bs, kw, rope):
+    """The route of long chunks against the one of short ones over the lengths
+    both take: empty, shorter than the new tokens, at tile edges, at and past
+    the table's and the hint's limit, negative, with a pool of other strides;
+    NaN and zero rows in the same places."""
+    Hq, Hk, Lq = 4, 2, 40
+    lens = [0, 1, 39, 40, 41, 63, 64, 65, 199, 200, 201, 256, 300, 301, -1, 2 ** 30]
+    g = torch.Generator().manual_seed(D + bs)
+    width = -(-300 // bs)
+    # ids of lengths within the table (-(-300 // bs) * bs tokens); any valid ids do for the others
+    bt = torch.randint(0, 70, (len(lens), width), generator=g).int().to(DEV)
+    pool = torch.randn(2, 70, Hk, bs, D + 8, generator=g).half().to(DEV)
+    kp, vp = pool[0, ..., :D].transpose(1, 2), pool[1, ..., :D].transpose(1, 2)
+    q = _randn(g, len(lens), Lq, Hq, D, dtype=torch.float16).to(DEV).transpose(1, 2)
+    lt = torch.tensor(lens, dtype=torch.int32, device=DEV)
+    tabs = tuple(t.to(DEV) for t in build_rope_cache(250, D)) if rope else None  # positions from 250 on are NaN rows
+    a = paged_attention(q, kp, vp, bt, lt, rope=tabs, **kw)
+    b = paged_prefill(q, kp, vp, bt, lt, rope=tabs, **kw)
+    _close(b, a.cpu(), 2e-3, "paged_prefill")
+    assert torch.isnan(a[-1]).all() and (a[0] == 0).all()
